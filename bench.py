@@ -46,9 +46,9 @@ def batch_roofline(weight_bytes, flops, seconds):
     """Both bounds of a configuration: packed weight bytes over the HBM peak
     and the product's fp32 arithmetic (2 x positions x rows x columns flops)
     over the fp32 vector peak; `bound` names the larger fraction. The
-    matrix-core and prefill paths compute the same exact products from three
-    bf16 limbs per activation, so this fp32 figure is the algorithmic rate,
-    not the matrix-core issue rate."""
+    matrix-core path computes the same products from two f16 limbs per
+    activation, so this fp32 figure is the algorithmic rate, not the
+    matrix-core issue rate."""
     gbs = weight_bytes / seconds / 1e9
     tflops = flops / seconds / 1e12
     hbm, fp32 = gbs / HBM_PEAK_GBS, tflops / FP32_PEAK_TFLOPS
@@ -195,10 +195,8 @@ ROWDOT_SHARED_SB = 16
 def kernel_name(fmt, M, tiled_units=None, cols=None):
     """The kernel a Q4_K / Q6_K launch of M positions over `tiled_units`
     (tile, unit) pairs of rows of `cols` columns runs (default tuning)."""
-    if M > 8:
-        return "prefill_kernel<%s,%d>" % (fmt, 1 if M <= 16 else 2)
-    if M >= (7 if fmt == "Q4_K" else 8):
-        return "matvec_mfma_kernel<%s,%d>" % (fmt, M)
+    if M >= 5 or (M >= 2 and cols is not None and cols <= 16 * 256):
+        return "chunk_kernel<%s,%d>" % (fmt, 1 if M <= 4 else 2 if M <= 8 else 4 if M <= 16 else 8)
     rowdot = os.environ.get("QMV_ROWDOT", "1") != "0"
     if fmt == "Q6_K" and M == 1 and cols is not None and rowdot and os.environ.get("QMV_ROWDOT_Q6K", "1") != "0":
         sb = cols // 256

@@ -257,7 +257,8 @@ int qmv_device_matvec_swiglu_f32(qmv_device_tensor gate, qmv_device_tensor up,
  * launch: every workgroup normalises the whole input in LDS, so no h is
  * written and one launch is saved. Otherwise a norm launch writes h to
  * d_normed (batch_count x K floats, clear of the input, the weights and the
- * outputs) and the projection reads it; after the call the contents of
+ * outputs) and the projection reads it, or the chunked matrix-core kernel of
+ * 2 to 32 positions applies it as it stages the input; after the call the contents of
  * d_normed are unspecified. Results are within the row tolerance of the
  * reference's norm followed by its matvec either way. Argument rules: those
  * of qmv_device_rms_norm_f32 (epsilon <= 0 fails) and of the plain entry
@@ -354,10 +355,15 @@ int qmv_device_count(void);
  * K is split across workgroups as far as that requires, and the last split to
  * finish adds the partials in split order.
  * target_waves, if set, instead grows the units per wave until about that
- * many waves cover the launch. Q4_K and Q6_K batches of at least
- * mfma_min_batch positions (default 7 for Q4_K, 8 for Q6_K; a value above
- * QMV_MAX_BATCH turns it off, and then batches run in launches of 8 on the
- * VALU path) run on the matrix cores, and so do Q5_0 launches of 5 to 8
+ * many waves cover the launch. By default launches of 2 to 8 positions run on
+ * the chunked matrix-core kernel where it is the faster one (by K, positions
+ * and size of the launch), which this plan does not describe; with any
+ * argument set they run as described here. Past 8 positions every launch runs
+ * on it, except that Q4_K and Q6_K batches below a set mfma_min_batch run in
+ * launches of 8 on the VALU path (a value above QMV_MAX_BATCH: all of them).
+ * Of the launches of up to 8 positions that are left, Q4_K and Q6_K batches
+ * of at least mfma_min_batch positions (default 7 for Q4_K, 8 for Q6_K) run on
+ * the matrix cores, and so do Q5_0 launches of 5 to 8
  * positions and Q8_0 launches of 4 to 8 (QMV_Q5_MFMA_MIN_BATCH /
  * QMV_Q8_MFMA_MIN_BATCH in the environment; 0 turns them off). Defaults may also come from the
  * QMV_TARGET_WAVES / QMV_UNITS_PER_WAVE / QMV_WAVES_PER_GROUP /

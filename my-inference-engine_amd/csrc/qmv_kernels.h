@@ -11,12 +11,10 @@
 
 #define QMV_MAX_WAVES 8
 #define QMV_MAX_JOBS 8
-/* Positions per launch: the VALU kernels take up to 8, the matrix-core
- * kernels (Q4_K, Q6_K) up to 32 in blocks of 16. */
+/* Positions per launch: the matvec kernels take up to 8, chunk_kernel up to
+ * 32. */
 #define QMV_VALU_MAX_POSITIONS 8
 #define QMV_MFMA_MAX_POSITIONS 32
-/* Tiles (one per wave) per prefill workgroup. */
-#define QMV_PF_TILES 4
 /* Floats of split-K workspace past the last partial: the VALU kernels' last
  * split loads a batch of partials from one base pointer and may read up to
  * this far beyond its tile's (discarding what it reads there). */
@@ -60,7 +58,7 @@ struct MatvecParams {
      * tile then has units x parts items of consecutive sub-blocks, and
      * units_per_wave (1) / units_per_split count items. */
     int parts;
-    int positions;    /* positions in this launch (the prefill kernel's position rows past it are padding) */
+    int positions;    /* positions in this launch */
     /* Fused greedy argmax (single tensor, M = 1; result non-null): tile and
      * group candidates (argmax_words(tiles) words), group and top arrival
      * counts (argmax_counts(tiles), zero between launches) and the result. */
@@ -83,10 +81,6 @@ struct MatvecParams {
      * (partials [tiles][splits][2][64] at job 0's offsets), so no second
      * count per tile pair is needed. */
     int pair_waves;
-    /* Prefill launches (set by launch_prefill): the splits publish their
-     * partials and stop, and a second kernel (pf_reduce_kernel) sums them and
-     * runs the epilogue; no arrival counts are taken. */
-    int pf_deferred;
 };
 
 /* One tensor of a row-major single-position launch: `w` holds the GGUF bytes
@@ -123,6 +117,37 @@ struct RowdotParams {
     int groups;
 };
 
+/* One tensor of a matrix-core launch of up to 32 positions (chunk_kernel). */
+struct BatchJob {
+    const uint8_t *w; /* tiled device layout */
+    float *y;         /* output, y[m * rows + row] */
+    const float *add; /* optional: y[m * rows + row] += add[m * ldadd + row] */
+    int rows;
+    int ldadd;
+    int group_begin; /* its first group of 16 rows among the launch's */
+};
+
+struct BatchParams {
+    BatchJob job[QMV_MAX_JOBS];
+    int njobs;
+    const float *x; /* x[m * cols + k], shared by all jobs */
+    int cols;       /* K */
+    int units;      /* tiled K-units per row */
+    int positions;
+    int swiglu;          /* jobs 0 (gate) and 1 (up), equal rows: job 0's y = up * silu(gate) */
+    const float *norm_w; /* optional: the RMSNorm of x by these weights, in the launch */
+    float norm_eps;
+    int groups;     /* groups of 16 rows in all */
+    int wg_groups;  /* of a workgroup (a multiple of the groups per wave; even with swiglu) */
+    int segs;       /* K in segments of seg_units units, the first seg_more of one more; a wave each */
+    int seg_units;
+    int seg_more;
+    int chunk_segs; /* of a workgroup (all of them in a fused launch) */
+    int chunk_wgs;  /* workgroups per chunk */
+    float *partials; /* [segs][positions][16 groups], launches that are not fused */
+    double *ssq;     /* with norm_w, launches that are not fused: [units][position slots] */
+};
+
 /* Row-major epilogues. */
 #define QMV_ROWDOT_STORE 0
 #define QMV_ROWDOT_SWIGLU 1
@@ -132,6 +157,11 @@ struct RowdotParams {
 inline size_t argmax_words(size_t tiles) { return tiles + (tiles + 63) / 64; }
 inline size_t argmax_counts(size_t tiles) { return (tiles + 63) / 64 + 1; }
 
+/* Matrix-core launch: nr rounds of 4 positions (1, 2, 4 or 8), r row groups
+ * per wave (1 or 2). */
+hipError_t launch_batch(int fmt, const BatchParams &p, int nr, int r, bool fused, int waves, hipStream_t s);
+/* LDS bytes of one unit's activations. */
+size_t batch_stage_bytes(int fmt, int nr);
 hipError_t launch_matvec(int fmt, const MatvecParams &p, int m, int grid, int waves, hipStream_t s);
 /* Row-major Q4_K launch at one position, one 64-weight group per lane.
  * Rows of at most 16 super-blocks: workgroups of QMV_ROWGROUP_WAVES waves
@@ -165,11 +195,6 @@ hipError_t launch_gather(int fmt, const uint8_t *w, const int *ids, int count, f
 hipError_t launch_repack(int fmt, const uint8_t *raw, uint8_t *out, int rows, int blocks_per_row,
                          int units, int blocks_per_unit, int block_bytes, int unit_bytes, int tiles,
                          hipStream_t s);
-/* Prefill launch (up to `rows` = 16 or 32 positions): grid = sum over jobs
- * of ceil(tiles / 4) tile groups x splits; for launches whose split-K finish
- * would take QMV_PF_DEFER_ROUNDS or more rounds of partial loads, followed by
- * the reduction kernel. */
-hipError_t launch_prefill(int fmt, const MatvecParams &p, int rows, int grid, hipStream_t s);
 /* Plain fp32 copy (n elements) as a kernel, e.g. from mapped host memory. */
 hipError_t launch_copy(const float *src, float *dst, size_t n, hipStream_t s);
 /* dst[0..n) = v (a fill kernel, no memset node). */

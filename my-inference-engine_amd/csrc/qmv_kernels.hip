@@ -1865,847 +1865,6 @@ matvec_mfma_kernel(MatvecParams p)
     finish_tile<M, 64>(p, w, blockDim.x >> 6, lane, red);
 }
 
-/* ---- Prefill batches (9..32 positions), all four formats: GEMM-shaped -------
- * A workgroup of four waves owns four consecutive 64-row tiles of one tensor
- * (one per wave) and a range of K-units. For each unit the 256 threads stage
- * the unit's activations of all positions once, as the three bf16 limbs (see
- * the matrix-core section above) laid out in MFMA A-fragment order, and each
- * wave then runs its tile's unit with A read from LDS: an activation is
- * loaded and split once per workgroup instead of once per wave, and the
- * codes a wave decodes serve every position block of 16. The next unit's
- * activations are loaded into registers, and its weight headers and first
- * codes issued, while the current unit computes. Each wave finishes its own
- * tile with the split-K protocol of finish_tile, so a position's arithmetic
- * does not depend on the other positions of the launch. */
-#define QMV_PF_WAVES QMV_PF_TILES
-/* Sub-block (Q4_K, of 8) and step (Q6_K, of 16) at which a wave issues the
- * next unit's first weight loads. */
-#ifndef QMV_PF_NEXT_SB
-#define QMV_PF_NEXT_SB 6
-#endif
-#ifndef QMV_PF_NEXT_T
-#define QMV_PF_NEXT_T 13
-#endif
-/* A prefill launch carries P position blocks of 16 (P = 1 for up to 16
- * positions, 2 for up to 32). */
-
-/* The staging buffer is addressed through an explicit LDS pointer type so
- * that every access compiles to ds_read / ds_write. */
-typedef __attribute__((address_space(3))) uint8_t lds_u8;
-
-/* An LDS offset that cannot be used before `dep` exists (see ptr_after):
- * keeps a sub-block's A-fragment reads from being hoisted across the unit. */
-__device__ __forceinline__ int lds_off_after(int off, float dep)
-{
-    asm("" : "+v"(off) : "v"(dep));
-    return off;
-}
-
-/* LDS image of one unit: fragment (limb L, position block pb, k-block b) is
- * 64 lanes x KL bf16, lane 16 kc + n holding A[n][KL kc .. KL kc + KL - 1] =
- * limb L of x[16 pb + n][4 KL b + KL kc ..]. */
-template <int KL, int P, int UW = 256> struct PfLayout {
-    static constexpr int kBlocks = UW / (4 * KL);      /* 8 (Q4_K), 16 (Q6_K) or 4 (Q5_0) */
-    static constexpr int kFrag = 64 * 2 * KL;          /* bytes per fragment */
-    static constexpr int kChunks = P * kBlocks * 64;   /* (pb, b, lane) chunks of KL activations */
-    static constexpr int kPerThread = kChunks / (QMV_PF_WAVES * 64);
-    static constexpr int kBytes = 3 * P * kBlocks * kFrag; /* 24 KB per position block */
-    __device__ static int offset(int limb, int pb, int b) { return ((limb * P + pb) * kBlocks + b) * kFrag; }
-    /* Q4_K: the sub-block sums of the activations as an A operand of 8
-     * sub-blocks (fragment (limb, pb): lane n < 16 holds limb L of
-     * sum(x[16 pb + n][32 s .. 32 s + 31]) for s = 0..7; lanes 16..63 hold
-     * zeros), after the limb images. */
-    static constexpr int kSxBytes = 3 * P * 64 * 16;
-    __device__ static int sx_offset(int limb, int pb) { return kBytes + (limb * P + pb) * 64 * 16; }
-};
-
-/* Chunk c of a unit: lane = c % 64, block b, position block pb. Blocks from
- * kleft on (past K in a partial last Q5_0 unit) are not read and stage
- * zeros. */
-template <int KL, int P, int UW = 256>
-__device__ __forceinline__ void pf_load_x(const float *xu, int ldx, int npos, int tid,
-                                          float (&xr)[PfLayout<KL, P, UW>::kPerThread][KL], int kleft = UW)
-{
-    using L = PfLayout<KL, P, UW>;
-#pragma unroll
-    for (int i = 0; i < L::kPerThread; ++i) {
-        const int c = tid + i * QMV_PF_WAVES * 64;
-        const int lane = c & 63, rest = c >> 6, b = rest % L::kBlocks, pb = rest / L::kBlocks;
-        const int kc = lane >> 4, n = lane & 15, pos = 16 * pb + n;
-        const bool in_k = UW == 256 || 4 * KL * b < kleft; /* K is a multiple of 256 for K-quants */
-        /* Rows past the batch read position 0 (in bounds) and stage zeros. */
-        const float *src = xu + (size_t)(pos < npos ? pos : 0) * ldx + (in_k ? 4 * KL * b + KL * kc : 0);
-        float v[KL];
-#pragma unroll
-        for (int j = 0; j < KL; ++j) v[j] = src[j];
-#pragma unroll
-        for (int j = 0; j < KL; ++j) xr[i][j] = pos < npos && in_k ? v[j] : 0.0f;
-    }
-}
-
-template <int KL, int P, int UW = 256, bool kSubSums = false>
-__device__ __forceinline__ void pf_store_limbs(lds_u8 *lds, int tid,
-                                               const float (&xr)[PfLayout<KL, P, UW>::kPerThread][KL])
-{
-    using L = PfLayout<KL, P, UW>;
-    typedef __bf16 frag_t __attribute__((__vector_size__(KL * sizeof(__bf16))));
-#pragma unroll
-    for (int i = 0; i < L::kPerThread; ++i) {
-        const int c = tid + i * QMV_PF_WAVES * 64;
-        const int lane = c & 63, rest = c >> 6, b = rest % L::kBlocks, pb = rest / L::kBlocks;
-        frag_t h, m, l;
-        x_limbs<KL>(xr[i], true, h, m, l);
-        typedef __attribute__((address_space(3))) frag_t lds_frag;
-        *(lds_frag *)(lds + L::offset(0, pb, b) + lane * 2 * KL) = h;
-        *(lds_frag *)(lds + L::offset(1, pb, b) + lane * 2 * KL) = m;
-        *(lds_frag *)(lds + L::offset(2, pb, b) + lane * 2 * KL) = l;
-        if constexpr (kSubSums) {
-            /* Sub-block b's sum for position 16 pb + n: this lane's KL
-             * activations in order, then the four lanes n + 16 kc (the
-             * chunk's k quarters) pairwise, the same bits in all four. */
-            static_assert(KL == 8, "Q4_K sub-blocks: four chunks of 8");
-            float t = xr[i][0];
-#pragma unroll
-            for (int j = 1; j < KL; ++j) t += xr[i][j];
-            t += __shfl_xor(t, 16);
-            t += __shfl_xor(t, 32);
-            if (lane < 16) {
-                const __bf16 th = (__bf16)t;
-                const float r = t - (float)th;
-                const __bf16 tm = (__bf16)r;
-                const __bf16 tl = (__bf16)(r - (float)tm);
-                typedef __attribute__((address_space(3))) __bf16 lds_bf16;
-                const int at = lane * 16 + b * 2;
-                *(lds_bf16 *)(lds + L::sx_offset(0, pb) + at) = th;
-                *(lds_bf16 *)(lds + L::sx_offset(1, pb) + at) = tm;
-                *(lds_bf16 *)(lds + L::sx_offset(2, pb) + at) = tl;
-            }
-        }
-    }
-}
-
-/* One Q4_K unit of this wave's tile against the staged activations; h and q0
- * hold the unit's headers and group-0 codes on entry and those of `next` on
- * return (the caller passes the unit itself when there is no next one: the
- * loads are then harmless repeats, and no branch splits the unrolled body). */
-template <int P>
-__device__ __forceinline__ void q4k_unit_pf(const uint8_t *slab, const uint8_t *next, const lds_u8 *lds, int lane,
-                                            f32x4_t (&acc)[P][4], uint4 (&h)[4], uint2 (&q0)[4])
-{
-    using L = PfLayout<8, P>;
-    const int kc = lane >> 4, n = lane & 15;
-    const int qoff = (1 + (kc >> 1)) * 1024 + n * 16 + 8 * (kc & 1);
-    const uint8_t *qsp = slab + qoff;
-    uint2 q[2][4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) q[0][g] = q0[g];
-    uint4 hn[4];
-    uint2 qn[4];
-    /* The minimum terms of the whole unit on the matrix cores:
-     * sum_s m_s * sum(x over sub-block s) per row and position, with the
-     * staged sub-block sums (exact limbs) as A, k = s < 8, and each row's 8
-     * six-bit minimums (exact in bf16) as B; then acc -= dmin * that once. */
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        const uint4 hg = h[g];
-        const uint32_t mlo = hg.z & 0x3f3f3f3fu;
-        const uint32_t mhi = ((hg.w >> 4) & 0x0f0f0f0fu) | ((hg.z >> 2) & 0x30303030u);
-        const bf16x8_t bm = {(__bf16)ubyte(mlo, 0), (__bf16)ubyte(mlo, 1), (__bf16)ubyte(mlo, 2),
-                             (__bf16)ubyte(mlo, 3), (__bf16)ubyte(mhi, 0), (__bf16)ubyte(mhi, 1),
-                             (__bf16)ubyte(mhi, 2), (__bf16)ubyte(mhi, 3)};
-        const float dmin = f16_bits_to_f32(hg.x >> 16);
-#pragma unroll
-        for (int pb = 0; pb < P; ++pb) {
-            typedef __attribute__((address_space(3))) const bf16x8_t lds_a;
-            f32x4_t dm = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int limb = 0; limb < 3; ++limb)
-                dm = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(lds_a *)(lds + L::sx_offset(limb, pb) + lane * 16), bm,
-                                                             dm, 0, 0, 0);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[pb][g][j] = fmaf(-dmin, dm[j], acc[pb][g][j]);
-        }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    /* Group c's codes load two steps before the step that converts them
-     * (step 2c - 1, below): group 1's here, groups 2 and 3 at steps 1 and
-     * 3, each into the buffer the group before last used. */
-    {
-        gu8 *nq = bytes_after(qsp + 2048, acc[0][1][0]);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) q[1][g] = gload8(nq + g * 256);
-    }
-    /* A software pipeline over the 8 sub-blocks: step sb issues its MFMAs,
-     * the code conversion of sub-block sb + 1 (b -> bn) and the scale FMAs
-     * of sub-block sb - 1 (dp, sp), none of which depends on the others, so
-     * the VALU work runs under the matrix-core work. acc takes the
-     * sub-blocks in order, as without the pipeline. */
-    bf16x8_t b[4], bn[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) b[g] = q4_codes_bf16(q[0][g].x, q[0][g].y, false);
-    f32x4_t dp[P][4];
-    float sp[4];
-    /* One position block: the activation fragments of sub-block sb + 1 are
-     * read from LDS during step sb, as in q6k_unit_pf (gate|up at 16
-     * positions 34.1 -> 32.2 µs in a cold graph of its launches, the
-     * 16-position decode set 2.582 -> 2.572 ms). Two blocks keep the reads
-     * in the step: the 24 more VGPRs take the kernel from 248 to 267 and to
-     * one wave per SIMD (gate|up at 32 positions 47.2 -> 60.0 µs). */
-    constexpr bool kAhead = P == 1;
-    typedef __attribute__((address_space(3))) const bf16x8_t lds_a;
-    bf16x8_t fa[P][3], fn[P][3];
-    if constexpr (kAhead) {
-#pragma unroll
-        for (int pb = 0; pb < P; ++pb) {
-            const lds_u8 *la = lds + lds_off_after(lane * 16, acc[pb][3][3]);
-#pragma unroll
-            for (int l = 0; l < 3; ++l) fa[pb][l] = *(lds_a *)(la + L::offset(l, pb, 0));
-        }
-    }
-#pragma unroll
-    for (int sb = 0; sb < 8; ++sb) {
-        const bool high = sb & 1;
-        if (high && (sb + 3) / 2 < 4) {
-            const int cn = (sb + 3) / 2;
-            gu8 *nq = bytes_after(qsp + cn * 2048, acc[0][1][0]);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) q[cn & 1][g] = gload8(nq + g * 256);
-        }
-        if (sb == QMV_PF_NEXT_SB) {
-            gu8 *np = bytes_after(next, acc[0][2][0]);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                hn[g] = gload16(np + n * 16 + g * 256);
-                qn[g] = gload8(np + qoff + g * 256);
-            }
-        }
-        if (sb + 1 < 8)
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                bn[g] = q4_codes_bf16(q[((sb + 1) >> 1) & 1][g].x, q[((sb + 1) >> 1) & 1][g].y, !high);
-        float sa[4];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const uint4 hg = h[g];
-            const float dd = f16_bits_to_f32(hg.x);
-            const uint32_t scw = sb < 4 ? hg.y & 0x3f3f3f3fu : (hg.w & 0x0f0f0f0fu) | ((hg.y >> 2) & 0x30303030u);
-            sa[g] = dd * ubyte(scw, sb & 3);
-        }
-        f32x4_t d[P][4];
-#pragma unroll
-        for (int pb = 0; pb < P; ++pb) {
-            bf16x8_t a0, a1, a2;
-            if constexpr (kAhead) {
-                a0 = fa[pb][0];
-                a1 = fa[pb][1];
-                a2 = fa[pb][2];
-                if (sb + 1 < 8)
-#pragma unroll
-                    for (int l = 0; l < 3; ++l) fn[pb][l] = *(lds_a *)(lds + lane * 16 + L::offset(l, pb, sb + 1));
-            } else {
-                const lds_u8 *la = lds + lds_off_after(lane * 16, acc[pb][3][3]);
-                a0 = *(lds_a *)(la + L::offset(0, pb, sb));
-                a1 = *(lds_a *)(la + L::offset(1, pb, sb));
-                a2 = *(lds_a *)(la + L::offset(2, pb, sb));
-            }
-#pragma unroll
-            for (int g = 0; g < 4; ++g) d[pb][g] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int g = 0; g < 4; ++g) d[pb][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[g], d[pb][g], 0, 0, 0);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) d[pb][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[g], d[pb][g], 0, 0, 0);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) d[pb][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b[g], d[pb][g], 0, 0, 0);
-        }
-        if (sb > 0)
-#pragma unroll
-            for (int pb = 0; pb < P; ++pb)
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) acc[pb][g][j] = fmaf(sp[g], dp[pb][g][j], acc[pb][g][j]);
-        /* One step per scheduling region: only the pipeline's hand-over
-         * values live across it. */
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            b[g] = bn[g];
-            sp[g] = sa[g];
-#pragma unroll
-            for (int pb = 0; pb < P; ++pb) dp[pb][g] = d[pb][g];
-        }
-        if constexpr (kAhead)
-#pragma unroll
-            for (int pb = 0; pb < P; ++pb)
-#pragma unroll
-                for (int l = 0; l < 3; ++l) fa[pb][l] = fn[pb][l];
-    }
-#pragma unroll
-    for (int pb = 0; pb < P; ++pb)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[pb][g][j] = fmaf(sp[g], dp[pb][g][j], acc[pb][g][j]);
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        h[g] = hn[g];
-        q0[g] = qn[g];
-    }
-}
-
-/* Q6_K: sc, dg and w0 (the first (G, hf) pair's words) hold this unit's on
- * entry and those of `next` on return (as for Q4_K). */
-template <int P>
-__device__ __forceinline__ void q6k_unit_pf(const uint8_t *slab, const uint8_t *next, const lds_u8 *lds, int lane,
-                                            f32x4_t (&acc)[P][4], uint4 (&sc)[4], uint32_t (&dgw)[4],
-                                            uint32_t (&w0)[4][3])
-{
-    using L = PfLayout<4, P>;
-    const int kc = lane >> 4, n = lane & 15;
-    const int woff = n * 16 + 4 * kc;
-    const uint8_t *wp = slab + woff;
-    float dg[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) dg[g] = f16_bits_to_f32(dgw[g] & 0xffffu);
-    uint32_t w[3][4][3];
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-#pragma unroll
-        for (int e = 0; e < 3; ++e) w[0][g][e] = w0[g][e];
-    uint4 scn[4];
-    uint32_t dgn[4], wn[4][3];
-    /* The code words of pair pn (the ql / qh dwords of four sub-blocks) into
-     * buffer pn % 3: pair 1 here, pairs 2 and 3 at steps 2 and 6, so each
-     * lands 4-5 steps before the step that converts its first codes (step
-     * 4 pn - 1) and overwrites the buffer of a pair converted for the last
-     * time at step 4 (pn - 3) + 2. Two buffers (loads 3 steps ahead) ran
-     * Q6_K at 32 positions 43.6 against 43.3 µs, at 16 35.7 against 35.3. */
-    auto load_pair = [&](int pn, gu8 *base) {
-        const int Gn = pn >> 1, hn = pn & 1;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            w[pn % 3][g][0] = *(gu32 *)(base + (4 * Gn + hn) * 1024 + g * 256);
-            w[pn % 3][g][1] = *(gu32 *)(base + (4 * Gn + 2 + hn) * 1024 + g * 256);
-            w[pn % 3][g][2] = *(gu32 *)(base + (8 + 2 * Gn + hn) * 1024 + g * 256);
-        }
-    };
-    load_pair(1, bytes_after(wp, acc[0][1][0]));
-    /* Step t's code operands: one combined operand per code (q - 32, exact
-     * in bf16), converted once for every position block. The two-operand
-     * form of the M <= 8 kernel (q6_codes_bf16) would double the MFMAs of
-     * each block, and using it for one block only would make a position's
-     * rounding depend on the number of positions in its launch. */
-    auto decode = [&](int t, bf16x4_t (&b)[4]) {
-        const int pr = t >> 2, r = t & 3;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const uint32_t lw = w[pr % 3][g][r & 1];
-            const uint32_t hw = w[pr % 3][g][2];
-            const uint32_t c = codes(((lw >> (4 * (r >> 1))) & 0x0f0f0f0fu) | (((hw >> (2 * r)) & 0x03030303u) << 4));
-#pragma unroll
-            for (int i = 0; i < 4; ++i) b[g][i] = (__bf16)(ubyte(c, i) - 32.0f); /* exact: -32..31 */
-        }
-    };
-    /* A software pipeline over the 16 steps: step t issues its MFMAs, the
-     * code conversion of step t + 1 (b -> bn) and the scale FMAs of step
-     * t - 1 (dp, sp), none of which depends on the others, so the VALU work
-     * runs under the matrix-core work instead of before and after it. acc
-     * takes the steps in order, as without the pipeline. */
-    bf16x4_t b[4], bn[4];
-    decode(0, b);
-    f32x4_t dp[P][4];
-    float sp[4];
-    /* The staged activation fragments of step t (sub-block sub_of(t)) are
-     * read from LDS during step t - 1 (fa: this step's, fn: the next
-     * step's), so no step waits for its LDS reads: M = 32 decode set
-     * 3.430-3.456 -> 3.382-3.387 ms (Q6_K launches 44.8 -> 43.6 µs). The
-     * Q4_K unit keeps its reads in the step: the same change takes it from
-     * 248 to 267 VGPRs, one wave per SIMD, and the set to 3.81 against 3.47
-     * ms. */
-    auto sub_of = [](int t) { return 8 * (t >> 3) + 2 * (t & 3) + ((t >> 2) & 1); };
-    typedef __attribute__((address_space(3))) const bf16x4_t lds_a;
-    bf16x4_t fa[P][3], fn[P][3];
-#pragma unroll
-    for (int pb = 0; pb < P; ++pb) {
-        const lds_u8 *la = lds + lds_off_after(lane * 8, acc[pb][3][3]);
-#pragma unroll
-        for (int l = 0; l < 3; ++l) fa[pb][l] = *(lds_a *)(la + L::offset(l, pb, sub_of(0)));
-    }
-#pragma unroll
-    for (int t = 0; t < 16; ++t) {
-        const int pr = t >> 2, r = t & 3;
-        const int G = pr >> 1;
-        const int j = 8 * G + 2 * r + (pr & 1);
-        if (t == 2 || t == 6) load_pair((t + 6) / 4, bytes_after(wp, acc[0][1][0]));
-        if (t == QMV_PF_NEXT_T) {
-            gu8 *np = bytes_after(next, acc[0][2][0]);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                scn[g] = gload16(np + 12 * 1024 + (16 * g + n) * 16);
-                dgn[g] = *(gu16 *)(np + 13312 + (16 * g + n) * 2);
-                wn[g][0] = *(gu32 *)(np + woff + 0 * 1024 + g * 256);
-                wn[g][1] = *(gu32 *)(np + woff + 2 * 1024 + g * 256);
-                wn[g][2] = *(gu32 *)(np + woff + 8 * 1024 + g * 256);
-            }
-        }
-        if (t + 1 < 16) decode(t + 1, bn);
-        float s[4];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) s[g] = dg[g] * sbyte(word(sc[g], j >> 2), j & 3);
-        f32x4_t d[P][4];
-#pragma unroll
-        for (int pb = 0; pb < P; ++pb) {
-            const bf16x4_t a0 = fa[pb][0], a1 = fa[pb][1], a2 = fa[pb][2];
-            if (t + 1 < 16) {
-                const lds_u8 *la = lds + lane * 8;
-#pragma unroll
-                for (int l = 0; l < 3; ++l) fn[pb][l] = *(lds_a *)(la + L::offset(l, pb, sub_of(t + 1)));
-            }
-#pragma unroll
-            for (int g = 0; g < 4; ++g) d[pb][g] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int g = 0; g < 4; ++g) d[pb][g] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0, b[g], d[pb][g], 0, 0, 0);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) d[pb][g] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, b[g], d[pb][g], 0, 0, 0);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) d[pb][g] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a2, b[g], d[pb][g], 0, 0, 0);
-        }
-        if (t > 0)
-#pragma unroll
-            for (int pb = 0; pb < P; ++pb)
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[pb][g][i] = fmaf(sp[g], dp[pb][g][i], acc[pb][g][i]);
-        /* One step per scheduling region: only the pipeline's hand-over
-         * values live across it. */
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            b[g] = bn[g];
-            sp[g] = s[g];
-#pragma unroll
-            for (int pb = 0; pb < P; ++pb) dp[pb][g] = d[pb][g];
-        }
-#pragma unroll
-        for (int pb = 0; pb < P; ++pb)
-#pragma unroll
-            for (int l = 0; l < 3; ++l) fa[pb][l] = fn[pb][l];
-    }
-#pragma unroll
-    for (int pb = 0; pb < P; ++pb)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[pb][g][i] = fmaf(sp[g], dp[pb][g][i], acc[pb][g][i]);
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        sc[g] = scn[g];
-        dgw[g] = dgn[g];
-#pragma unroll
-        for (int e = 0; e < 3; ++e) w0[g][e] = wn[g][e];
-    }
-}
-
-/* Q8_0: as q50_unit_pf with one code operand per block (q8_codes_bf16); dw
- * and q0 (block 0's codes) carry over to `next`. */
-template <int P>
-__device__ __forceinline__ void q80_unit_pf(const uint8_t *slab, const uint8_t *next, const lds_u8 *lds, int lane,
-                                            int nvalid, f32x4_t (&acc)[P][4], uint2 (&dw)[4], uint2 (&q0)[4])
-{
-    using L = PfLayout<8, P, 128>;
-    const int kc = lane >> 4, n = lane & 15;
-    const int qoff = (kc >> 1) * 1024 + n * 16 + 8 * (kc & 1); /* + 2048 j + 256 g */
-    const uint8_t *qsp = slab + qoff;
-    uint2 q[2][4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) q[0][g] = q0[g];
-    uint2 dn[4], qn[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        if (j + 1 < 4) {
-            gu8 *nq = bytes_after(qsp + (j + 1) * 2048, acc[0][1][0]);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) q[(j + 1) & 1][g] = gload8(nq + g * 256);
-        }
-        if (j == 2) {
-            gu8 *np = bytes_after(next, acc[0][2][0]);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                dn[g] = gload8(np + 8192 + (16 * g + n) * 8);
-                qn[g] = gload8(np + qoff + g * 256);
-            }
-        }
-        if (j < nvalid) { /* uniform */
-            bf16x8_t b[4];
-            float sd[4];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                b[g] = q8_codes_bf16(q[j & 1][g].x, q[j & 1][g].y);
-                sd[g] = f16_bits_to_f32(word(dw[g], j >> 1) >> (16 * (j & 1)));
-            }
-#pragma unroll
-            for (int pb = 0; pb < P; ++pb) {
-                typedef __attribute__((address_space(3))) const bf16x8_t lds_a;
-                const lds_u8 *la = lds + lds_off_after(lane * 16, acc[pb][3][3]);
-                const bf16x8_t a0 = *(lds_a *)(la + L::offset(0, pb, j));
-                const bf16x8_t a1 = *(lds_a *)(la + L::offset(1, pb, j));
-                const bf16x8_t a2 = *(lds_a *)(la + L::offset(2, pb, j));
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    f32x4_t d = {0.0f, 0.0f, 0.0f, 0.0f};
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b[g], d, 0, 0, 0);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b[g], d, 0, 0, 0);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b[g], d, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[pb][g][i] = fmaf(sd[g], d[i], acc[pb][g][i]);
-                }
-            }
-        }
-        /* One block's codes live at a time. */
-        __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        dw[g] = dn[g];
-        q0[g] = qn[g];
-    }
-}
-
-/* Q5_0: the unit's four blocks against the staged activations, each block's
- * two code operands (q5_codes_bf16) converted once for every position block.
- * dw (the four d's), qh (the four qh words) and q0 (block 0's codes) hold
- * this unit's on entry and those of `next` on return (as for Q4_K). Blocks
- * from nvalid on lie past K (zero bytes, zeros staged) and are skipped. */
-template <int P>
-__device__ __forceinline__ void q50_unit_pf(const uint8_t *slab, const uint8_t *next, const lds_u8 *lds, int lane,
-                                            int nvalid, f32x4_t (&acc)[P][4], uint2 (&dw)[4], uint4 (&qh)[4],
-                                            uint2 (&q0)[4])
-{
-    using L = PfLayout<8, P, 128>;
-    const int kc = lane >> 4, n = lane & 15;
-    const int qoff = n * 16 + 8 * (kc & 1); /* + 1024 j + 256 g */
-    const uint8_t *qsp = slab + qoff;
-    const int nsh = 4 * (kc >> 1), bsh = 8 * kc;
-    uint2 q[2][4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) q[0][g] = q0[g];
-    uint2 dn[4], qn[4];
-    uint4 hn[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        if (j + 1 < 4) {
-            gu8 *nq = bytes_after(qsp + (j + 1) * 1024, acc[0][1][0]);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) q[(j + 1) & 1][g] = gload8(nq + g * 256);
-        }
-        if (j == 2) {
-            gu8 *np = bytes_after(next, acc[0][2][0]);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                dn[g] = gload8(np + 5120 + (16 * g + n) * 8);
-                hn[g] = gload16(np + 4096 + (16 * g + n) * 16);
-                qn[g] = gload8(np + qoff + g * 256);
-            }
-        }
-        if (j < nvalid) { /* uniform */
-            bf16x8_t bl[4], bh[4];
-            float sd[4];
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                q5_codes_bf16((q[j & 1][g].x >> nsh) & 0x0f0f0f0fu, (q[j & 1][g].y >> nsh) & 0x0f0f0f0fu,
-                              (word(qh[g], j) >> bsh) & 0xffu, bl[g], bh[g]);
-                sd[g] = f16_bits_to_f32(word(dw[g], j >> 1) >> (16 * (j & 1)));
-            }
-#pragma unroll
-            for (int pb = 0; pb < P; ++pb) {
-                typedef __attribute__((address_space(3))) const bf16x8_t lds_a;
-                const lds_u8 *la = lds + lds_off_after(lane * 16, acc[pb][3][3]);
-                const bf16x8_t a0 = *(lds_a *)(la + L::offset(0, pb, j));
-                const bf16x8_t a1 = *(lds_a *)(la + L::offset(1, pb, j));
-                const bf16x8_t a2 = *(lds_a *)(la + L::offset(2, pb, j));
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    f32x4_t d = {0.0f, 0.0f, 0.0f, 0.0f};
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, bl[g], d, 0, 0, 0);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, bh[g], d, 0, 0, 0);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, bl[g], d, 0, 0, 0);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, bh[g], d, 0, 0, 0);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, bl[g], d, 0, 0, 0);
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, bh[g], d, 0, 0, 0);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[pb][g][i] = fmaf(sd[g], d[i], acc[pb][g][i]);
-                }
-            }
-        }
-        /* One block's codes live at a time. */
-        __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        dw[g] = dn[g];
-        qh[g] = hn[g];
-        q0[g] = qn[g];
-    }
-}
-
-/* The workgroup's place in a prefill launch: job, tile group, K-split; this
- * wave's tile is 4 * group + wave (it may lie past the job's last tile, and
- * then the wave only helps stage). */
-__device__ __forceinline__ WgWork locate_pf(const MatvecParams &p, int wave)
-{
-    WgWork w;
-    const int j = job_of_block(p);
-    const MatvecJob &job = p.job[j];
-    const int local = blockIdx.x - job.wg_begin;
-    const int group = local / job.splits;
-    w.job = j;
-    w.split = local - group * job.splits;
-    w.tile = group * QMV_PF_WAVES + wave;
-    w.u_begin = w.split * job.units_per_split;
-    w.u_end = min(w.u_begin + job.units_per_split, p.units);
-    return w;
-}
-
-/* Prefill epilogue. A wave's tile values v(m) = val[m * 64 + lane] (m <
- * npos) live in its LDS slice, and the loops over positions stay rolled:
- * unrolled over 32 positions, the epilogue alone would be several times the
- * instruction cache. Same split-K, addend and SwiGLU protocols (and the same
- * partial order) as finish_tile / emit_tile. */
-typedef __attribute__((address_space(3))) float lds_f32;
-
-template <int MP>
-__device__ __forceinline__ void pf_emit(const MatvecParams &p, const WgWork &w, int lane, lds_f32 *val, int npos)
-{
-    const MatvecJob &job = p.job[w.job];
-    const int row = w.tile * 64 + lane;
-    const bool valid = row < job.rows;
-    if (job.add != nullptr && valid)
-        for (int m = 0; m < npos; ++m) val[m * 64 + lane] += job.add[(size_t)m * job.ldadd + row];
-    if (p.swiglu) {
-        const MatvecJob &out = p.job[0];
-        float *mine = p.pair_vals + ((size_t)w.job * out.tiles + w.tile) * MP * 64 + lane;
-        for (int m = 0; m < npos; ++m) store_partial(mine + m * 64, val[m * 64 + lane]);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        unsigned prev = 0;
-        if (lane == 0)
-            prev = __hip_atomic_fetch_add(p.pair_count + w.tile * QMV_COUNTER_STRIDE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        prev = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_readlane(prev, 0));
-        if (prev == 0u) return;
-        asm volatile("" ::: "memory");
-        const float *other = p.pair_vals + ((size_t)(1 - w.job) * out.tiles + w.tile) * MP * 64 + lane;
-        for (int m0 = 0; m0 < npos; m0 += 8) {
-            float o[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) o[i] = m0 + i < npos ? load_partial(other + (m0 + i) * 64) : 0.0f;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                if (m0 + i >= npos) break;
-                const float v = val[(m0 + i) * 64 + lane];
-                const float g = w.job == 0 ? v : o[i];
-                const float u = w.job == 0 ? o[i] : v;
-                if (valid) out.y[(size_t)(m0 + i) * out.ldy + row] = swiglu_value(g, u);
-            }
-        }
-        if (lane == 0) __hip_atomic_store(p.pair_count + w.tile * QMV_COUNTER_STRIDE, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return;
-    }
-    if (valid)
-        for (int m = 0; m < npos; ++m) job.y[(size_t)m * job.ldy + row] = val[m * 64 + lane];
-}
-
-template <int MP>
-__device__ __forceinline__ void pf_finish(const MatvecParams &p, const WgWork &w, int lane, lds_f32 *val, int npos)
-{
-    const MatvecJob &job = p.job[w.job];
-    const int S = job.splits;
-    if (S > 1) {
-        /* The tile's partials, split-major; within a split, quad q of lane l
-         * (position rows 4q..4q+3) at [split][q][l], so a lane publishes and
-         * reads them with 16-byte accesses (MP / 4 per split instead of MP)
-         * and each access of the wave covers 1 KiB of consecutive bytes:
-         * M = 32 set 3.82 -> 3.74 ms. The accesses are agent-coherent (sc1),
-         * as store_partial's, written as global instructions (the buffer
-         * forms of the same accesses ran the set in 4.6 ms). The stores are
-         * complete at the explicit wait below; the loads complete inside
-         * their own asm statement, so no value is read before it lands. */
-        float *part = p.partials + job.partial_offset + ((size_t)w.tile * S) * MP * 64;
-        unsigned *count = p.counters + job.counter_offset + w.tile * QMV_COUNTER_STRIDE;
-        float *mine = part + ((size_t)w.split * (MP / 4) * 64 + lane) * 4;
-#pragma unroll
-        for (int q = 0; q < MP / 4; ++q) {
-            const f32x4_t v = {val[(4 * q) * 64 + lane], val[(4 * q + 1) * 64 + lane], val[(4 * q + 2) * 64 + lane],
-                               val[(4 * q + 3) * 64 + lane]};
-            asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(mine + q * 256), "v"(v) : "memory");
-        }
-        /* Deferred finish: pf_reduce_kernel, launched next, sums the tile. */
-        if (p.pf_deferred) return;
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        unsigned prev = 0;
-        if (lane == 0) prev = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        prev = __builtin_amdgcn_readfirstlane(__builtin_amdgcn_readlane(prev, 0));
-        if (prev != (unsigned)S - 1u) return;
-        asm volatile("" ::: "memory");
-        /* 16 quads per round (two splits of 32 position rows, or four of 16),
-         * splits past the last repeating it and not added; each position is
-         * summed in split order, as sum_partials does. */
-        static_assert(MP == 32 || MP == 16, "position rows of a prefill launch");
-        constexpr int SB = 64 / MP;
-        float sum[MP];
-        for (int s0 = 0; s0 < S; s0 += SB) {
-            f32x4_t v[16];
-            const float *pk[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                pk[k] = part + ((size_t)min(s0 + (MP == 32 ? k / 2 : k), S - 1) * (MP / 4) * 64 + lane) * 4 +
-                        (MP == 32 ? (k & 1) * 1024 : 0);
-            asm volatile("global_load_dwordx4 %0, %16, off sc1\n global_load_dwordx4 %1, %16, off offset:1024 sc1\n"
-                         "global_load_dwordx4 %2, %16, off offset:2048 sc1\n global_load_dwordx4 %3, %16, off offset:3072 sc1\n"
-                         "global_load_dwordx4 %4, %17, off sc1\n global_load_dwordx4 %5, %17, off offset:1024 sc1\n"
-                         "global_load_dwordx4 %6, %17, off offset:2048 sc1\n global_load_dwordx4 %7, %17, off offset:3072 sc1\n"
-                         "global_load_dwordx4 %8, %18, off sc1\n global_load_dwordx4 %9, %18, off offset:1024 sc1\n"
-                         "global_load_dwordx4 %10, %18, off offset:2048 sc1\n global_load_dwordx4 %11, %18, off offset:3072 sc1\n"
-                         "global_load_dwordx4 %12, %19, off sc1\n global_load_dwordx4 %13, %19, off offset:1024 sc1\n"
-                         "global_load_dwordx4 %14, %19, off offset:2048 sc1\n global_load_dwordx4 %15, %19, off offset:3072 sc1\n"
-                         "s_waitcnt vmcnt(0)"
-                         : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]),
-                           "=&v"(v[7]), "=&v"(v[8]), "=&v"(v[9]), "=&v"(v[10]), "=&v"(v[11]), "=&v"(v[12]),
-                           "=&v"(v[13]), "=&v"(v[14]), "=&v"(v[15])
-                         : "v"(pk[0]), "v"(pk[1]), "v"(pk[2]), "v"(pk[3])
-                         : "memory");
-#pragma unroll
-            for (int k = 0; k < SB; ++k)
-                if (s0 + k < S)
-#pragma unroll
-                    for (int q = 0; q < MP / 4; ++q)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const float x = v[k * (MP / 4) + q][e];
-                            sum[4 * q + e] = s0 + k == 0 ? x : sum[4 * q + e] + x;
-                        }
-        }
-#pragma unroll
-        for (int i = 0; i < MP; ++i)
-            if (i < npos) val[i * 64 + lane] = sum[i];
-        if (lane == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    pf_emit<MP>(p, w, lane, val, npos);
-}
-
-template <int FMT, int P>
-__global__ void __launch_bounds__(QMV_PF_WAVES * 64) prefill_kernel(MatvecParams p)
-{
-    constexpr int KL = FMT == QMV_FMT_Q6_K ? 4 : 8;
-    constexpr int SLAB = UnitOf<FMT>::kBytes * 64;
-    constexpr int UW = UnitOf<FMT>::kWeights;
-    constexpr int MP = 16 * P; /* position rows of the launch */
-    using L = PfLayout<KL, P, UW>;
-    /* The combine buffer (each wave's tile, MP x 64 floats) reuses the
-     * staging buffer. */
-    constexpr bool kSubSums = FMT == QMV_FMT_Q4_K; /* the minimum terms on the matrix cores (q4k_unit_pf) */
-    constexpr int kStage = L::kBytes + (kSubSums ? L::kSxBytes : 0);
-    constexpr int kLds = kStage > QMV_PF_WAVES * MP * 64 * 4 ? kStage : QMV_PF_WAVES * MP * 64 * 4;
-    __shared__ __attribute__((aligned(16))) uint8_t lds_buf[kLds];
-    lds_u8 *lds = (lds_u8 *)lds_buf;
-
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const WgWork w = locate_pf(p, wave);
-    const MatvecJob &job = p.job[w.job];
-    const bool active = w.tile < job.tiles;
-    const int npos = p.positions;
-    const uint8_t *wtile = job.w + (size_t)(active ? w.tile : 0) * p.units * SLAB;
-    const int kc = lane >> 4, n = lane & 15;
-
-    f32x4_t acc[P][4];
-#pragma unroll
-    for (int pb = 0; pb < P; ++pb)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) acc[pb][g] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-
-    /* First unit's weights (this wave's tile) and activations. */
-    uint4 h[4];
-    uint2 q0[4], dw[4];
-    uint32_t dgw[4], w0[4][3];
-    const uint8_t *first = wtile + (size_t)w.u_begin * SLAB;
-    if constexpr (FMT == QMV_FMT_Q8_0) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            dw[g] = *(const uint2 *)(first + 8192 + (16 * g + n) * 8);
-            q0[g] = *(const uint2 *)(first + (kc >> 1) * 1024 + n * 16 + 8 * (kc & 1) + g * 256);
-        }
-    } else if constexpr (FMT == QMV_FMT_Q5_0) {
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            dw[g] = *(const uint2 *)(first + 5120 + (16 * g + n) * 8);
-            h[g] = ld16(first + 4096 + (16 * g + n) * 16);
-            q0[g] = *(const uint2 *)(first + n * 16 + 8 * (kc & 1) + g * 256);
-        }
-    } else if constexpr (FMT == QMV_FMT_Q4_K) {
-        const int qoff = (1 + (kc >> 1)) * 1024 + n * 16 + 8 * (kc & 1);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            h[g] = ld16(first + n * 16 + g * 256);
-            q0[g] = *(const uint2 *)(first + qoff + g * 256);
-        }
-    } else {
-        const int woff = n * 16 + 4 * kc;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            h[g] = ld16(first + 12 * 1024 + (16 * g + n) * 16);
-            dgw[g] = *(const unsigned short *)(first + 13312 + (16 * g + n) * 2);
-            w0[g][0] = *(const uint32_t *)(first + woff + 0 * 1024 + g * 256);
-            w0[g][1] = *(const uint32_t *)(first + woff + 2 * 1024 + g * 256);
-            w0[g][2] = *(const uint32_t *)(first + woff + 8 * 1024 + g * 256);
-        }
-    }
-    float xr[L::kPerThread][KL];
-    pf_load_x<KL, P, UW>(p.x + (size_t)w.u_begin * UW, p.ldx, npos, tid, xr, p.cols - w.u_begin * UW);
-    if constexpr (kSubSums) {
-        /* Lanes 16..63 of the sub-sum fragments stay zero (only lanes 0..15
-         * are rewritten per unit); the first barrier below orders this. */
-        typedef __attribute__((address_space(3))) u32v4 lds_v4;
-        for (int i = tid; i < L::kSxBytes / 16; i += QMV_PF_WAVES * 64)
-            *(lds_v4 *)(lds + L::kBytes + 16 * i) = u32v4{0u, 0u, 0u, 0u};
-    }
-
-    for (int u = w.u_begin; u < w.u_end; ++u) {
-        __syncthreads(); /* every wave is done with the previous unit's image */
-        pf_store_limbs<KL, P, UW, kSubSums>(lds, tid, xr);
-        __syncthreads();
-        if (u + 1 < w.u_end)
-            pf_load_x<KL, P, UW>(p.x + (size_t)(u + 1) * UW, p.ldx, npos, tid, xr, p.cols - (u + 1) * UW);
-        const uint8_t *slab = wtile + (size_t)u * SLAB;
-        const uint8_t *next = u + 1 < w.u_end ? slab + SLAB : slab;
-        if (active) {
-            if constexpr (FMT == QMV_FMT_Q5_0 || FMT == QMV_FMT_Q8_0) {
-                const int kleft = p.cols - u * UW; /* K is a multiple of 32 */
-                const int nvalid = kleft >= 128 ? 4 : kleft / 32;
-                if constexpr (FMT == QMV_FMT_Q5_0) q50_unit_pf<P>(slab, next, lds, lane, nvalid, acc, dw, h, q0);
-                else q80_unit_pf<P>(slab, next, lds, lane, nvalid, acc, dw, q0);
-            } else if constexpr (FMT == QMV_FMT_Q4_K) {
-                q4k_unit_pf<P>(slab, next, lds, lane, acc, h, q0);
-            } else {
-                q6k_unit_pf<P>(slab, next, lds, lane, acc, h, dgw, w0);
-            }
-        }
-    }
-
-    /* Each wave transposes its tile through its own slice of the (now free)
-     * staging buffer, then finishes the tile on its own. */
-    __syncthreads();
-    lds_f32 *val = (lds_f32 *)lds + wave * MP * 64;
-#pragma unroll
-    for (int pb = 0; pb < P; ++pb)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) val[(16 * pb + 4 * kc + j) * 64 + 16 * g + n] = acc[pb][g][j];
-    if (!active) return;
-    pf_finish<MP>(p, w, lane, val, npos);
-}
-
 /* ---- dequantisation kernel --------------------------------------------------
  * One wave per (tile, unit); lane = row. Rows outside [first, first+count)
  * and blocks past K are skipped. */
@@ -3837,112 +2996,6 @@ hipError_t launch_argmax(const float *logits, int n, float *bval, int *bidx, int
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(argmax_stage2, dim3(1), dim3(64), 0, s, bval, bidx, bbad, nblocks, result);
-    return hipGetLastError();
-}
-
-/* The deferred split-K finish of a prefill launch: thread (tile, quad q,
- * lane) sums the quad of position rows 4q..4q+3 of row 64 tile + lane over
- * the tile's splits, in split order as pf_finish does (so the values are
- * those of the in-kernel finish bit for bit), with up to 16 splits' loads in
- * flight at once (one round for the usual 14-15 splits; batches of 8 and
- * workgroups of 256 threads measured 0.2-0.5% slower on the M = 32 decode
- * set), then applies pf_emit's addend and SwiGLU epilogues (the up
- * sums of job 1 are read alongside, so no pairing protocol is needed). The
- * partials were written by the previous kernel on this stream, whose end
- * makes them visible: plain loads. */
-template <int MP>
-__global__ void __launch_bounds__(64) pf_reduce_kernel(MatvecParams p)
-{
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = gid & 63;
-    const int q = (gid >> 6) % (MP / 4);
-    int t = (gid >> 6) / (MP / 4);
-    const int nj = p.swiglu ? 1 : p.njobs;
-    int j = 0;
-    while (j < nj && t >= p.job[j].tiles) {
-        t -= p.job[j].tiles;
-        ++j;
-    }
-    if (j >= nj) return;
-    const MatvecJob &job = p.job[j];
-    const int row = t * 64 + lane;
-    if (row >= job.rows) return;
-    const int S = job.splits;
-    auto total = [&](const MatvecJob &jb) {
-        const float *part = p.partials + jb.partial_offset + ((size_t)t * S) * MP * 64 + ((size_t)q * 64 + lane) * 4;
-        f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int s0 = 0; s0 < S; s0 += 16) {
-            /* splits past the last repeat it and are not added */
-            f32x4_t v[16];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = *(const f32x4_t *)(part + (size_t)min(s0 + i, S - 1) * (MP / 4) * 256);
-#pragma unroll
-            for (int i = 0; i < 16; ++i)
-                if (s0 + i < S) sum = s0 + i == 0 ? v[i] : sum + v[i];
-        }
-        return sum;
-    };
-    const f32x4_t a = total(job);
-    const f32x4_t u = p.swiglu ? total(p.job[1]) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int m = 4 * q + e;
-        if (m >= p.positions) break;
-        float v = a[e];
-        if (job.add != nullptr) v += job.add[(size_t)m * job.ldadd + row];
-        if (p.swiglu) {
-            float w = u[e];
-            if (p.job[1].add != nullptr) w += p.job[1].add[(size_t)m * p.job[1].ldadd + row];
-            v = swiglu_value(v, w);
-        }
-        job.y[(size_t)m * job.ldy + row] = v;
-    }
-}
-
-/* Prefill launches whose in-kernel finish would take this many rounds of
- * partial loads or more (ceil(splits / (64 / rows)); 16 quads per round)
- * finish in pf_reduce_kernel instead. Measured on MI355X (µs per launch,
- * Qwen2.5-7B layer shapes, cold graphs of 28, in-kernel / deferred): at 32
- * positions q|k|v (14 splits, 7 rounds) 18.5 / 16.3, o (7 rounds) 17.5 /
- * 14.4, down (15 splits, 8 rounds) 46.3 / 44.5, gate|up (3 splits, 2 rounds)
- * 47.8 / 49.6; at 16 positions q|k|v (4 rounds) 13.3 / 12.3, o 12.4 / 11.1,
- * down (4 rounds) 35.0 / 35.4, gate|up (1 round) 33.1 / 35.8. In the
- * decode-step set (same box) deferring the launches of 4 rounds or more gave
- * 3.513 against 3.655 ms at 32 positions but 2.612 against 2.600 at 16, so
- * the 4-round launches keep the in-kernel finish. */
-#ifndef QMV_PF_DEFER_ROUNDS
-#define QMV_PF_DEFER_ROUNDS 5
-#endif
-
-static hipError_t launch_prefill_kernel(int fmt, const MatvecParams &p, int rows, int grid, hipStream_t s)
-{
-    const dim3 g(grid), b(QMV_PF_WAVES * 64);
-    if (fmt == QMV_FMT_Q4_K && rows == 16) hipLaunchKernelGGL((prefill_kernel<QMV_FMT_Q4_K, 1>), g, b, 0, s, p);
-    else if (fmt == QMV_FMT_Q4_K && rows == 32) hipLaunchKernelGGL((prefill_kernel<QMV_FMT_Q4_K, 2>), g, b, 0, s, p);
-    else if (fmt == QMV_FMT_Q6_K && rows == 16) hipLaunchKernelGGL((prefill_kernel<QMV_FMT_Q6_K, 1>), g, b, 0, s, p);
-    else if (fmt == QMV_FMT_Q6_K && rows == 32) hipLaunchKernelGGL((prefill_kernel<QMV_FMT_Q6_K, 2>), g, b, 0, s, p);
-    else if (fmt == QMV_FMT_Q5_0 && rows == 16) hipLaunchKernelGGL((prefill_kernel<QMV_FMT_Q5_0, 1>), g, b, 0, s, p);
-    else if (fmt == QMV_FMT_Q5_0 && rows == 32) hipLaunchKernelGGL((prefill_kernel<QMV_FMT_Q5_0, 2>), g, b, 0, s, p);
-    else if (fmt == QMV_FMT_Q8_0 && rows == 16) hipLaunchKernelGGL((prefill_kernel<QMV_FMT_Q8_0, 1>), g, b, 0, s, p);
-    else if (fmt == QMV_FMT_Q8_0 && rows == 32) hipLaunchKernelGGL((prefill_kernel<QMV_FMT_Q8_0, 2>), g, b, 0, s, p);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
-}
-
-hipError_t launch_prefill(int fmt, const MatvecParams &params, int rows, int grid, hipStream_t s)
-{
-    if (rows != 16 && rows != 32) return hipErrorInvalidValue;
-    MatvecParams p = params;
-    const int S = p.job[0].splits, per_round = 64 / rows;
-    p.pf_deferred = S > 1 && (S + per_round - 1) / per_round >= QMV_PF_DEFER_ROUNDS ? 1 : 0;
-    const hipError_t e = launch_prefill_kernel(fmt, p, rows, grid, s);
-    if (e != hipSuccess || !p.pf_deferred) return e;
-    long long tiles = 0;
-    for (int j = 0; j < (p.swiglu ? 1 : p.njobs); ++j) tiles += p.job[j].tiles;
-    const long long threads = tiles * (rows / 4) * 64;
-    const dim3 rg((unsigned)(threads / 64)), rb(64); /* one wave per workgroup */
-    if (rows == 16) hipLaunchKernelGGL((pf_reduce_kernel<16>), rg, rb, 0, s, p);
-    else hipLaunchKernelGGL((pf_reduce_kernel<32>), rg, rb, 0, s, p);
     return hipGetLastError();
 }
 

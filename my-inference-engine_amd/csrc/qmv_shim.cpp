@@ -715,7 +715,7 @@ bool use_matrix_cores(int fmt, int batch)
 std::atomic<int> g_q5_prefill{env_int("QMV_Q5_PREFILL", 1)};
 std::atomic<int> g_q8_prefill{env_int("QMV_Q8_PREFILL", 1)};
 
-/* Launches of 9..32 positions: the prefill kernel (all four formats). */
+/* Launches of 9..32 positions, which only chunk_kernel takes. */
 bool use_prefill(int fmt, int batch)
 {
     if (batch <= QMV_VALU_MAX_POSITIONS) return false;
@@ -813,35 +813,6 @@ struct Epilogue {
     float norm_eps = 0.0f;
 };
 
-/* Prefill launches (9..32 positions): a workgroup takes QMV_PF_TILES tiles
- * and a range of K-units (units per split). Measured on MI355X at M = 32
- * (us per launch, cold): rows of fewer than 32 units take one unit per split
- * in at most 20 tile groups (Qwen2.5-7B q|k|v, 18 groups: 19.7 against 20.9
- * at two; o 18.9 against 20.0; Qwen2.5-1.5B q|k|v 14.6 against 15.4, o 13.9
- * against 15.1), five in 100 groups or more (7B gate|up, 148 groups: 48.8
- * against 58.2 at three and 61.5 at four) and two in between (1.5B gate|up,
- * 70 groups: 19.25 against 21.0 at one); long rows take two in at most 8
- * tile groups (1.5B down 1536 x 8960: 23.0 against 24.7 at three) and five
- * beyond (7B down, 14 groups: 52.7 against 57.3 at three). More splits keep
- * more CUs busy until their partials cost more than they spread.
- * units_per_wave, when forced, sets the units per split instead. */
-Plan plan_prefill(long long groups, int units)
-{
-    const int force_u = g_force_u.load();
-    int ups = force_u > 0                ? force_u
-              : units >= 32              ? (groups <= 8 ? 2 : 5)
-              : groups >= 100            ? 5
-              : groups <= 20             ? 1
-                                         : 2;
-    if (ups > units) ups = units;
-    Plan p;
-    p.units_per_wave = ups;
-    p.waves = QMV_PF_TILES;
-    p.units_per_split = ups;
-    p.splits = (units + ups - 1) / ups;
-    return p;
-}
-
 /* One launch over `count` tensors sharing the input, for positions
  * [b0, b0 + batch) of the caller's batch (the caller's pointers are offset
  * here), planned but not enqueued: the parameters, the grid and the workspace
@@ -850,11 +821,15 @@ Plan plan_prefill(long long groups, int units)
  * entry point). */
 struct ChunkPlan {
     qmv::MatvecParams p;
+    qmv::BatchParams bp;                   /* matrix-core launch (batch): its parameters */
+    bool batch = false;                    /* batch_kernel */
+    int bt_nr = 0, bt_r = 0; /* its position rounds and row groups per wave */
+    bool bt_fused = false;
     qmv::RowdotParams rp;                  /* row-major launch (rowdot): its parameters */
     bool rowdot = false;                   /* rowgroup_q4k_kernel */
     int rd_rows = 0, rd_seg = 0, rd_epi = 0; /* rows per segment, lanes per row segment, epilogue */
     bool rd_norm = false;                    /* the fused RMSNorm of the input */
-    bool prefill = false, paired = false;
+    bool paired = false;
     int mt = 1, grid = 0, waves = 0, fmt = 0;
     size_t partials = 0, counters = 0;     /* floats / words of split-K workspace */
     size_t pair_vals = 0, pair_count = 0;  /* offsets of the SwiGLU tile-pair region */
@@ -896,7 +871,7 @@ bool plan_rowdot_q6k(QmvDeviceTensor *const *ts, int count, const float *d_in, i
     cp->rd_seg = 64;
     cp->rd_epi = epi.swiglu ? QMV_ROWDOT_SWIGLU : epi.argmax ? QMV_ROWDOT_ARGMAX : QMV_ROWDOT_STORE;
     cp->rd_norm = false;
-    cp->prefill = cp->paired = false;
+    cp->paired = false;
     cp->mt = 1;
     cp->grid = (int)((total + waves - 1) / waves);
     cp->waves = waves;
@@ -990,7 +965,7 @@ bool plan_rowdot(QmvDeviceTensor *const *ts, int count, const float *d_in, int b
         rp.argmax_result = epi.argmax;
         rp.argmax_tiles = (int)cand;
     }
-    cp->prefill = cp->paired = false;
+    cp->paired = false;
     cp->mt = 1;
     cp->grid = (int)wg;
     cp->waves = waves;
@@ -1001,32 +976,195 @@ bool plan_rowdot(QmvDeviceTensor *const *ts, int count, const float *d_in, int b
     return true;
 }
 
-int plan_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch, float *const *d_out,
+/* Launches of up to 8 positions that chunk_kernel takes (past 8: use_prefill
+ * decides), for K of `units` tiled units and weights of `bytes`, with the
+ * RMSNorm in front (`norm`) or without. Where a workgroup holds all of K it
+ * wins by what the split-K tail and the norm's own launch cost; over longer
+ * rows its reduction is a launch of its own, which small launches of few
+ * positions do not earn back. Both sides over 400 drawn projections of 64 to
+ * 20000 rows and K of 512 to 19000, us in graphs over cold weights, geometric
+ * mean of chunk_kernel / matvec kernels: Q4_K at 3 to 8 positions 0.55-0.83
+ * up to 24 units, 0.72-0.94 beyond (small launches at 7 and 8 positions,
+ * which the matvec kernels also run on the matrix cores, 1.05-1.3); at 2
+ * positions 0.57-0.92 up to 24 units, 1.1-1.3 beyond. Q6_K at 5 to 8: 0.47-
+ * 0.83 throughout; at 3 and 4 0.52-0.84 up to 16 units, 1.02 (with the norm
+ * 0.77) up to 24, 1.06 to 35; at 2 0.57-0.93 up to 8 units, 1.18 at 17-24.
+ * Q8_0 and Q5_0 (units of 128 weights): 0.55-0.89 up to 12 units, 0.95-1.12
+ * at 13-16, with the norm 0.68-0.89 up to 20, 1.05-1.6 beyond 24. */
+bool use_chunks(int fmt, int units, double bytes, int batch, bool norm)
+{
+    if (batch > QMV_VALU_MAX_POSITIONS) return use_prefill(fmt, batch);
+    /* A plan or threshold set by the caller applies to the matvec kernels. */
+    if (g_target_waves.load() > 0 || g_force_u.load() > 0 || g_force_w.load() > 0 || g_mfma_min_batch.load() > 0)
+        return false;
+    if (batch < 2) return false;
+    if (fmt == QMV_FMT_Q8_0 || fmt == QMV_FMT_Q5_0) return units <= (norm ? 20 : batch == 2 ? 8 : 12);
+    if (batch == 2) return units <= (fmt == QMV_FMT_Q4_K ? 24 : 16);
+    if (fmt == QMV_FMT_Q4_K) return batch <= 6 || units <= 24 || bytes >= 12e6;
+    return batch >= 5 || units <= 24 || bytes >= 30e6;
+}
+
+/* How a chunk_kernel launch is cut up. */
+struct BatchShape {
+    int nr, r;  /* rounds of 4 positions; row groups per wave */
+    bool fused; /* all of K in one workgroup */
+    int waves, segs, chunk_segs, wg_groups;
+};
+
+constexpr int kLdsBytes = 160 * 1024, kCus = 256;
+
+/* The cut with the least estimated time, over segment lengths and segments
+ * per workgroup: one workgroup per CU; staging rounds and items per wave times
+ * their instructions (4 cycles each at 2.4 GHz, times the waves that share a
+ * SIMD, at least 0.45 us a unit for its loads); the weights at 5 TB/s; and
+ * for launches that are not fused 3 us and the partial sums' traffic. At the
+ * measured shapes it picks the fastest cut or one within 5% (Qwen2.5-7B o at
+ * 4 positions: two units a segment 7.1 us, one 7.7, four 7.7; down at 8, two
+ * segments of five a workgroup 23.2 us, of four 23.8, three of five 24.3).
+ * Waves: 16 (the registers of one row group of Q4_K, Q8_0, Q5_0 allow them),
+ * 12 for Q6_K and for chunks (down at 4: 23.8 us at 12 against 31.3 at 16 with
+ * spills); past 8 positions 12, and 8 where a wave takes two row groups to
+ * read the staged activations half as often (gate|up at 32 positions: 41.5
+ * us against 48.9 with one) or for Q6_K (down at 32: 36 against 58 at 12).
+ * The segments are the same with `swiglu` as without, and past 8 positions
+ * they do not depend on the positions. `alone`: only a cut without workspace
+ * (waves = 0 if there is none). */
+BatchShape batch_shape(int fmt, int units, long long groups, int batch, bool swiglu, bool alone)
+{
+    const bool q32 = fmt == QMV_FMT_Q8_0 || fmt == QMV_FMT_Q5_0, q6 = fmt == QMV_FMT_Q6_K;
+    const bool wide = batch > QMV_VALU_MAX_POSITIONS;
+    BatchShape best = {};
+    best.nr = batch <= 4 ? 1 : batch <= 8 ? 2 : batch <= 16 ? 4 : 8;
+    best.r = wide && groups > 512 && !q6 ? 2 : 1;
+    const int nr = best.nr, r = best.r, limbs = nr <= 2 ? 1 : nr / 2;
+    const int stage = (int)qmv::batch_stage_bytes(fmt, nr);
+    const auto round_to = [](long long g, int m) { return (g + m - 1) / m * m; };
+    const double stage_us = (q32 ? 100 : 185) * 4 / 2400.0;
+    const int instr = (fmt == QMV_FMT_Q4_K ? 130 : q6 ? 190 : fmt == QMV_FMT_Q8_0 ? 75 : 105) +
+                      (limbs - 1) * (q32 ? 20 : 15);
+    const double unit_us = r * (instr * 4 + 0.6 * limbs * 16 * (q6 ? 16 : q32 ? 4 : 9)) / 2400.0;
+    const int unit_bytes = fmt == QMV_FMT_Q4_K ? 144 : q6 ? 210 : fmt == QMV_FMT_Q8_0 ? 136 : 88;
+    const double weights_us = (double)groups * 16 * units * unit_bytes / 5.0e6;
+    const int kunits = q32 ? (units + 1) / 2 : units; /* of 256 weights */
+    const int fixed = !wide ? 0
+                            : (kunits <= 40 && (groups <= 512 || (q6 && kunits <= 16 && groups <= 2048)) ? 2 : 4) *
+                                  (q32 && units > 16 ? 2 : 1);
+    double best_us = 1e30;
+    static const int kLengths[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16};
+    for (int length : kLengths) {
+        const int segs = (units + (fixed ? fixed : length) - 1) / (fixed ? fixed : length);
+        const int longest = (units + segs - 1) / segs;
+        for (int cs = 0; cs <= (alone ? 0 : wide ? 1 : 4) && cs <= segs; ++cs) { /* 0: fused */
+            BatchShape c = best;
+            c.fused = cs == 0;
+            c.segs = segs;
+            c.chunk_segs = c.fused ? segs : cs;
+            const int chunks = (segs + c.chunk_segs - 1) / c.chunk_segs;
+            const long long per = std::max(1, kCus / chunks);
+            const long long g1 = round_to((groups + per - 1) / per, r), g2 = round_to(g1, 2);
+            const int staged = c.fused ? units : c.chunk_segs * longest;
+            const long long lds = (long long)staged * stage + (c.fused ? (segs * g2 * 64 + 4) * 4 * nr : 0);
+            if (lds > kLdsBytes) continue;
+            c.wg_groups = (int)(swiglu ? g2 : g1);
+            const long long items = g1 / r * c.chunk_segs;
+            c.waves = r == 2 || (q6 && wide) ? 8 : wide || q6 || !c.fused ? 12 : 16;
+            c.waves = (int)std::min<long long>(c.waves, std::max<long long>(items, staged * nr));
+            const long long busy = std::min<long long>(c.waves, items);
+            const double per_unit = std::max(unit_us * ((busy + 3) / 4), 0.45);
+            double us = stage_us * ((c.waves + 3) / 4) * ((staged * nr + c.waves - 1) / c.waves);
+            us += std::max((items + busy - 1) / busy * longest * per_unit, weights_us);
+            us += c.fused ? 0.6 + 0.06 * segs : 3.0 + 2.0 * segs * batch * groups * 64 / 4.0e6;
+            if (us < best_us) {
+                best_us = us;
+                best = c;
+            }
+        }
+        if (fixed) break;
+    }
+    return best;
+}
+
+/* A chunk_kernel launch, if it is one that kernel takes. */
+bool plan_batch(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch, float *const *d_out,
+                const Epilogue &epi, bool alone, ChunkPlan *cp)
+{
+    const QmvDeviceTensor *t0 = ts[0];
+    if (epi.argmax || (epi.swiglu && (count != 2 || ts[1]->rows != t0->rows))) return false;
+    const int fmt = t0->geo.format, units = t0->units;
+    long long groups = 0;
+    for (int i = 0; i < count; ++i) groups += (ts[i]->rows + 15) / 16;
+    if (groups > INT_MAX / 16) return false;
+    if (!use_chunks(fmt, units, (double)groups * 16 * units * t0->geo.unit_bytes, batch, epi.norm_w != nullptr))
+        return false;
+    const BatchShape b = batch_shape(fmt, units, groups, batch, epi.swiglu, alone);
+    if (b.waves == 0) return false;
+    const size_t partials = b.fused ? 0 : (size_t)b.segs * batch * groups * 16 + (epi.norm_w ? (size_t)units * 8 * b.nr : 0);
+    if (partials > (size_t)INT_MAX) return false;
+    qmv::BatchParams &p = cp->bp;
+    memset(&p, 0, sizeof p);
+    p.njobs = count;
+    p.x = d_in + (size_t)b0 * t0->cols;
+    p.cols = t0->cols;
+    p.units = units;
+    p.positions = batch;
+    p.swiglu = epi.swiglu;
+    p.norm_w = epi.norm_w;
+    p.norm_eps = epi.norm_eps;
+    p.groups = (int)groups;
+    p.wg_groups = b.wg_groups;
+    p.segs = b.segs;
+    p.seg_units = units / b.segs;
+    p.seg_more = units % b.segs;
+    p.chunk_segs = b.chunk_segs;
+    p.chunk_wgs = (int)((groups + b.wg_groups - 1) / b.wg_groups);
+    for (int i = count; i < QMV_MAX_JOBS; ++i) p.job[i].group_begin = INT_MAX; /* unused: past every group */
+    int begin = 0;
+    for (int i = 0; i < count; ++i) {
+        qmv::BatchJob &j = p.job[i];
+        j.w = ts[i]->data;
+        j.y = d_out[i] + (size_t)b0 * ts[i]->rows;
+        j.rows = ts[i]->rows;
+        j.group_begin = begin;
+        begin += (ts[i]->rows + 15) / 16;
+        if (epi.add && epi.add[i]) {
+            j.add = epi.add[i] + (size_t)b0 * epi.ldadd[i];
+            j.ldadd = epi.ldadd[i];
+        }
+    }
+    memset(&cp->p, 0, sizeof cp->p);
+    cp->batch = true;
+    cp->rowdot = cp->paired = false;
+    cp->bt_nr = b.nr;
+    cp->bt_r = b.r;
+    cp->bt_fused = b.fused;
+    cp->waves = b.waves;
+    cp->fmt = fmt;
+    cp->partials = partials;
+    cp->counters = 0;
+    cp->pair_vals = cp->pair_count = 0;
+    cp->argmax_tiles = 0;
+    return true;
+}
+
+/* A launch on the matvec kernels (up to 8 positions). */
+int plan_tiled(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch, float *const *d_out,
                const Epilogue &epi, ChunkPlan *cp)
 {
     const QmvDeviceTensor *t0 = ts[0];
-    cp->rowdot = false;
-    if (batch == 1 && plan_rowdot(ts, count, d_in, b0, d_out, epi, cp)) return 1;
+    cp->rowdot = cp->batch = false;
     if (epi.norm_w) {
         set_error("internal: a fused RMSNorm reached the tiled planner");
         return 0;
     }
-    const bool mfma = use_matrix_cores(t0->geo.format, batch);
-    /* Up to 8 positions: the matvec kernels for exactly `batch` positions.
-     * More: the prefill kernel, 16 or 32 position rows with the batch in the
-     * first. */
-    const bool prefill = batch > QMV_VALU_MAX_POSITIONS;
-    if (prefill && !use_prefill(t0->geo.format, batch)) {
+    if (batch > QMV_VALU_MAX_POSITIONS) {
         set_error("more than 8 positions per launch need the matrix-core path");
         return 0;
     }
-    const int mt = !prefill ? batch : batch <= 16 ? 16 : QMV_MFMA_MAX_POSITIONS;
-    long long total_tiles = 0, total_groups = 0;
-    for (int i = 0; i < count; ++i) {
-        total_tiles += ts[i]->tiles;
-        total_groups += (ts[i]->tiles + QMV_PF_TILES - 1) / QMV_PF_TILES;
-    }
-    const int parts = prefill ? 1 : mfma ? mfma_parts(t0->units, total_tiles) : batch >= 2 ? valu_parts(t0->units) : 1;
+    const bool mfma = use_matrix_cores(t0->geo.format, batch);
+    const int mt = batch;
+    long long total_tiles = 0;
+    for (int i = 0; i < count; ++i) total_tiles += ts[i]->tiles;
+    const int parts = mfma ? mfma_parts(t0->units, total_tiles) : batch >= 2 ? valu_parts(t0->units) : 1;
     /* Single-position launches of many units (the vocabulary projection:
      * 33236) run several rounds of resident waves; five waves per workgroup
      * (three splits of 14 units instead of four) measured 80.9 us against
@@ -1064,9 +1202,8 @@ int plan_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0,
                             : mfma                                          ? mfma_waves
                             : batch == 1 && total_tiles * t0->units > 2048  ? 2
                                                                             : 4;
-    const Plan plan = prefill ? plan_prefill(total_groups, t0->units)
-                              : plan_for(total_tiles, t0->units * parts, batch == 1 ? 6 : long_batch_waves, short_waves,
-                                         mfma || parts > 1 ? 1 : 8);
+    const Plan plan = plan_for(total_tiles, t0->units * parts, batch == 1 ? 6 : long_batch_waves, short_waves,
+                               mfma || parts > 1 ? 1 : 8);
 
     qmv::MatvecParams &p = cp->p;
     memset(&p, 0, sizeof p);
@@ -1077,7 +1214,7 @@ int plan_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0,
     p.units = t0->units;
     p.units_per_wave = plan.units_per_wave;
     p.parts = parts;
-    if ((mfma || parts > 1) && !prefill && plan.units_per_wave != 1) {
+    if ((mfma || parts > 1) && plan.units_per_wave != 1) {
         set_error("launch planned with more than one work item per wave");
         return 0;
     }
@@ -1085,7 +1222,7 @@ int plan_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0,
     /* Fused SwiGLU at M = 1 with one unit per wave: one workgroup per
      * (tile, split) of both projections (finish_paired), when the two halves
      * fit a workgroup. */
-    const bool paired = epi.swiglu && count == 2 && batch == 1 && !prefill && !mfma &&
+    const bool paired = epi.swiglu && count == 2 && batch == 1 && !mfma &&
                         plan.units_per_wave == 1 && 2 * plan.waves <= QMV_MAX_WAVES &&
                         ts[0]->rows == ts[1]->rows && g_paired_swiglu.load() != 0;
     size_t partials = 0, counters = 0;
@@ -1120,7 +1257,7 @@ int plan_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0,
             partials += (size_t)ts[i]->tiles * plan.splits * mt * 64;
             counters += (size_t)ts[i]->tiles * QMV_COUNTER_STRIDE;
         }
-        wg += (long long)(prefill ? (ts[i]->tiles + QMV_PF_TILES - 1) / QMV_PF_TILES : ts[i]->tiles) * plan.splits;
+        wg += (long long)ts[i]->tiles * plan.splits;
     }
     if (paired) p.pair_waves = plan.waves;
     /* Fused SwiGLU otherwise: both projections' final tiles, then one count
@@ -1151,7 +1288,6 @@ int plan_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0,
         p.argmax_tiles = t0->tiles;
         cp->argmax_tiles = (size_t)t0->tiles;
     }
-    cp->prefill = prefill;
     cp->paired = paired;
     cp->mt = mt;
     cp->grid = (int)wg;
@@ -1162,12 +1298,26 @@ int plan_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0,
     return 1;
 }
 
+/* alone: without workspace where chunk_kernel takes the launch. */
+int plan_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch, float *const *d_out,
+               const Epilogue &epi, ChunkPlan *cp, bool alone = false)
+{
+    cp->rowdot = cp->batch = false;
+    if (batch == 1 && plan_rowdot(ts, count, d_in, b0, d_out, epi, cp)) return 1;
+    if (plan_batch(ts, count, d_in, b0, batch, d_out, epi, alone, cp)) return 1;
+    return plan_tiled(ts, count, d_in, b0, batch, d_out, epi, cp);
+}
+
 /* Point the plan at its split-K workspace: partials[cp.partials] floats and
  * counters[cp.counters] words (zero between launches). */
 void bind_workspace(ChunkPlan &cp, float *partials, unsigned *counters)
 {
     cp.p.partials = partials;
     cp.p.counters = counters;
+    if (cp.batch && !cp.bt_fused) {
+        cp.bp.partials = partials;
+        cp.bp.ssq = (double *)(partials + (size_t)cp.bp.segs * cp.bp.positions * cp.bp.groups * 16);
+    }
     if (cp.p.swiglu) {
         cp.p.pair_vals = partials + cp.pair_vals;
         cp.p.pair_count = counters + cp.pair_count;
@@ -1176,25 +1326,47 @@ void bind_workspace(ChunkPlan &cp, float *partials, unsigned *counters)
 
 int enqueue_chunk(const ChunkPlan &cp, hipStream_t stream)
 {
-    if (cp.rowdot && cp.fmt == QMV_FMT_Q6_K)
+    if (cp.batch)
+        HIP_TRY(qmv::launch_batch(cp.fmt, cp.bp, cp.bt_nr, cp.bt_r, cp.bt_fused, cp.waves, stream));
+    else if (cp.rowdot && cp.fmt == QMV_FMT_Q6_K)
         HIP_TRY(qmv::launch_rowloop_q6k(cp.rp, cp.rd_epi, cp.grid, cp.waves, stream));
     else if (cp.rowdot)
         HIP_TRY(qmv::launch_rowgroup(cp.rp, cp.rd_rows, cp.rd_seg, cp.rd_epi, cp.grid, cp.waves, stream, cp.rd_norm));
-    else if (cp.prefill)
-        HIP_TRY(qmv::launch_prefill(cp.fmt, cp.p, cp.mt, cp.grid, stream));
     else
         HIP_TRY(qmv::launch_matvec(cp.fmt, cp.p, cp.mt, cp.grid, cp.waves, stream));
     return 1;
 }
 
 /* Plan a launch and enqueue it on the stream's own workspace (grown here if
- * needed, outside graph capture only). */
+ * needed, outside graph capture only). A chunk_kernel launch that would have
+ * to grow it during a capture is made as launches of up to 8 positions that
+ * need no workspace, where there are such (short rows, which never needed
+ * any). */
 int launch_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch,
                  float *const *d_out, hipStream_t stream, Workspace &ws, const Epilogue &epi)
 {
     ChunkPlan cp;
     if (!plan_chunk(ts, count, d_in, b0, batch, d_out, epi, &cp)) return 0;
     std::lock_guard<std::mutex> lock(ws.mu);
+    if (cp.batch && cp.partials > ws.partial_cap) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
+            std::vector<ChunkPlan> parts;
+            for (int b = 0; b < batch; b += QMV_VALU_MAX_POSITIONS) {
+                ChunkPlan part;
+                part.batch = false;
+                if (!plan_batch(ts, count, d_in, b0 + b, std::min(QMV_VALU_MAX_POSITIONS, batch - b), d_out, epi, true,
+                                &part))
+                    break;
+                parts.push_back(part);
+            }
+            if ((int)parts.size() * QMV_VALU_MAX_POSITIONS >= batch) {
+                for (const ChunkPlan &part : parts)
+                    if (!enqueue_chunk(part, stream)) return 0;
+                return 1;
+            }
+        }
+    }
     if (!workspace_reserve(ws, stream, cp.partials, cp.counters)) return 0;
     bind_workspace(cp, ws.partials, ws.counters);
     if (cp.argmax_tiles) {
@@ -1206,7 +1378,7 @@ int launch_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b
 }
 
 /* Positions per launch for the remaining `batch` positions of a call: up to
- * 32 where the prefill kernel takes them, else 8. */
+ * 32 where chunk_kernel takes them, else 8. */
 int chunk_positions(int fmt, int batch)
 {
     const int wide = batch < QMV_MFMA_MAX_POSITIONS ? batch : QMV_MFMA_MAX_POSITIONS;
@@ -1215,7 +1387,7 @@ int chunk_positions(int fmt, int batch)
 
 /* Positions of the launch that starts at position b0 of a `batch`-position
  * call. The chunk size is chosen again for every launch from the positions
- * left, so a tail that the prefill kernel does not take (for instance below
+ * left, so a tail that chunk_kernel does not take (for instance below
  * a raised matrix-core threshold) runs in launches of at most 8. */
 int next_chunk(int fmt, int batch, int b0)
 {
@@ -1605,6 +1777,38 @@ int scratch_address(int device, void **out)
     return 1;
 }
 
+/* The scratch that decides whether a launch is accepted (what the entry
+ * point takes does not depend on the kernel that runs it): up to 8 positions
+ * that of the matvec kernels; past 8, the partial sums of 16 or 32 position
+ * rows over K in splits of 1, 2 or 5 units by the tensors' groups of four
+ * tiles. */
+int scratch_rule(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch, float *const *d_out,
+                 size_t *partials, size_t *counters)
+{
+    ChunkPlan cp;
+    if (batch <= QMV_VALU_MAX_POSITIONS) {
+        cp.rowdot = cp.batch = false;
+        if (!(batch == 1 && plan_rowdot(ts, count, d_in, b0, d_out, Epilogue(), &cp)) &&
+            !plan_tiled(ts, count, d_in, b0, batch, d_out, Epilogue(), &cp))
+            return 0;
+        *partials = cp.partials;
+        *counters = cp.counters;
+        return 1;
+    }
+    const int units = ts[0]->units;
+    long long tiles = 0, fours = 0;
+    for (int i = 0; i < count; ++i) {
+        tiles += ts[i]->tiles;
+        fours += (ts[i]->tiles + 3) / 4;
+    }
+    const int split = units >= 32 ? (fours <= 8 ? 2 : 5) : fours >= 100 ? 5 : fours <= 20 ? 1 : 2;
+    if (units > split) {
+        *partials = (size_t)tiles * ((units + split - 1) / split) * (batch <= 16 ? 16 : 32) * 64 + QMV_PARTIAL_PAD;
+        *counters = (size_t)tiles * QMV_COUNTER_STRIDE;
+    }
+    return 1;
+}
+
 } // namespace
 
 QMV_API int qmv_device_matvec_group_noalloc_f32(const qmv_device_tensor *tensors, int count, const float *d_inputs,
@@ -1623,30 +1827,44 @@ QMV_API int qmv_device_matvec_group_noalloc_f32(const qmv_device_tensor *tensors
     const int fmt = ts[0]->geo.format;
     /* Every launch is planned and checked before the first is enqueued, so a
      * call that does not fit launches nothing. */
+    std::vector<ChunkPlan> plans;
     for (int b0 = 0; b0 < batch_count;) {
         const int nb = next_chunk(fmt, batch_count, b0);
-        ChunkPlan cp;
-        if (!plan_chunk(ts, count, d_inputs, b0, nb, d_outputs, Epilogue(), &cp)) return 0;
-        if (cp.partials > partial_cap || cp.counters > counter_cap) {
+        size_t need_partials = 0, need_counters = 0;
+        if (!scratch_rule(ts, count, d_inputs, b0, nb, d_outputs, &need_partials, &need_counters)) return 0;
+        bool fits = need_partials <= partial_cap && need_counters <= counter_cap;
+        /* A launch past 8 positions whose partial sums do not fit is made as
+         * several of at least 9, which have the same bits. */
+        int pieces = 1;
+        for (; fits; ++pieces) {
+            ChunkPlan cp;
+            if (!plan_chunk(ts, count, d_inputs, b0, (nb + pieces - 1) / pieces, d_outputs, Epilogue(), &cp)) return 0;
+            need_partials = cp.partials;
+            if (cp.partials <= partial_cap && cp.counters <= counter_cap) break;
+            fits = nb / (pieces + 1) > QMV_VALU_MAX_POSITIONS;
+        }
+        if (!fits) {
             set_error("launch needs %zu partial floats and %zu counters; the no-allocation scratch holds %zu and "
                       "%zu (use qmv_device_matvec_group_f32)",
-                      cp.partials, cp.counters, partial_cap, counter_cap);
+                      need_partials, need_counters, partial_cap, counter_cap);
             return 0;
+        }
+        for (int i = 0, b = b0; i < pieces; ++i) {
+            const int n = nb / pieces + (i < nb % pieces ? 1 : 0);
+            plans.emplace_back();
+            if (!plan_chunk(ts, count, d_inputs, b, n, d_outputs, Epilogue(), &plans.back())) return 0;
+            b += n;
         }
         b0 += nb;
     }
     hipStream_t s = (hipStream_t)stream;
-    for (int b0 = 0; b0 < batch_count;) {
-        const int nb = next_chunk(fmt, batch_count, b0);
-        ChunkPlan cp;
-        if (!plan_chunk(ts, count, d_inputs, b0, nb, d_outputs, Epilogue(), &cp)) return 0;
+    for (ChunkPlan &cp : plans) {
         bind_workspace(cp, partials, counters);
         /* The counters must be zero when the launch starts. Completed
          * launches leave them zero; the fill (a kernel, not a memset node, so
          * the call can be captured) also covers an interrupted earlier one. */
         HIP_TRY(qmv::launch_fill_u32(counters, cp.counters, 0u, s));
         if (!enqueue_chunk(cp, s)) return 0;
-        b0 += nb;
     }
     return 1;
 }
@@ -1739,6 +1957,17 @@ static int norm_then_group(QmvDeviceTensor *const *ts, int count, const float *d
         if (plan_rowdot(ts, count, d_in, 0, d_out, epi, &cp)) return enqueue_chunk(cp, s);
         epi.norm_w = nullptr;
     }
+    /* Every workgroup reads the norm weights, so an output over them keeps
+     * the two launches. */
+    bool apart = true;
+    for (int i = 0; i < count; ++i)
+        apart = apart && !overlap(d_out[i], (size_t)batch * ts[i]->rows * 4, d_w, (size_t)ts[0]->cols * 4);
+    epi.norm_w = d_w;
+    epi.norm_eps = eps;
+    ChunkPlan cp;
+    if (batch > 1 && apart && plan_batch(ts, count, d_in, 0, batch, d_out, epi, false, &cp))
+        return launch_chunk(ts, count, d_in, 0, batch, d_out, s, ws, epi);
+    epi.norm_w = nullptr;
     HIP_TRY(qmv::launch_rms_norm(d_in, d_w, ts[0]->cols, batch, eps, d_normed, s));
     return launch_group(ts, count, d_normed, batch, d_out, s, ws, epi);
 }

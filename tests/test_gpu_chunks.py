@@ -1,0 +1,188 @@
+"""Matrix-core launches of 2 to 32 positions (chunk_kernel): the reference's
+quantized_tensor_matmul_f32 (src/quantized_matvec.cpp:164-224) and the norm,
+bias and SwiGLU around it, at the edges of the kernel's cuts: row groups of
+16, rounds of 4 positions, fragments of 8, 16 and 32, K in one workgroup or
+in chunks, partial 128-weight units.
+
+Bar: every row of every position within 1e-5 * sum |w x| of the oracle, the
+bar of every product here. The kernel's activations are two f16 limbs under a
+power of two per position and unit, exact to 2^-24 of each value within 2^28
+of the unit's largest, so a value 2^26 below its unit's largest must count
+as fully as on the VALU kernels."""
+import numpy as np
+import pytest
+
+import _blocks as B
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5
+
+
+@pytest.fixture(scope="module")
+def hip(qmv):
+    import importlib
+    return importlib.import_module("my-inference-engine_amd.hip_runtime")
+
+
+def _bits(a):
+    return np.ascontiguousarray(a, dtype=np.float32).view(np.uint32)
+
+
+def _tensor(qmv, t, rows, cols, seed):
+    raw = qmv.synth_tensor(t, rows, cols, seed=seed)
+    return raw, qmv.DeviceTensor(qmv.make_view(raw, t, rows, cols))
+
+
+def _check(oracle, raw, t, rows, cols, x, y, what, scale=1.0):
+    for b in range(x.shape[0]):
+        ref = oracle.matvec(raw, t, rows, cols, x[b])
+        _, absdot = oracle.row_stats(raw, t, rows, cols, x[b])
+        assert (np.abs(y[b].astype(np.float64) - ref) <= scale * TOL * absdot).all(), f"{what}: position {b}"
+
+
+# K: one unit, an odd number, the last that one workgroup takes, chunks; the
+# 32-weight formats also with a partial last unit.
+KS = {B.Q4_K: [256, 1280, 4352, 8960], B.Q6_K: [256, 1280, 4096, 10240],
+      B.Q8_0: [32, 480, 1536, 4864], B.Q5_0: [96, 672, 2080, 5120]}
+
+
+@pytest.mark.parametrize("t", B.ALL_TYPES)
+@pytest.mark.parametrize("rows,batch", [(1, 2), (15, 4), (16, 5), (17, 8), (65, 9), (130, 16), (47, 17), (1000, 32)])
+def test_chunk_edges(qmv, oracle, gpu, hip, t, rows, batch):
+    with hip.Stream() as s:
+        for cols in KS[t]:
+            raw, dt = _tensor(qmv, t, rows, cols, rows + batch)
+            x = qmv.synth_normal(batch * cols, seed=batch).reshape(batch, cols)
+            dx, dy = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(4 * (batch * rows + 64))
+            dy.fill(0x7F)  # nothing past the outputs is written
+            print(f"chunks: {B.NAMES[t]} {rows}x{cols} M={batch}", flush=True)
+            dt.matvec(dx.ptr, batch, dy.ptr, s.handle)
+            s.synchronize()
+            y = dy.to_array(np.float32, (batch * rows + 64,))
+            assert np.all(_bits(y[batch * rows:]) == 0x7F7F7F7F)
+            _check(oracle, raw, t, rows, cols, x, y[:batch * rows].reshape(batch, rows), f"K={cols}")
+            dt.close()
+
+
+@pytest.mark.parametrize("t", B.ALL_TYPES)
+@pytest.mark.parametrize("batch", [2, 6, 20])
+def test_chunk_small_beside_large(qmv, oracle, gpu, hip, t, batch):
+    """The first sub-block's scale is 0, so its products are 0, and its
+    activations are 2^26 times the others of the same unit: the others keep
+    full precision."""
+    rows, cols = 40, 1024
+    raw = qmv.synth_tensor(t, rows, cols, seed=9).reshape(rows, -1).copy()
+    w = raw.reshape(rows, cols // B.BLOCK_ELEMENTS[t], -1)
+    if t == B.Q4_K:  # 6-bit scale and minimum of sub-block 0
+        w[:, 0, 4] &= 0xC0
+        w[:, 0, 8] &= 0xC0
+    elif t == B.Q6_K:
+        w[:, 0, 192] = 0
+    else:
+        w[:, 0, :2] = 0
+    raw = np.ascontiguousarray(raw.reshape(-1))
+    dt = qmv.DeviceTensor(qmv.make_view(raw, t, rows, cols))
+    x = qmv.synth_normal(batch * cols, seed=10).reshape(batch, cols)
+    x[:, :16 if t == B.Q6_K else 32] *= np.float32(2.0 ** 26)
+    with hip.Stream() as s:
+        dx, dy = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(4 * batch * rows)
+        print(f"chunks: {B.NAMES[t]} outliers M={batch}", flush=True)
+        dt.matvec(dx.ptr, batch, dy.ptr, s.handle)
+        s.synchronize()
+        _check(oracle, raw, t, rows, cols, x, dy.to_array(np.float32, (batch, rows)), "outliers")
+    dt.close()
+
+
+@pytest.mark.parametrize("t", B.ALL_TYPES)
+@pytest.mark.parametrize("batch,cols", [(3, 1024), (8, 1024), (12, 1024), (32, 1024), (13, 5120), (6, 8960)])
+def test_chunk_norm_group(qmv, oracle, gpu, hip, t, batch, cols):
+    """RMSNorm, three tensors of unequal rows and biases in one call, then the
+    gate and up pair, against the oracle's norm and products; a NaN in one
+    position stays there, and an infinity gives no finite row."""
+    rows = [100, 16, 33]
+    raws, dts = zip(*[_tensor(qmv, t, r, cols, 40 + i) for i, r in enumerate(rows)])
+    rng = np.random.default_rng(batch)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    nw = (1 + 0.1 * rng.standard_normal(cols)).astype(np.float32)
+    bias = [rng.standard_normal(r).astype(np.float32) for r in rows]
+    normed = np.stack([oracle.rms_norm(x[b], nw, 1e-6)[1] for b in range(batch)])
+    with hip.Stream() as s:
+        dx, dw, dn = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer.from_array(nw), hip.DeviceBuffer(4 * batch * cols)
+        db = [hip.DeviceBuffer.from_array(b) for b in bias]
+        ys = [hip.DeviceBuffer(4 * batch * r) for r in rows]
+
+        def call():
+            qmv.device_rms_norm_matvec_add_group(list(dts), dx.ptr, dw.ptr, 1e-6, batch, [b.ptr for b in db], [0, 0, 0],
+                                                 [y.ptr for y in ys], dn.ptr, s.handle)
+            s.synchronize()
+            return [y.to_array(np.float32, (batch, r)) for y, r in zip(ys, rows)]
+
+        print(f"chunks: {B.NAMES[t]} norm group K={cols} M={batch}", flush=True)
+        first = call()
+        for raw, r, y, b in zip(raws, rows, first, bias):
+            _check(oracle, raw, t, r, cols, normed, y - b[None, :], f"rows {r}", scale=2.0)
+        for bad in (np.nan, np.inf):
+            x2 = x.copy()
+            x2[1, cols // 3] = bad
+            dx = hip.DeviceBuffer.from_array(x2)
+            again = call()
+            for a, f in zip(again, first):
+                keep = [p for p in range(batch) if p != 1]
+                assert np.array_equal(_bits(a[keep]), _bits(f[keep]))
+                if np.isnan(bad):
+                    assert np.isnan(a[1]).all()
+        dx = hip.DeviceBuffer.from_array(x)
+        raw_u, du = _tensor(qmv, t, rows[0], cols, 77)
+        gate, up, act = (hip.DeviceBuffer(4 * batch * rows[0]) for _ in range(3))
+        dxn = hip.DeviceBuffer.from_array(normed)
+        qmv.device_matvec_group([dts[0], du], dxn.ptr, batch, [gate.ptr, up.ptr], s.handle)
+        qmv.device_rms_norm_matvec_swiglu(dts[0], du, dx.ptr, dw.ptr, 1e-6, batch, act.ptr, dn.ptr, s.handle)
+        s.synchronize()
+        g, u, a = (v.to_array(np.float32, (batch, rows[0])).astype(np.float64) for v in (gate, up, act))
+        absg, absu = (np.stack([oracle.row_stats(r, t, rows[0], cols, normed[b])[1] for b in range(batch)])
+                      for r in (raws[0], raw_u))
+        # |d silu| <= 1.1 |d g|; both projections within 2e-5 of their sums
+        bound = 2 * TOL * (1.1 * absg * np.abs(u) + absu * np.abs(g / (1 + np.exp(-g))) + 2 * TOL * absg * absu) + 1e-6
+        assert (np.abs(a - u * g / (1 + np.exp(-g))) <= bound).all()
+        du.close()
+    for d in dts:
+        d.close()
+
+
+@pytest.mark.parametrize("t,rows,cols,batch", [(B.Q4_K, 64, 256, 32), (B.Q8_0, 900, 96, 20), (B.Q6_K, 5200, 512, 24)])
+def test_chunk_capture_without_a_first_call(qmv, oracle, gpu, hip, t, rows, cols, batch):
+    """Launches over one or two K-units need no workspace, so a stream that
+    never ran one can capture them; replays match the eager launch's bar."""
+    raw, dt = _tensor(qmv, t, rows, cols, 5)
+    x = qmv.synth_normal(batch * cols, seed=6).reshape(batch, cols)
+    dx, dy = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(4 * batch * rows)
+    with hip.Stream() as s, hip.Graph(s) as g:
+        print(f"chunks: capture {B.NAMES[t]} {rows}x{cols} M={batch}", flush=True)
+        g.begin()
+        dt.matvec(dx.ptr, batch, dy.ptr, s.handle)
+        g.end()
+        for _ in range(3):
+            dy.fill(0)
+            g.replay()
+            s.synchronize()
+            _check(oracle, raw, t, rows, cols, x, dy.to_array(np.float32, (batch, rows)), "replay")
+    dt.close()
+
+
+def test_chunk_output_over_norm_weights(qmv, oracle, gpu, hip):
+    """An output that lies over the norm weights is written after they are
+    read (the norm then runs as a launch of its own)."""
+    t, rows, cols, batch = B.Q4_K, 64, 512, 4
+    raw, dt = _tensor(qmv, t, rows, cols, 8)
+    x = qmv.synth_normal(batch * cols, seed=6).reshape(batch, cols)
+    nw = np.abs(qmv.synth_normal(cols, seed=7)).astype(np.float32) + 0.5
+    normed = np.stack([oracle.rms_norm(x[b], nw, 1e-6)[1] for b in range(batch)])
+    with hip.Stream() as s:
+        dx, dw, dn = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer.from_array(nw), hip.DeviceBuffer(4 * batch * cols)
+        print("chunks: output over norm weights", flush=True)
+        qmv.device_rms_norm_matvec_add_group([dt], dx.ptr, dw.ptr, 1e-6, batch, [0], [0], [dw.ptr], dn.ptr, s.handle)
+        s.synchronize()
+        _check(oracle, raw, t, rows, cols, normed, dw.to_array(np.float32, (cols,))[:batch * rows].reshape(batch, rows),
+               "over the weights", scale=2.0)
+    dt.close()
