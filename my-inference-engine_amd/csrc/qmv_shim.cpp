@@ -981,27 +981,31 @@ bool plan_rowdot(QmvDeviceTensor *const *ts, int count, const float *d_in, int b
  * RMSNorm in front (`norm`) or without. Where a workgroup holds all of K it
  * wins by what the split-K tail and the norm's own launch cost; over longer
  * rows its reduction is a launch of its own, which small launches of few
- * positions do not earn back. Both sides over 400 drawn projections of 64 to
+ * positions do not earn back. Both sides over 650 drawn projections of 64 to
  * 20000 rows and K of 512 to 19000, us in graphs over cold weights, geometric
- * mean of chunk_kernel / matvec kernels: Q4_K at 3 to 8 positions 0.55-0.83
- * up to 24 units, 0.72-0.94 beyond (small launches at 7 and 8 positions,
- * which the matvec kernels also run on the matrix cores, 1.05-1.3); at 2
- * positions 0.57-0.92 up to 24 units, 1.1-1.3 beyond. Q6_K at 5 to 8: 0.47-
- * 0.83 throughout; at 3 and 4 0.52-0.84 up to 16 units, 1.02 (with the norm
- * 0.77) up to 24, 1.06 to 35; at 2 0.57-0.93 up to 8 units, 1.18 at 17-24.
- * Q8_0 and Q5_0 (units of 128 weights): 0.55-0.89 up to 12 units, 0.95-1.12
- * at 13-16, with the norm 0.68-0.89 up to 20, 1.05-1.6 beyond 24. */
+ * mean of chunk_kernel / matvec kernels: Q4_K at 3 to 8 positions 0.51-0.83
+ * up to 24 units, 0.72-0.94 beyond, but launches under 6 MB 1.13-1.35 (at 7
+ * and 8, which the matvec kernels also run on the matrix cores, 1.02-1.15
+ * from 17 units); at 2 positions 0.57-0.92 up to 24 units, 1.1-1.3 beyond.
+ * Q6_K at 5 to 8: 0.47-0.83 throughout; at 3 and 4 0.52-0.84 up to 16 units,
+ * 1.02-1.09 from 17, at 4 0.86 in launches of 50 MB; at 2 0.57-0.93 up to 8
+ * units, 1.18 at 17-24. Q8_0 and Q5_0 (units of 128 weights): 0.55-0.89 up to
+ * 12 units (Q5_0 at 3 and 4 1.03-1.07 from 9), 0.95-1.12 at 13-16, with the
+ * norm 0.68-0.89 up to 20, 1.05-1.6 beyond 24. One position: Q8_0 and Q5_0
+ * with the norm, 0.87-0.94 up to 8 units (Q8_0: 12), 1.0-1.1 at 13-20, 1.2-2.5
+ * beyond; without it never. */
 bool use_chunks(int fmt, int units, double bytes, int batch, bool norm)
 {
     if (batch > QMV_VALU_MAX_POSITIONS) return use_prefill(fmt, batch);
     /* A plan or threshold set by the caller applies to the matvec kernels. */
     if (g_target_waves.load() > 0 || g_force_u.load() > 0 || g_force_w.load() > 0 || g_mfma_min_batch.load() > 0)
         return false;
-    if (batch < 2) return false;
-    if (fmt == QMV_FMT_Q8_0 || fmt == QMV_FMT_Q5_0) return units <= (norm ? 20 : batch == 2 ? 8 : 12);
-    if (batch == 2) return units <= (fmt == QMV_FMT_Q4_K ? 24 : 16);
-    if (fmt == QMV_FMT_Q4_K) return batch <= 6 || units <= 24 || bytes >= 12e6;
-    return batch >= 5 || units <= 24 || bytes >= 30e6;
+    const bool q8 = fmt == QMV_FMT_Q8_0, q5 = fmt == QMV_FMT_Q5_0;
+    if (batch == 1) return norm && ((q8 && units <= 12) || (q5 && units <= 8));
+    if (q8 || q5) return units <= (norm ? 20 : batch == 2 || (q5 && batch <= 4) ? 8 : 12);
+    if (batch == 2) return units <= (fmt == QMV_FMT_Q4_K ? 24 : 8);
+    if (fmt == QMV_FMT_Q4_K) return units <= (batch >= 7 ? 16 : 24) || bytes >= 6e6;
+    return batch >= 5 || units <= 16 || (batch == 4 && bytes >= 30e6);
 }
 
 /* How a chunk_kernel launch is cut up. */
@@ -1016,8 +1020,9 @@ constexpr int kLdsBytes = 160 * 1024, kCus = 256;
 /* The cut with the least estimated time, over segment lengths and segments
  * per workgroup: one workgroup per CU; staging rounds and items per wave times
  * their instructions (4 cycles each at 2.4 GHz, times the waves that share a
- * SIMD, at least 0.45 us a unit for its loads); the weights at 5 TB/s; and
- * for launches that are not fused 3 us and the partial sums' traffic. At the
+ * SIMD, at least 0.45 us a unit for its loads); half the weights' time at 5 TB/s
+ * (the rest runs beside the products); what a segment and its length cost; and
+ * for launches that are not fused 4.6 us and the partial sums' traffic. At the
  * measured shapes it picks the fastest cut or one within 5% (Qwen2.5-7B o at
  * 4 positions: two units a segment 7.1 us, one 7.7, four 7.7; down at 8, two
  * segments of five a workgroup 23.2 us, of four 23.8, three of five 24.3).
@@ -1066,14 +1071,14 @@ BatchShape batch_shape(int fmt, int units, long long groups, int batch, bool swi
             const long long lds = (long long)staged * stage + (c.fused ? (segs * g2 * 64 + 4) * 4 * nr : 0);
             if (lds > kLdsBytes) continue;
             c.wg_groups = (int)(swiglu ? g2 : g1);
-            const long long items = g1 / r * c.chunk_segs;
+            const long long items = g1 / r * c.chunk_segs, made = c.wg_groups / r * c.chunk_segs;
             c.waves = r == 2 || (q6 && wide) ? 8 : wide || q6 || !c.fused ? 12 : 16;
-            c.waves = (int)std::min<long long>(c.waves, std::max<long long>(items, staged * nr));
+            c.waves = (int)std::min<long long>(c.waves, std::max<long long>(made, staged * nr));
             const long long busy = std::min<long long>(c.waves, items);
             const double per_unit = std::max(unit_us * ((busy + 3) / 4), 0.45);
             double us = stage_us * ((c.waves + 3) / 4) * ((staged * nr + c.waves - 1) / c.waves);
-            us += std::max((items + busy - 1) / busy * longest * per_unit, weights_us);
-            us += c.fused ? 0.6 + 0.06 * segs : 3.0 + 2.0 * segs * batch * groups * 64 / 4.0e6;
+            us += (items + busy - 1) / busy * longest * per_unit + 0.5 * weights_us;
+            us += 0.15 * longest + (c.fused ? 0.6 + 0.09 * segs : 4.6 + 2.0 * segs * batch * groups * 64 / 4.0e6);
             if (us < best_us) {
                 best_us = us;
                 best = c;
@@ -1950,13 +1955,6 @@ static int norm_then_group(QmvDeviceTensor *const *ts, int count, const float *d
                            int batch, float *const *d_out, float *d_normed, hipStream_t s, Workspace &ws,
                            Epilogue epi)
 {
-    if (batch == 1) {
-        epi.norm_w = d_w;
-        epi.norm_eps = eps;
-        ChunkPlan cp;
-        if (plan_rowdot(ts, count, d_in, 0, d_out, epi, &cp)) return enqueue_chunk(cp, s);
-        epi.norm_w = nullptr;
-    }
     /* Every workgroup reads the norm weights, so an output over them keeps
      * the two launches. */
     bool apart = true;
@@ -1965,7 +1963,8 @@ static int norm_then_group(QmvDeviceTensor *const *ts, int count, const float *d
     epi.norm_w = d_w;
     epi.norm_eps = eps;
     ChunkPlan cp;
-    if (batch > 1 && apart && plan_batch(ts, count, d_in, 0, batch, d_out, epi, false, &cp))
+    if (apart && batch == 1 && plan_rowdot(ts, count, d_in, 0, d_out, epi, &cp)) return enqueue_chunk(cp, s);
+    if (apart && plan_batch(ts, count, d_in, 0, batch, d_out, epi, false, &cp))
         return launch_chunk(ts, count, d_in, 0, batch, d_out, s, ws, epi);
     epi.norm_w = nullptr;
     HIP_TRY(qmv::launch_rms_norm(d_in, d_w, ts[0]->cols, batch, eps, d_normed, s));
@@ -2072,9 +2071,6 @@ QMV_API int qmv_device_embed_rows_f32(qmv_device_tensor t, const int *d_token_id
     }
     HIP_TRY(hipSetDevice(t->device));
     hipStream_t s = (hipStream_t)stream;
-    /* The status starts at 1 (a fill kernel, so the call can be captured)
-     * and the gather clears it on an out-of-range id. */
-    if (d_status != nullptr) HIP_TRY(qmv::launch_fill_u32((unsigned *)d_status, 1, 1u, s));
     HIP_TRY(qmv::launch_gather(t->geo.format, t->data, d_token_ids, count, d_output, t->rows, t->cols, t->units,
                                d_status, s));
     return 1;

@@ -95,7 +95,7 @@ def test_chunk_small_beside_large(qmv, oracle, gpu, hip, t, batch):
 
 
 @pytest.mark.parametrize("t", B.ALL_TYPES)
-@pytest.mark.parametrize("batch,cols", [(3, 1024), (8, 1024), (12, 1024), (32, 1024), (13, 5120), (6, 8960)])
+@pytest.mark.parametrize("batch,cols", [(1, 1024), (3, 1024), (8, 1024), (12, 1024), (32, 1024), (13, 5120), (6, 8960)])
 def test_chunk_norm_group(qmv, oracle, gpu, hip, t, batch, cols):
     """RMSNorm, three tensors of unequal rows and biases in one call, then the
     gate and up pair, against the oracle's norm and products; a NaN in one
@@ -122,7 +122,7 @@ def test_chunk_norm_group(qmv, oracle, gpu, hip, t, batch, cols):
         first = call()
         for raw, r, y, b in zip(raws, rows, first, bias):
             _check(oracle, raw, t, r, cols, normed, y - b[None, :], f"rows {r}", scale=2.0)
-        for bad in (np.nan, np.inf):
+        for bad in (np.nan, np.inf) if batch > 1 else ():
             x2 = x.copy()
             x2[1, cols // 3] = bad
             dx = hip.DeviceBuffer.from_array(x2)
