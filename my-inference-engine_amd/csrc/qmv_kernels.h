@@ -189,7 +189,7 @@ hipError_t launch_rowloop_q6k(const RowdotParams &p, int epi, int grid, int wave
 hipError_t launch_rowmajor_q6k(const uint8_t *raw, uint8_t *out, int rows, int sb, hipStream_t s);
 hipError_t launch_dequant(int fmt, const uint8_t *w, float *out, int rows, int cols, int units,
                           int first_row, int row_count, hipStream_t s);
-/* status (may be null): cleared to 0 if any id is outside [0, rows). */
+/* status (may be null): set to 1, or to 0 if any id is outside [0, rows). */
 hipError_t launch_gather(int fmt, const uint8_t *w, const int *ids, int count, float *out, int rows, int cols,
                          int units, int *status, hipStream_t s);
 hipError_t launch_repack(int fmt, const uint8_t *raw, uint8_t *out, int rows, int blocks_per_row,
