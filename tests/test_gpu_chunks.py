@@ -186,3 +186,24 @@ def test_chunk_output_over_norm_weights(qmv, oracle, gpu, hip):
         _check(oracle, raw, t, rows, cols, normed, dw.to_array(np.float32, (cols,))[:batch * rows].reshape(batch, rows),
                "over the weights", scale=2.0)
     dt.close()
+
+
+@pytest.mark.parametrize("t,rows,cols,batch", [(B.Q4_K, 4000, 1024, 170), (B.Q8_0, 3000, 512, 77)])
+def test_host_calls_of_several_launches(qmv, oracle, gpu, hip, t, rows, cols, batch):
+    """A host call of more launches than may wait at once (170 positions: 6)
+    and one of three, whose inputs and outputs are copied while launches run:
+    the bits of the same positions in calls of one launch each; an input
+    inside the output's memory is read before it is overwritten."""
+    raw = qmv.synth_tensor(t, rows, cols, seed=21)
+    v = qmv.make_view(raw, t, rows, cols)
+    x = qmv.synth_normal(batch * cols, seed=22).reshape(batch, cols)
+    print(f"chunks: host {B.NAMES[t]} {rows}x{cols} M={batch}", flush=True)
+    y = qmv.matvec(v, x)
+    parts = np.concatenate([qmv.matvec(v, x[b:b + 32]).reshape(-1, rows) for b in range(0, batch, 32)])
+    assert np.array_equal(_bits(y), _bits(parts))
+    shared = np.zeros(batch * rows, dtype=np.float32)
+    inp = shared[-batch * cols:]
+    inp[:] = x.reshape(-1)
+    assert qmv.quantized_tensor_matmul_f32(v, inp, cols, batch, shared, rows) == 1
+    assert np.array_equal(_bits(shared), _bits(y.reshape(-1)))
+    qmv.release_tensor(v.data)
