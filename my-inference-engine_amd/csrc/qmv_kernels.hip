@@ -905,23 +905,6 @@ __device__ __forceinline__ void publish_tile_candidate(const P &p, int tile, flo
     }
 }
 
-/* Index of the job that owns this workgroup (jobs own consecutive ranges of
- * workgroups from their wg_begin), walking the jobs: the prefill kernel's
- * choice. The single-position and matrix-core kernels read every job's start
- * in one batch of scalar loads instead (launch_args), and so does the
- * row-major kernel: each dependent kernel-argument load before the first
- * weight load is a scalar-cache round trip on every wave's critical path
- * (measured on the Qwen2.5-7B set: q|k|v 4.72 -> 4.60 us, o 3.95 -> 3.83,
- * gate|up 16.1-16.9 -> 15.7, the fused SwiGLU 16.8-16.9 -> 15.8-16.1, the
- * M = 8 set 2.282 -> 2.253 ms; down, a single job, unchanged). */
-template <typename P>
-__device__ __forceinline__ int job_of_block(const P &p)
-{
-    int j = 0;
-    while (j + 1 < p.njobs && (int)blockIdx.x >= p.job[j + 1].wg_begin) ++j;
-    return j;
-}
-
 /* The workgroup's place in a launch: job, tile, K-split, and this wave's
  * K-units [u_begin, u_end). */
 struct WgWork {
@@ -929,7 +912,10 @@ struct WgWork {
 };
 
 /* Kernel arguments a tiled launch needs before its first weight load, read in
- * one batch of scalar loads: the launch-wide values, job 0's fields, and the
+ * one batch of scalar loads (each dependent load before the first weight load
+ * is a scalar-cache round trip on every wave's critical path: the Qwen2.5-7B
+ * M = 8 set went 2.282 -> 2.253 ms, the row-major q|k|v 4.72 -> 4.60 us, with
+ * the jobs no longer walked): the launch-wide values, job 0's fields, and the
  * other jobs' first workgroups (unused job slots start past every workgroup,
  * set by the launchers). The job is the last one starting at or before this
  * workgroup; a job other than 0 then reads its own fields from lines this
