@@ -202,7 +202,9 @@ int qmv_device_matvec_group_f32(const qmv_device_tensor *tensors, int count,
  * counters are cleared by a fill kernel before each launch (no memset node).
  * All calls on one GPU share its array: calls that overlap in time on one
  * GPU (other streams, other threads) race and must be serialised by the
- * caller. Results are bit-identical to qmv_device_matvec_group_f32.
+ * caller. A launch of 9 to 32 positions that the rule accepts and whose
+ * partial sums would not fit is made with fewer of them or in pieces. Results
+ * are bit-identical to qmv_device_matvec_group_f32.
  */
 #define QMV_NOALLOC_SCRATCH_BYTES (32u << 20)
 #define QMV_NOALLOC_COUNTER_BYTES (512u << 10)

@@ -1027,6 +1027,7 @@ struct BatchShape {
     int nr, r;  /* rounds of 4 positions; row groups per wave */
     bool fused; /* all of K in one workgroup */
     int waves, segs, chunk_segs, wg_groups;
+    size_t partials; /* floats of workspace */
 };
 
 constexpr int kLdsBytes = 160 * 1024, kCus = 256;
@@ -1046,9 +1047,10 @@ constexpr int kLdsBytes = 160 * 1024, kCus = 256;
  * read the staged activations half as often (gate|up at 32 positions: 41.5
  * us against 48.9 with one) or for Q6_K (down at 32: 36 against 58 at 12).
  * The segments are the same with `swiglu` as without, and past 8 positions
- * they do not depend on the positions. `alone`: only a cut without workspace
- * (waves = 0 if there is none). */
-BatchShape batch_shape(int fmt, int units, long long groups, int batch, bool swiglu, bool alone)
+ * they do not depend on the positions. room: at most this many floats of
+ * workspace, which may take other cuts than those (waves = 0 if there is
+ * none). */
+BatchShape batch_shape(int fmt, int units, long long groups, int batch, bool swiglu, bool norm, size_t room)
 {
     const bool q32 = fmt == QMV_FMT_Q8_0 || fmt == QMV_FMT_Q5_0, q6 = fmt == QMV_FMT_Q6_K;
     const bool wide = batch > QMV_VALU_MAX_POSITIONS;
@@ -1069,21 +1071,30 @@ BatchShape batch_shape(int fmt, int units, long long groups, int batch, bool swi
                             : (kunits <= 40 && (groups <= 512 || (q6 && kunits <= 16 && groups <= 2048)) ? 2 : 4) *
                                   (q32 && units > 16 ? 2 : 1);
     double best_us = 1e30;
-    static const int kLengths[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16};
-    for (int length : kLengths) {
-        const int segs = (units + (fixed ? fixed : length) - 1) / (fixed ? fixed : length);
+    const int lengths[] = {fixed, 1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16};
+    for (int i = 0; i < 12; ++i) {
+        const int length = lengths[i];
+        if (length == 0) continue;
+        const int segs = (units + length - 1) / length;
         const int longest = (units + segs - 1) / segs;
-        for (int cs = 0; cs <= (alone ? 0 : wide ? 1 : 4) && cs <= segs; ++cs) { /* 0: fused */
+        for (int cs = 0; cs <= (wide ? 1 : 4) && cs <= segs; ++cs) { /* 0: fused */
             BatchShape c = best;
             c.fused = cs == 0;
             c.segs = segs;
             c.chunk_segs = c.fused ? segs : cs;
             const int chunks = (segs + c.chunk_segs - 1) / c.chunk_segs;
             const long long per = std::max(1, kCus / chunks);
-            const long long g1 = round_to((groups + per - 1) / per, r), g2 = round_to(g1, 2);
+            long long g1 = round_to((groups + per - 1) / per, r), g2 = round_to(g1, 2);
             const int staged = c.fused ? units : c.chunk_segs * longest;
+            if (c.fused && room != SIZE_MAX) { /* more workgroups than CUs rather than no cut */
+                const long long fit = ((long long)kLdsBytes - (long long)staged * stage - 16 * nr) / (segs * 256 * nr) & ~1ll;
+                if (fit >= 2 && g2 > fit) g1 = g2 = fit;
+            }
+            const double rounds = (double)std::max(1LL, (groups + g1 * kCus - 1) / (g1 * kCus));
             const long long lds = (long long)staged * stage + (c.fused ? (segs * g2 * 64 + 4) * 4 * nr : 0);
             if (lds > kLdsBytes) continue;
+            c.partials = c.fused ? 0 : (size_t)segs * batch * groups * 16 + (norm ? (size_t)units * 8 * nr : 0);
+            if (c.partials > room) continue;
             c.wg_groups = (int)(swiglu ? g2 : g1);
             const long long items = g1 / r * c.chunk_segs, made = c.wg_groups / r * c.chunk_segs;
             c.waves = r == 2 || (q6 && wide) ? 8 : wide || q6 || !c.fused ? 12 : 16;
@@ -1091,21 +1102,22 @@ BatchShape batch_shape(int fmt, int units, long long groups, int batch, bool swi
             const long long busy = std::min<long long>(c.waves, items);
             const double per_unit = std::max(unit_us * ((busy + 3) / 4), 0.45);
             double us = stage_us * ((c.waves + 3) / 4) * ((staged * nr + c.waves - 1) / c.waves);
-            us += (items + busy - 1) / busy * longest * per_unit + 0.5 * weights_us;
+            us = (us + (items + busy - 1) / busy * longest * per_unit) * (c.fused ? rounds : 1) + 0.5 * weights_us;
             us += 0.15 * longest + (c.fused ? 0.6 + 0.09 * segs : 4.6 + 2.0 * segs * batch * groups * 64 / 4.0e6);
             if (us < best_us) {
                 best_us = us;
                 best = c;
             }
         }
-        if (fixed) break;
+        if (i == 0 && (best_us < 1e30 || room == SIZE_MAX)) break; /* the fixed length, if it fits */
     }
     return best;
 }
 
-/* A chunk_kernel launch, if it is one that kernel takes. */
+/* A chunk_kernel launch, if it is one that kernel takes (and has a cut of at
+ * most `room` floats of workspace). */
 bool plan_batch(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch, float *const *d_out,
-                const Epilogue &epi, bool alone, ChunkPlan *cp)
+                const Epilogue &epi, ChunkPlan *cp, size_t room = SIZE_MAX)
 {
     const QmvDeviceTensor *t0 = ts[0];
     if (epi.argmax || (epi.swiglu && (count != 2 || ts[1]->rows != t0->rows))) return false;
@@ -1115,10 +1127,8 @@ bool plan_batch(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0
     if (groups > INT_MAX / 16) return false;
     if (!use_chunks(fmt, units, (double)groups * 16 * units * t0->geo.unit_bytes, batch, epi.norm_w != nullptr))
         return false;
-    const BatchShape b = batch_shape(fmt, units, groups, batch, epi.swiglu, alone);
-    if (b.waves == 0) return false;
-    const size_t partials = b.fused ? 0 : (size_t)b.segs * batch * groups * 16 + (epi.norm_w ? (size_t)units * 8 * b.nr : 0);
-    if (partials > (size_t)INT_MAX) return false;
+    const BatchShape b = batch_shape(fmt, units, groups, batch, epi.swiglu, epi.norm_w != nullptr, room);
+    if (b.waves == 0 || b.partials > (size_t)INT_MAX) return false;
     qmv::BatchParams &p = cp->bp;
     memset(&p, 0, sizeof p);
     p.njobs = count;
@@ -1158,32 +1168,30 @@ bool plan_batch(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0
     cp->bt_fused = b.fused;
     cp->waves = b.waves;
     cp->fmt = fmt;
-    cp->partials = partials;
+    cp->partials = b.partials;
     cp->counters = 0;
     cp->pair_vals = cp->pair_count = 0;
     cp->argmax_tiles = 0;
     return true;
 }
 
-/* A launch on the matvec kernels (up to 8 positions). */
-int plan_tiled(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch, float *const *d_out,
-               const Epilogue &epi, ChunkPlan *cp)
+/* How the matvec kernels (up to 8 positions) cut a launch, and the workspace
+ * that takes. */
+struct TiledCut {
+    Plan plan;
+    int parts; /* work items per unit */
+    bool mfma, paired;
+    size_t partials = 0, counters = 0;
+};
+
+TiledCut tiled_cut(QmvDeviceTensor *const *ts, int count, int batch, const Epilogue &epi)
 {
     const QmvDeviceTensor *t0 = ts[0];
-    cp->rowdot = cp->batch = false;
-    if (epi.norm_w) {
-        set_error("internal: a fused RMSNorm reached the tiled planner");
-        return 0;
-    }
-    if (batch > QMV_VALU_MAX_POSITIONS) {
-        set_error("more than 8 positions per launch need the matrix-core path");
-        return 0;
-    }
-    const bool mfma = use_matrix_cores(t0->geo.format, batch);
-    const int mt = batch;
+    TiledCut c;
+    const bool mfma = c.mfma = use_matrix_cores(t0->geo.format, batch);
     long long total_tiles = 0;
     for (int i = 0; i < count; ++i) total_tiles += ts[i]->tiles;
-    const int parts = mfma ? mfma_parts(t0->units, total_tiles) : batch >= 2 ? valu_parts(t0->units) : 1;
+    const int parts = c.parts = mfma ? mfma_parts(t0->units, total_tiles) : batch >= 2 ? valu_parts(t0->units) : 1;
     /* Single-position launches of many units (the vocabulary projection:
      * 33236) run several rounds of resident waves; five waves per workgroup
      * (three splits of 14 units instead of four) measured 80.9 us against
@@ -1221,8 +1229,48 @@ int plan_tiled(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0,
                             : mfma                                          ? mfma_waves
                             : batch == 1 && total_tiles * t0->units > 2048  ? 2
                                                                             : 4;
-    const Plan plan = plan_for(total_tiles, t0->units * parts, batch == 1 ? 6 : long_batch_waves, short_waves,
-                               mfma || parts > 1 ? 1 : 8);
+    const Plan plan = c.plan = plan_for(total_tiles, t0->units * parts, batch == 1 ? 6 : long_batch_waves, short_waves,
+                                        mfma || parts > 1 ? 1 : 8);
+    /* Fused SwiGLU at M = 1 with one unit per wave: one workgroup per
+     * (tile, split) of both projections (finish_paired), when the two halves
+     * fit a workgroup. */
+    c.paired = epi.swiglu && count == 2 && batch == 1 && !mfma &&
+               plan.units_per_wave == 1 && 2 * plan.waves <= QMV_MAX_WAVES &&
+               ts[0]->rows == ts[1]->rows && g_paired_swiglu.load() != 0;
+    /* The split-K workspace: each split's sums (paired: gate's and up's, one
+     * count per tile), then with SwiGLU otherwise both projections' final
+     * tiles and one count per tile pair. */
+    if (plan.splits > 1) {
+        const size_t tiles = c.paired ? t0->tiles : (size_t)total_tiles;
+        c.partials = tiles * plan.splits * (c.paired ? 2 : batch) * 64;
+        c.counters = tiles * QMV_COUNTER_STRIDE;
+    }
+    if (epi.swiglu && !c.paired) {
+        c.partials += (size_t)2 * t0->tiles * batch * 64;
+        c.counters += (size_t)t0->tiles * QMV_COUNTER_STRIDE;
+    }
+    if (c.partials) c.partials += QMV_PARTIAL_PAD; /* padding past the last partial */
+    return c;
+}
+
+/* A launch on the matvec kernels (up to 8 positions). */
+int plan_tiled(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch, float *const *d_out,
+               const Epilogue &epi, ChunkPlan *cp)
+{
+    const QmvDeviceTensor *t0 = ts[0];
+    cp->rowdot = cp->batch = false;
+    if (epi.norm_w) {
+        set_error("internal: a fused RMSNorm reached the tiled planner");
+        return 0;
+    }
+    if (batch > QMV_VALU_MAX_POSITIONS) {
+        set_error("more than 8 positions per launch need the matrix-core path");
+        return 0;
+    }
+    const TiledCut cut = tiled_cut(ts, count, batch, epi);
+    const Plan &plan = cut.plan;
+    const int mt = batch, parts = cut.parts;
+    const bool mfma = cut.mfma, paired = cut.paired;
 
     qmv::MatvecParams &p = cp->p;
     memset(&p, 0, sizeof p);
@@ -1238,12 +1286,6 @@ int plan_tiled(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0,
         return 0;
     }
     p.positions = batch;
-    /* Fused SwiGLU at M = 1 with one unit per wave: one workgroup per
-     * (tile, split) of both projections (finish_paired), when the two halves
-     * fit a workgroup. */
-    const bool paired = epi.swiglu && count == 2 && batch == 1 && !mfma &&
-                        plan.units_per_wave == 1 && 2 * plan.waves <= QMV_MAX_WAVES &&
-                        ts[0]->rows == ts[1]->rows && g_paired_swiglu.load() != 0;
     size_t partials = 0, counters = 0;
     long long wg = 0;
     for (int i = 0; i < count; ++i) {
@@ -1312,19 +1354,107 @@ int plan_tiled(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0,
     cp->grid = (int)wg;
     cp->waves = paired ? 2 * plan.waves : plan.waves;
     cp->fmt = t0->geo.format;
-    cp->partials = partials ? partials + QMV_PARTIAL_PAD : 0; /* padding past the last partial */
-    cp->counters = counters;
+    cp->partials = cut.partials;
+    cp->counters = cut.counters;
     return 1;
 }
 
-/* alone: without workspace where chunk_kernel takes the launch. */
 int plan_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch, float *const *d_out,
-               const Epilogue &epi, ChunkPlan *cp, bool alone = false)
+               const Epilogue &epi, ChunkPlan *cp, size_t room = SIZE_MAX)
 {
     cp->rowdot = cp->batch = false;
     if (batch == 1 && plan_rowdot(ts, count, d_in, b0, d_out, epi, cp)) return 1;
-    if (plan_batch(ts, count, d_in, b0, batch, d_out, epi, alone, cp)) return 1;
+    if (plan_batch(ts, count, d_in, b0, batch, d_out, epi, cp, room)) return 1;
     return plan_tiled(ts, count, d_in, b0, batch, d_out, epi, cp);
+}
+
+/* A launch made as even pieces of its positions, each planned within `room`
+ * floats of workspace. */
+struct Cut {
+    int pieces = 1;
+    size_t room = SIZE_MAX;
+};
+
+/* Positions of piece i of a launch of `batch`. */
+int piece_positions(int batch, int pieces, int i) { return batch / pieces + (i < batch % pieces ? 1 : 0); }
+
+/* Whether every piece of a launch needs at most `partials` floats and
+ * `counters` words when planned within c->room. */
+bool cut_fits(QmvDeviceTensor *const *ts, int count, const float *d_in, int batch, float *const *d_out,
+              const Epilogue &epi, const Cut &c, size_t partials, size_t counters)
+{
+    ChunkPlan cp;
+    const int longer = piece_positions(batch, c.pieces, 0), shorter = piece_positions(batch, c.pieces, c.pieces - 1);
+    for (int nb = longer; nb >= shorter; --nb)
+        if (!plan_chunk(ts, count, d_in, 0, nb, d_out, epi, &cp, c.room) || cp.partials > partials ||
+            cp.counters > counters)
+            return false;
+    return true;
+}
+
+/* The no-allocation entry point's scratch array (include/qmv_hip.h). */
+constexpr size_t kScratchCounters = QMV_NOALLOC_COUNTER_BYTES / sizeof(unsigned);
+constexpr size_t kScratchPartials = (QMV_NOALLOC_SCRATCH_BYTES - QMV_NOALLOC_COUNTER_BYTES) / sizeof(float);
+
+struct WorkspaceNeed {
+    size_t partials = 0, counters = 0;
+};
+
+/* The workspace that decides whether the no-allocation entry point accepts a
+ * launch (what it takes does not depend on the kernel that runs it): up to 8
+ * positions that of the matvec kernels; past 8, the partial sums of 16 or 32
+ * position rows over K in splits of 1, 2 or 5 units by the tensors' groups of
+ * four tiles (a forced plan's units per wave). */
+WorkspaceNeed workspace_rule(QmvDeviceTensor *const *ts, int count, const float *d_in, int batch, float *const *d_out,
+                             const Epilogue &epi)
+{
+    WorkspaceNeed n;
+    if (batch <= QMV_VALU_MAX_POSITIONS) {
+        ChunkPlan cp;
+        if (batch == 1 && plan_rowdot(ts, count, d_in, 0, d_out, epi, &cp)) return n;
+        const TiledCut cut = tiled_cut(ts, count, batch, epi);
+        n.partials = cut.partials;
+        n.counters = cut.counters;
+        return n;
+    }
+    const int units = ts[0]->units, force_u = g_force_u.load();
+    long long tiles = 0, fours = 0;
+    for (int i = 0; i < count; ++i) {
+        tiles += ts[i]->tiles;
+        fours += (ts[i]->tiles + 3) / 4;
+    }
+    const int split = force_u > 0    ? force_u
+                      : units >= 32  ? (fours <= 8 ? 2 : 5)
+                      : fours >= 100 ? 5
+                      : fours <= 20  ? 1
+                                     : 2;
+    const size_t rows = batch <= 16 ? 16 : QMV_MFMA_MAX_POSITIONS;
+    if (units > split) {
+        n.partials = (size_t)tiles * ((units + split - 1) / split) * rows * 64;
+        n.counters = (size_t)tiles * QMV_COUNTER_STRIDE;
+    }
+    if (epi.swiglu) {
+        n.partials += (size_t)2 * ts[0]->tiles * rows * 64;
+        n.counters += (size_t)ts[0]->tiles * QMV_COUNTER_STRIDE;
+    }
+    if (n.partials) n.partials += QMV_PARTIAL_PAD;
+    return n;
+}
+
+/* How the no-allocation entry point makes a launch that workspace_rule
+ * accepts: whole; where its partial sums do not fit, as several pieces past 8
+ * positions, which have the same bits; else within the scratch, whole or in
+ * pieces. The last have other bits than the launch without a limit, so the
+ * plain entry point makes those in the same way. */
+bool scratch_cut(QmvDeviceTensor *const *ts, int count, const float *d_in, int batch, float *const *d_out, Cut *c)
+{
+    *c = Cut();
+    for (c->pieces = 1; c->pieces == 1 || batch / c->pieces > QMV_VALU_MAX_POSITIONS; ++c->pieces)
+        if (cut_fits(ts, count, d_in, batch, d_out, Epilogue(), *c, kScratchPartials, kScratchCounters)) return true;
+    c->room = kScratchPartials;
+    for (c->pieces = 1; c->pieces == 1 || batch / c->pieces >= 2; ++c->pieces)
+        if (cut_fits(ts, count, d_in, batch, d_out, Epilogue(), *c, kScratchPartials, kScratchCounters)) return true;
+    return false;
 }
 
 /* Point the plan at its split-K workspace: partials[cp.partials] floats and
@@ -1366,6 +1496,13 @@ int launch_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b
 {
     ChunkPlan cp;
     if (!plan_chunk(ts, count, d_in, b0, batch, d_out, epi, &cp)) return 0;
+    Cut cut;
+    if (cp.batch && cp.partials > kScratchPartials && !epi.add && !epi.swiglu && !epi.norm_w) {
+        const WorkspaceNeed rule = workspace_rule(ts, count, d_in, batch, d_out, epi);
+        if (rule.partials > kScratchPartials || rule.counters > kScratchCounters ||
+            !scratch_cut(ts, count, d_in, batch, d_out, &cut) || cut.room == SIZE_MAX)
+            cut = Cut();
+    }
     std::lock_guard<std::mutex> lock(ws.mu);
     if (cp.batch && cp.partials > ws.partial_cap) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -1374,8 +1511,8 @@ int launch_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b
             for (int b = 0; b < batch; b += QMV_VALU_MAX_POSITIONS) {
                 ChunkPlan part;
                 part.batch = false;
-                if (!plan_batch(ts, count, d_in, b0 + b, std::min(QMV_VALU_MAX_POSITIONS, batch - b), d_out, epi, true,
-                                &part))
+                if (!plan_batch(ts, count, d_in, b0 + b, std::min(QMV_VALU_MAX_POSITIONS, batch - b), d_out, epi,
+                                &part, 0))
                     break;
                 parts.push_back(part);
             }
@@ -1386,14 +1523,22 @@ int launch_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b
             }
         }
     }
-    if (!workspace_reserve(ws, stream, cp.partials, cp.counters)) return 0;
-    bind_workspace(cp, ws.partials, ws.counters);
-    if (cp.argmax_tiles) {
-        if (!workspace_fused_argmax(ws, stream, cp.argmax_tiles)) return 0;
-        cp.p.argmax_cand = cp.rp.argmax_cand = ws.fused_cand;
-        cp.p.argmax_count = cp.rp.argmax_count = ws.fused_count;
+    for (int i = 0; i < cut.pieces; ++i) {
+        const int nb = piece_positions(batch, cut.pieces, i);
+        if ((cut.pieces > 1 || cut.room != SIZE_MAX) &&
+            !plan_chunk(ts, count, d_in, b0, nb, d_out, epi, &cp, cut.room))
+            return 0;
+        if (!workspace_reserve(ws, stream, cp.partials, cp.counters)) return 0;
+        bind_workspace(cp, ws.partials, ws.counters);
+        if (cp.argmax_tiles) {
+            if (!workspace_fused_argmax(ws, stream, cp.argmax_tiles)) return 0;
+            cp.p.argmax_cand = cp.rp.argmax_cand = ws.fused_cand;
+            cp.p.argmax_count = cp.rp.argmax_count = ws.fused_count;
+        }
+        if (!enqueue_chunk(cp, stream)) return 0;
+        b0 += nb;
     }
-    return enqueue_chunk(cp, stream);
+    return 1;
 }
 
 /* Positions per launch for the remaining `batch` positions of a call: up to
@@ -1830,38 +1975,6 @@ int scratch_address(int device, void **out)
     return 1;
 }
 
-/* The scratch that decides whether a launch is accepted (what the entry
- * point takes does not depend on the kernel that runs it): up to 8 positions
- * that of the matvec kernels; past 8, the partial sums of 16 or 32 position
- * rows over K in splits of 1, 2 or 5 units by the tensors' groups of four
- * tiles. */
-int scratch_rule(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch, float *const *d_out,
-                 size_t *partials, size_t *counters)
-{
-    ChunkPlan cp;
-    if (batch <= QMV_VALU_MAX_POSITIONS) {
-        cp.rowdot = cp.batch = false;
-        if (!(batch == 1 && plan_rowdot(ts, count, d_in, b0, d_out, Epilogue(), &cp)) &&
-            !plan_tiled(ts, count, d_in, b0, batch, d_out, Epilogue(), &cp))
-            return 0;
-        *partials = cp.partials;
-        *counters = cp.counters;
-        return 1;
-    }
-    const int units = ts[0]->units;
-    long long tiles = 0, fours = 0;
-    for (int i = 0; i < count; ++i) {
-        tiles += ts[i]->tiles;
-        fours += (ts[i]->tiles + 3) / 4;
-    }
-    const int split = units >= 32 ? (fours <= 8 ? 2 : 5) : fours >= 100 ? 5 : fours <= 20 ? 1 : 2;
-    if (units > split) {
-        *partials = (size_t)tiles * ((units + split - 1) / split) * (batch <= 16 ? 16 : 32) * 64 + QMV_PARTIAL_PAD;
-        *counters = (size_t)tiles * QMV_COUNTER_STRIDE;
-    }
-    return 1;
-}
-
 } // namespace
 
 QMV_API int qmv_device_matvec_group_noalloc_f32(const qmv_device_tensor *tensors, int count, const float *d_inputs,
@@ -1874,50 +1987,43 @@ QMV_API int qmv_device_matvec_group_noalloc_f32(const qmv_device_tensor *tensors
     if (!scratch_address(dev, &base)) return 0;
     unsigned *counters = (unsigned *)base;
     float *partials = (float *)((unsigned char *)base + QMV_NOALLOC_COUNTER_BYTES);
-    const size_t counter_cap = QMV_NOALLOC_COUNTER_BYTES / sizeof(unsigned);
-    const size_t partial_cap = (QMV_NOALLOC_SCRATCH_BYTES - QMV_NOALLOC_COUNTER_BYTES) / sizeof(float);
     QmvDeviceTensor *const *ts = const_cast<QmvDeviceTensor *const *>(tensors);
     const int fmt = ts[0]->geo.format;
     /* Every launch is planned and checked before the first is enqueued, so a
      * call that does not fit launches nothing. */
-    std::vector<ChunkPlan> plans;
-    for (int b0 = 0; b0 < batch_count;) {
+    Cut cuts[QMV_MAX_BATCH];
+    int n = 0;
+    for (int b0 = 0; b0 < batch_count; ++n) {
         const int nb = next_chunk(fmt, batch_count, b0);
-        size_t need_partials = 0, need_counters = 0;
-        if (!scratch_rule(ts, count, d_inputs, b0, nb, d_outputs, &need_partials, &need_counters)) return 0;
-        bool fits = need_partials <= partial_cap && need_counters <= counter_cap;
-        /* A launch past 8 positions whose partial sums do not fit is made as
-         * several of at least 9, which have the same bits. */
-        int pieces = 1;
-        for (; fits; ++pieces) {
-            ChunkPlan cp;
-            if (!plan_chunk(ts, count, d_inputs, b0, (nb + pieces - 1) / pieces, d_outputs, Epilogue(), &cp)) return 0;
-            need_partials = cp.partials;
-            if (cp.partials <= partial_cap && cp.counters <= counter_cap) break;
-            fits = nb / (pieces + 1) > QMV_VALU_MAX_POSITIONS;
-        }
-        if (!fits) {
+        const WorkspaceNeed need = workspace_rule(ts, count, d_inputs, nb, d_outputs, Epilogue());
+        if (need.partials > kScratchPartials || need.counters > kScratchCounters) {
             set_error("launch needs %zu partial floats and %zu counters; the no-allocation scratch holds %zu and "
                       "%zu (use qmv_device_matvec_group_f32)",
-                      need_partials, need_counters, partial_cap, counter_cap);
+                      need.partials, need.counters, kScratchPartials, kScratchCounters);
             return 0;
         }
-        for (int i = 0, b = b0; i < pieces; ++i) {
-            const int n = nb / pieces + (i < nb % pieces ? 1 : 0);
-            plans.emplace_back();
-            if (!plan_chunk(ts, count, d_inputs, b, n, d_outputs, Epilogue(), &plans.back())) return 0;
-            b += n;
+        if (!scratch_cut(ts, count, d_inputs, nb, d_outputs, &cuts[n])) {
+            set_error("internal: no plan of %d positions fits the no-allocation scratch", nb);
+            return 0;
         }
         b0 += nb;
     }
     hipStream_t s = (hipStream_t)stream;
-    for (ChunkPlan &cp : plans) {
-        bind_workspace(cp, partials, counters);
-        /* The counters must be zero when the launch starts. Completed
-         * launches leave them zero; the fill (a kernel, not a memset node, so
-         * the call can be captured) also covers an interrupted earlier one. */
-        HIP_TRY(qmv::launch_fill_u32(counters, cp.counters, 0u, s));
-        if (!enqueue_chunk(cp, s)) return 0;
+    n = 0;
+    for (int b0 = 0; b0 < batch_count; ++n) {
+        const int nb = next_chunk(fmt, batch_count, b0);
+        for (int i = 0; i < cuts[n].pieces; ++i) {
+            ChunkPlan cp;
+            const int np = piece_positions(nb, cuts[n].pieces, i);
+            if (!plan_chunk(ts, count, d_inputs, b0, np, d_outputs, Epilogue(), &cp, cuts[n].room)) return 0;
+            bind_workspace(cp, partials, counters);
+            /* The counters must be zero when the launch starts. Completed
+             * launches leave them zero; the fill (a kernel, not a memset node, so
+             * the call can be captured) also covers an interrupted earlier one. */
+            HIP_TRY(qmv::launch_fill_u32(counters, cp.counters, 0u, s));
+            if (!enqueue_chunk(cp, s)) return 0;
+            b0 += np;
+        }
     }
     return 1;
 }
@@ -2012,7 +2118,7 @@ static int norm_then_group(QmvDeviceTensor *const *ts, int count, const float *d
     epi.norm_eps = eps;
     ChunkPlan cp;
     if (apart && batch == 1 && plan_rowdot(ts, count, d_in, 0, d_out, epi, &cp)) return enqueue_chunk(cp, s);
-    if (apart && plan_batch(ts, count, d_in, 0, batch, d_out, epi, false, &cp))
+    if (apart && plan_batch(ts, count, d_in, 0, batch, d_out, epi, &cp))
         return launch_chunk(ts, count, d_in, 0, batch, d_out, s, ws, epi);
     epi.norm_w = nullptr;
     HIP_TRY(qmv::launch_rms_norm(d_in, d_w, ts[0]->cols, batch, eps, d_normed, s));

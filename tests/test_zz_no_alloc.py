@@ -144,3 +144,17 @@ def test_graph_capture_and_replays(qmv, gpu, hip, t, rows, cols, batch):
                 qmv.device_matvec_group_noalloc(dts, dx.ptr, batch, [dy.ptr], stream.handle)
                 stream.synchronize()
         dts[0].close()
+
+
+@pytest.mark.parametrize("t,rows,cols,batch", [(B.Q6_K, 151936, 3584, 16), (B.Q4_K, 128256, 4864, 13),
+                                               (B.Q8_0, 262144, 640, 17), (B.Q8_0, 262144, 640, 18)])
+def test_launches_within_the_scratch(qmv, gpu, hip, t, rows, cols, batch):
+    """Launches whose segments' sums would not fit the scratch array: with
+    fewer segments at 13 and 16 positions and in pieces at 17, by both entry
+    points; at 18, of which pieces have the bits of the whole, in pieces by
+    the no-allocation one only."""
+    with hip.Stream() as stream:
+        dts = _tensors(qmv, t, [rows], cols, seed=rows + batch)
+        log(f"noalloc: {B.NAMES[t]} {rows}x{cols}, M={batch}")
+        _run_both(qmv, hip, dts, batch, seed=batch, stream=stream)
+        dts[0].close()
