@@ -171,6 +171,10 @@ int qmv_device_tensor_info(qmv_device_tensor tensor, int *rows, int *columns,
  * stream without host synchronisation (1 <= batch_count <= QMV_MAX_BATCH).
  * Batches of 9 to 32 positions (prefill chunks larger than the reference's
  * 8, src/qwen2_internal.h:7) read the weights once, on the matrix cores.
+ * Under graph capture a launch that would have to grow the stream's workspace
+ * is made within the workspace there is, where it can be (rows of a few
+ * K-units need none), and fails otherwise: run the call once before it is
+ * captured. Made so, it may sum in another order than the eager call.
  */
 int qmv_device_matvec_f32(qmv_device_tensor tensor, const float *d_inputs,
                           int batch_count, float *d_outputs, void *stream);

@@ -1128,7 +1128,7 @@ bool plan_batch(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0
     if (!use_chunks(fmt, units, (double)groups * 16 * units * t0->geo.unit_bytes, batch, epi.norm_w != nullptr))
         return false;
     const BatchShape b = batch_shape(fmt, units, groups, batch, epi.swiglu, epi.norm_w != nullptr, room);
-    if (b.waves == 0 || b.partials > (size_t)INT_MAX) return false;
+    if (b.waves == 0) return false;
     qmv::BatchParams &p = cp->bp;
     memset(&p, 0, sizeof p);
     p.njobs = count;
@@ -1392,6 +1392,17 @@ bool cut_fits(QmvDeviceTensor *const *ts, int count, const float *d_in, int batc
     return true;
 }
 
+/* A launch within `partials` floats and `counters` words: whole, or in the
+ * fewest pieces. Its bits are not those of the launch without a limit. */
+bool cut_within(QmvDeviceTensor *const *ts, int count, const float *d_in, int batch, float *const *d_out,
+                const Epilogue &epi, size_t partials, size_t counters, Cut *c)
+{
+    c->room = partials;
+    for (c->pieces = 1; c->pieces == 1 || batch / c->pieces >= 2; ++c->pieces)
+        if (cut_fits(ts, count, d_in, batch, d_out, epi, *c, partials, counters)) return true;
+    return false;
+}
+
 /* The no-allocation entry point's scratch array (include/qmv_hip.h). */
 constexpr size_t kScratchCounters = QMV_NOALLOC_COUNTER_BYTES / sizeof(unsigned);
 constexpr size_t kScratchPartials = (QMV_NOALLOC_SCRATCH_BYTES - QMV_NOALLOC_COUNTER_BYTES) / sizeof(float);
@@ -1451,10 +1462,7 @@ bool scratch_cut(QmvDeviceTensor *const *ts, int count, const float *d_in, int b
     *c = Cut();
     for (c->pieces = 1; c->pieces == 1 || batch / c->pieces > QMV_VALU_MAX_POSITIONS; ++c->pieces)
         if (cut_fits(ts, count, d_in, batch, d_out, Epilogue(), *c, kScratchPartials, kScratchCounters)) return true;
-    c->room = kScratchPartials;
-    for (c->pieces = 1; c->pieces == 1 || batch / c->pieces >= 2; ++c->pieces)
-        if (cut_fits(ts, count, d_in, batch, d_out, Epilogue(), *c, kScratchPartials, kScratchCounters)) return true;
-    return false;
+    return cut_within(ts, count, d_in, batch, d_out, Epilogue(), kScratchPartials, kScratchCounters, c);
 }
 
 /* Point the plan at its split-K workspace: partials[cp.partials] floats and
@@ -1488,9 +1496,10 @@ int enqueue_chunk(const ChunkPlan &cp, hipStream_t stream)
 
 /* Plan a launch and enqueue it on the stream's own workspace (grown here if
  * needed, outside graph capture only). A chunk_kernel launch that would have
- * to grow it during a capture is made as launches of up to 8 positions that
- * need no workspace, where there are such (short rows, which never needed
- * any). */
+ * to grow it during a capture is made within what there is, if it can be:
+ * with fewer segments, or in pieces (so its bits may not be those of the
+ * eager launch). Short rows need no workspace on any path but this kernel's
+ * fastest, so a stream that never ran them can capture them. */
 int launch_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch,
                  float *const *d_out, hipStream_t stream, Workspace &ws, const Epilogue &epi)
 {
@@ -1506,22 +1515,9 @@ int launch_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b
     std::lock_guard<std::mutex> lock(ws.mu);
     if (cp.batch && cp.partials > ws.partial_cap) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
-            std::vector<ChunkPlan> parts;
-            for (int b = 0; b < batch; b += QMV_VALU_MAX_POSITIONS) {
-                ChunkPlan part;
-                part.batch = false;
-                if (!plan_batch(ts, count, d_in, b0 + b, std::min(QMV_VALU_MAX_POSITIONS, batch - b), d_out, epi,
-                                &part, 0))
-                    break;
-                parts.push_back(part);
-            }
-            if ((int)parts.size() * QMV_VALU_MAX_POSITIONS >= batch) {
-                for (const ChunkPlan &part : parts)
-                    if (!enqueue_chunk(part, stream)) return 0;
-                return 1;
-            }
-        }
+        if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone &&
+            !cut_within(ts, count, d_in, batch, d_out, epi, ws.partial_cap, ws.counter_cap, &cut))
+            cut = Cut();
     }
     for (int i = 0; i < cut.pieces; ++i) {
         const int nb = piece_positions(batch, cut.pieces, i);

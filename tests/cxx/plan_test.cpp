@@ -4,7 +4,9 @@
  * launch is made. `plan_test scratch`: every launch that the no-allocation
  * entry point's rule accepts is made (its plans fit the scratch and a
  * workgroup's LDS), and as the plain entry point makes it (equal segments, so
- * equal bits).
+ * equal bits). `plan_test capture`: every launch that fits a workspace of
+ * that rule's size can be captured on a stream that holds just that, which
+ * for short rows is nothing: plain and grouped, with the norm and SwiGLU.
  */
 #include "../../my-inference-engine_amd/csrc/qmv_shim.cpp"
 
@@ -85,6 +87,41 @@ void check_scratch(const QmvDeviceTensor &t, int batch)
     if (b0 != batch) fail("pieces do not add up", t, batch);
 }
 
+void check_capture(const QmvDeviceTensor &t, int batch)
+{
+    const QmvDeviceTensor kv = tensor(t.geo.format, (t.rows + 7) / 8, t.units);
+    QmvDeviceTensor *ts[3] = {const_cast<QmvDeviceTensor *>(&t), const_cast<QmvDeviceTensor *>(&kv),
+                              const_cast<QmvDeviceTensor *>(&kv)};
+    QmvDeviceTensor *pair[2] = {ts[0], ts[0]};
+    float dummy = 0.0f, *out[3] = {&dummy, &dummy, &dummy};
+    for (int form = 0; form < 5; ++form) {
+        const bool swiglu = form >= 3, norm = form == 2 || form == 4;
+        QmvDeviceTensor *const *tensors = swiglu ? pair : ts;
+        const int count = swiglu ? 2 : form == 0 ? 1 : 3;
+        Epilogue epi;
+        epi.swiglu = swiglu;
+        const WorkspaceNeed rule = workspace_rule(tensors, count, &dummy, batch, out, epi);
+        ChunkPlan cp;
+        if (norm) { /* as norm_then_group */
+            epi.norm_w = &dummy;
+            if (batch == 1 && plan_rowdot(tensors, count, &dummy, 0, out, epi, &cp)) continue;
+            if (!plan_batch(tensors, count, &dummy, 0, batch, out, epi, &cp)) epi.norm_w = nullptr;
+        }
+        if (!plan_chunk(tensors, count, &dummy, 0, batch, out, epi, &cp)) { fail("not planned", t, batch); continue; }
+        if (!lds_fits(cp)) fail("over LDS", t, batch);
+        if (cp.partials <= rule.partials && cp.counters <= rule.counters) continue;
+        Cut cut;
+        if (!cut_within(tensors, count, &dummy, batch, out, epi, rule.partials, rule.counters, &cut)) {
+            fail("cannot be captured", t, batch);
+            continue;
+        }
+        for (int i = 0; i < cut.pieces; ++i)
+            if (!plan_chunk(tensors, count, &dummy, 0, piece_positions(batch, cut.pieces, i), out, epi, &cp, cut.room) ||
+                cp.partials > rule.partials || cp.counters > rule.counters || !lds_fits(cp))
+                fail("piece over the workspace or LDS", t, batch);
+    }
+}
+
 } // namespace
 
 int main(int argc, char **argv)
@@ -97,6 +134,7 @@ int main(int argc, char **argv)
                 for (int batch = 1; batch <= QMV_MAX_BATCH; ++batch) {
                     const QmvDeviceTensor t = tensor(f, rows, units);
                     if (!strcmp(argv[1], "scratch")) check_scratch(t, batch);
+                    else if (!strcmp(argv[1], "capture")) check_capture(t, batch);
                     else return 2;
                     ++launches;
                 }

@@ -207,3 +207,33 @@ def test_host_calls_of_several_launches(qmv, oracle, gpu, hip, t, rows, cols, ba
     assert qmv.quantized_tensor_matmul_f32(v, inp, cols, batch, shared, rows) == 1
     assert np.array_equal(_bits(shared), _bits(y.reshape(-1)))
     qmv.release_tensor(v.data)
+
+
+@pytest.mark.parametrize("t,rows,cols,batch,norm", [(B.Q4_K, 151936, 1024, 25, False), (B.Q6_K, 151936, 1024, 17, False),
+                                                    (B.Q8_0, 262144, 640, 17, False), (B.Q8_0, 262144, 640, 9, True)])
+def test_chunk_capture_of_short_rows(qmv, oracle, gpu, hip, t, rows, cols, batch, norm):
+    """Many short rows, whose fastest launch has a workspace: captured on a
+    stream that has none, at positions that leave one over from eights; the
+    replays against the oracle at three positions."""
+    raw, dt = _tensor(qmv, t, rows, cols, 5)
+    x = qmv.synth_normal(batch * cols, seed=6).reshape(batch, cols)
+    nw = (1 + 0.1 * qmv.synth_normal(cols, seed=7)).astype(np.float32)
+    dx, dy = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(4 * batch * rows)
+    dw, dn = hip.DeviceBuffer.from_array(nw), hip.DeviceBuffer(4 * batch * cols)
+    ref_x = np.stack([oracle.rms_norm(v, nw, 1e-6)[1] for v in x]) if norm else x
+    with hip.Stream() as s, hip.Graph(s) as g:
+        print(f"chunks: capture of short rows {B.NAMES[t]} {rows}x{cols} M={batch}", flush=True)
+        g.begin()
+        if norm:
+            qmv.device_rms_norm_matvec_add_group([dt], dx.ptr, dw.ptr, 1e-6, batch, [0], [0], [dy.ptr], dn.ptr, s.handle)
+        else:
+            dt.matvec(dx.ptr, batch, dy.ptr, s.handle)
+        g.end()
+        for _ in range(2):
+            dy.fill(0)
+            g.replay()
+            s.synchronize()
+            some = [0, batch // 2, batch - 1]
+            _check(oracle, raw, t, rows, cols, ref_x[some], dy.to_array(np.float32, (batch, rows))[some], "replay",
+                   scale=2.0 if norm else 1.0)
+    dt.close()

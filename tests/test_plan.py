@@ -9,7 +9,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-@pytest.mark.parametrize("what", ["scratch"])
+@pytest.mark.parametrize("what", ["scratch", "capture"])
 def test_plans(what):
     exe = os.path.join(ROOT, "tests", "cxx", "plan_test")
     assert os.path.exists(exe), "tests/cxx/plan_test missing: run __graft_entry__.build()"
