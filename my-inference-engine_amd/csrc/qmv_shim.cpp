@@ -18,6 +18,7 @@
  */
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cstdarg>
 #include <cstdint>
@@ -1412,7 +1413,8 @@ struct WorkspaceNeed {
 };
 
 /* The workspace that decides whether the no-allocation entry point accepts a
- * launch (what it takes does not depend on the kernel that runs it): up to 8
+ * launch, and that an eager launch leaves for later captures (neither depends
+ * on the kernel that runs it): up to 8
  * positions that of the matvec kernels; past 8, the partial sums of 16 or 32
  * position rows over K in splits of 1, 2 or 5 units by the tensors' groups of
  * four tiles (a forced plan's units per wave). */
@@ -1499,7 +1501,10 @@ int enqueue_chunk(const ChunkPlan &cp, hipStream_t stream)
  * to grow it during a capture is made within what there is, if it can be:
  * with fewer segments, or in pieces (so its bits may not be those of the
  * eager launch). Short rows need no workspace on any path but this kernel's
- * fastest, so a stream that never ran them can capture them. */
+ * fastest, so a stream that never ran them can capture them. An eager one
+ * leaves the workspace at least as large as workspace_rule says, so that a
+ * launch on the matvec kernels can be captured after a chunk_kernel launch of
+ * the same tensors (a decode step after a prompt), whichever kernels ran. */
 int launch_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0, int batch,
                  float *const *d_out, hipStream_t stream, Workspace &ws, const Epilogue &epi)
 {
@@ -1513,18 +1518,26 @@ int launch_chunk(QmvDeviceTensor *const *ts, int count, const float *d_in, int b
             cut = Cut();
     }
     std::lock_guard<std::mutex> lock(ws.mu);
-    if (cp.batch && cp.partials > ws.partial_cap) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone &&
-            !cut_within(ts, count, d_in, batch, d_out, epi, ws.partial_cap, ws.counter_cap, &cut))
-            cut = Cut();
+    WorkspaceNeed least; /* what the workspace holds after the call, at least */
+    if (cp.batch) {
+        least = workspace_rule(ts, count, d_in, batch, d_out, epi);
+        if (cp.partials > ws.partial_cap || least.partials > ws.partial_cap || least.counters > ws.counter_cap) {
+            hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+            if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
+                least = WorkspaceNeed();
+                if (cp.partials > ws.partial_cap &&
+                    !cut_within(ts, count, d_in, batch, d_out, epi, ws.partial_cap, ws.counter_cap, &cut))
+                    cut = Cut();
+            }
+        }
     }
     for (int i = 0; i < cut.pieces; ++i) {
         const int nb = piece_positions(batch, cut.pieces, i);
         if ((cut.pieces > 1 || cut.room != SIZE_MAX) &&
             !plan_chunk(ts, count, d_in, b0, nb, d_out, epi, &cp, cut.room))
             return 0;
-        if (!workspace_reserve(ws, stream, cp.partials, cp.counters)) return 0;
+        if (!workspace_reserve(ws, stream, std::max(cp.partials, least.partials), std::max(cp.counters, least.counters)))
+            return 0;
         bind_workspace(cp, ws.partials, ws.counters);
         if (cp.argmax_tiles) {
             if (!workspace_fused_argmax(ws, stream, cp.argmax_tiles)) return 0;
@@ -1708,8 +1721,9 @@ QMV_API int qmv_reserve_calls(const QmvTensorView *matrix, int max_batch)
         if (nb > QMV_VALU_MAX_POSITIONS && !use_prefill(tp->geo.format, nb)) continue;
         ChunkPlan cp;
         if (!plan_chunk(&tp, 1, &dummy, 0, nb, &out, Epilogue(), &cp)) return 0;
-        if (cp.partials > need.partials) need.partials = cp.partials;
-        if (cp.counters > need.counters) need.counters = cp.counters;
+        const WorkspaceNeed rule = workspace_rule(&tp, 1, &dummy, nb, &out, Epilogue());
+        need.partials = std::max({need.partials, cp.partials, rule.partials});
+        need.counters = std::max({need.counters, cp.counters, rule.counters});
     }
     return pool_reserve(need, 1);
 }

@@ -237,3 +237,29 @@ def test_chunk_capture_of_short_rows(qmv, oracle, gpu, hip, t, rows, cols, batch
             _check(oracle, raw, t, rows, cols, ref_x[some], dy.to_array(np.float32, (batch, rows))[some], "replay",
                    scale=2.0 if norm else 1.0)
     dt.close()
+
+
+@pytest.mark.parametrize("t,rows,cols,warm,batch", [(B.Q8_0, 1000, 1280, 8, 1), (B.Q6_K, 1000, 2560, 4, 1),
+                                                    (B.Q5_0, 1000, 1280, 16, 4), (B.Q4_K, 300, 8960, 32, 5)])
+def test_chunk_call_then_capture_of_another_kernel(qmv, oracle, gpu, hip, t, rows, cols, warm, batch):
+    """A call of chunk_kernel, then the first call of the same tensor on a
+    matvec kernel, captured: the stream's workspace holds what it needs."""
+    raw, dt = _tensor(qmv, t, rows, cols, 15)
+    x = qmv.synth_normal(warm * cols, seed=16).reshape(warm, cols)
+    dx, dy = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(4 * warm * rows)
+    with hip.Stream() as s, hip.Graph(s) as g:
+        print(f"chunks: capture after {warm}: {B.NAMES[t]} {rows}x{cols} M={batch}", flush=True)
+        dt.matvec(dx.ptr, warm, dy.ptr, s.handle)
+        s.synchronize()
+        g.begin()
+        dt.matvec(dx.ptr, batch, dy.ptr, s.handle)
+        g.end()
+        for _ in range(3):
+            dy.fill(0)
+            g.replay()
+            s.synchronize()
+            y = dy.to_array(np.float32, (warm, rows))[:batch]
+            _check(oracle, raw, t, rows, cols, x[:batch], y, "replay")
+            dt.matvec(dx.ptr, warm, dy.ptr, s.handle)
+            s.synchronize()
+    dt.close()
