@@ -200,15 +200,10 @@ template <int FMT, int NR> struct BatchStage {
     __device__ static int l_row(int pos) { return F == 1 ? P + pos : pos & 15; }
 };
 
-/* Stage one position's share of a unit: lane i = 0..15 of the position holds
- * v[j] = x[64 j + 4 i ..]. */
-template <int FMT, int NR>
-__device__ __forceinline__ void stage_position(uint8_t *lds, const f4_t (&v)[BatchFmt<FMT>::kUnit / 64], int pos, int i)
+/* The largest magnitude of a position's share of a unit as bits, shifted left
+ * by one: 0xff000000 and up for an infinity or a NaN. */
+template <int NJ> __device__ __forceinline__ uint32_t largest_bits(const f4_t (&v)[NJ])
 {
-    using B = BatchFmt<FMT>;
-    using L = BatchStage<FMT, NR>;
-    constexpr int NJ = B::kUnit / 64;
-    /* the largest magnitude as bits (a NaN counts as the largest) */
     uint32_t mx = 0;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
@@ -217,7 +212,28 @@ __device__ __forceinline__ void stage_position(uint8_t *lds, const f4_t (&v)[Bat
     mx = max(mx, dpp_bits<DPP_XOR1>(mx));
     mx = max(mx, dpp_bits<DPP_XOR2>(mx));
     mx = max(mx, dpp_bits<DPP_HALF_MIRROR>(mx));
-    mx = max(mx, dpp_bits<DPP_ROR8>(mx));
+    return max(mx, dpp_bits<DPP_ROR8>(mx));
+}
+
+/* Stage one position's share of a unit: lane i = 0..15 of the position holds
+ * v[j] = x[64 j + 4 i ..]. Infinities and NaN, which two limbs cannot hold
+ * (inf - inf), are staged as zeros; true if there are any (add_wild adds
+ * them). */
+template <int FMT, int NR>
+__device__ __forceinline__ bool stage_position(uint8_t *lds, f4_t (&v)[BatchFmt<FMT>::kUnit / 64], int pos, int i)
+{
+    using B = BatchFmt<FMT>;
+    using L = BatchStage<FMT, NR>;
+    constexpr int NJ = B::kUnit / 64;
+    uint32_t mx = largest_bits(v);
+    const bool wild = __any(mx >= 0xff000000u);
+    if (wild) { /* the whole wave, which the exchange of maxima needs */
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[j][e] = __builtin_isfinite(v[j][e]) ? v[j][e] : 0.0f;
+        mx = largest_bits(v);
+    }
     /* 2^(14 - its exponent), at most 2^114 (all-zero and tiny units) */
     const int e = 268 - (int)(mx >> 24);
     const int b = e < 241 ? e : 241;
@@ -253,6 +269,7 @@ __device__ __forceinline__ void stage_position(uint8_t *lds, const f4_t (&v)[Bat
             }
         }
     }
+    return wild;
 }
 
 /* ---- a unit's products --------------------------------------------------------------- */
@@ -552,6 +569,43 @@ __device__ __forceinline__ T strided_sum(const S *s, size_t stride, int n)
     return (v[0] + v[1]) + (v[2] + v[3]);
 }
 
+/* Weight i of the row in lane `row` of a tile, in the unit at slab. */
+template <int FMT> __device__ float tiled_weight(const uint8_t *slab, int row, int i)
+{
+    const auto byte = [&](int j) { return (int)slab[(j >> 4) * 1024 + row * 16 + (j & 15)]; }; /* of the 16-byte planes */
+    const auto half = [&](int at) { return half_bits(*(const uint16_t *)(slab + at)); };
+    if constexpr (FMT == QMV_FMT_Q8_0) return half(8 * 1024 + row * 8 + 2 * (i >> 5)) * (float)(int8_t)byte(i);
+    if constexpr (FMT == QMV_FMT_Q5_0) {
+        const int b = i >> 5, j = i & 31, q = byte(16 * b + (j & 15)) >> (j < 16 ? 0 : 4) & 15;
+        const int top = byte(64 + 4 * b + (j >> 3)) >> (j & 7) & 1;
+        return half(5 * 1024 + row * 8 + 2 * b) * (float)((q | top << 4) - 16);
+    }
+    if constexpr (FMT == QMV_FMT_Q6_K) {
+        const int h = i >> 7, k = i >> 5 & 3, l = i & 31;
+        const int q = byte(64 * h + 32 * (k & 1) + l) >> (k < 2 ? 0 : 4) & 15, top = byte(128 + 32 * h + l) >> 2 * k & 3;
+        return half(13 * 1024 + row * 2) * (float)(int8_t)byte(192 + (i >> 4)) * (float)((q | top << 4) - 32);
+    }
+    const int k = i >> 5, q = byte(16 + 32 * (i >> 6) + (i & 31)) >> (k & 1 ? 4 : 0) & 15;
+    const int lo = byte(4 + (k & 3)), mid = byte(8 + (k & 3)), hi = k < 4 ? 0 : byte(8 + k);
+    const int sc = k < 4 ? lo & 63 : (hi & 15) | (lo >> 6) << 4, m = k < 4 ? mid & 63 : hi >> 4 | (mid >> 6) << 4;
+    return __fsub_rn(__fmul_rn(half(row * 16), (float)sc) * (float)q, __fmul_rn(half(row * 16 + 2), (float)m));
+}
+
+/* What infinities and NaN among the activations add to one row: each times
+ * its weight, over the units [u0, u1) of x. */
+template <int FMT>
+__device__ float wild_sum(const float *x, const float *norm_w, int cols, const uint8_t *tile, int row, int u0, int u1)
+{
+    constexpr int kUnit = BatchFmt<FMT>::kUnit;
+    float sum = 0.0f;
+    for (int k = u0 * kUnit; k < u1 * kUnit && k < cols; ++k) {
+        const float v = norm_w ? x[k] * norm_w[k] : x[k];
+        if (!__builtin_isfinite(v))
+            sum += v * tiled_weight<FMT>(tile + (size_t)(k / kUnit) * (64 * BatchFmt<FMT>::kUnitBytes), row, k % kUnit);
+    }
+    return sum;
+}
+
 __device__ __forceinline__ void store_row(const BatchJob &job, int pos, int row, float v)
 {
     if (job.add) v += job.add[(size_t)pos * job.ldadd + row];
@@ -614,6 +668,7 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
     /* Stage the chunk: a wave per unit and round of 4 positions, up to four
      * loads ahead of the first split. */
     const int stages = nu * NR;
+    bool wild = false;
     for (int s0 = wave; s0 < stages; s0 += 4 * nw) {
         f4_t v[4][NJ];
 #pragma unroll
@@ -657,13 +712,21 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
                     if (!FUSED && g0 == 0) p.ssq[(u0 + su) * P + pos] = ssq;
                 }
             }
-            stage_position<FMT, NR>(out, v[q], pos, n);
+            wild |= stage_position<FMT, NR>(out, v[q], pos, n);
         }
     }
+    uint32_t *flags = (uint32_t *)(lds + nu * L::kBytes); /* of each wave: whether it staged infinities or NaN */
+    if (lane == 0) flags[wave] = wild;
     __syncthreads();
 
     const int arow = F == 1 ? (n >> 3) * P + (n & (P - 1)) : n; /* this lane's row of a fragment */
-    float *part = (float *)(lds + nu * L::kBytes); /* FUSED: [segment][row group][position][16] */
+    float *part = (float *)(flags + 16); /* FUSED: [segment][row group][position][16] */
+    /* Where the sums of segment seg and row group g go: of position pos, at pos * ld. */
+    const auto sums = [&](int seg, int g) {
+        return FUSED ? part + ((size_t)seg * p.wg_groups + g) * (P * 16) + n
+                     : p.partials + (size_t)(seg0 + seg) * p.positions * p.groups * 16 + (size_t)(g0 + g) * 16 + n;
+    };
+    const size_t ld = FUSED ? 16 : (size_t)p.groups * 16;
     f4_t y[R][L::kBlocks];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -695,10 +758,7 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int g = set * R + r; /* of the workgroup */
-            float *o = FUSED ? part + ((size_t)seg * p.wg_groups + g) * (P * 16) + n
-                             : p.partials + (size_t)(seg0 + seg) * p.positions * p.groups * 16 +
-                                   (size_t)(g0 + g) * 16 + n;
-            const size_t ld = FUSED ? 16 : (size_t)p.groups * 16;
+            float *o = sums(seg, g);
             const bool real = R == 1 || g < ng;
 #pragma unroll
             for (int f = 0; f < L::kBlocks; ++f)
@@ -714,6 +774,26 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
                 }
 #pragma unroll
             for (int f = 0; f < L::kBlocks; ++f) y[r][f] = f4_t{0, 0, 0, 0};
+        }
+    }
+    if (__any(lane < nw && flags[lane & 15])) { /* rare: the wave's items again, for what was not staged */
+        for (ig = wave / nseg, is = wave % nseg; ig * R < ng;) {
+            open_item();
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int g = ig * R + r;
+                if (g >= ng) break;
+                float *o = sums(is, g);
+                for (int pos = 4 * kc; pos < p.positions; pos += (pos & 3) < 3 ? 1 : 13) /* this lane's */
+                    o[pos * ld] += wild_sum<FMT>(p.x + (size_t)pos * p.cols, NORM ? p.norm_w : nullptr, p.cols, wp[r],
+                                                 wrow[r], u, uend);
+            }
+            is += step_s;
+            ig += step_g;
+            if (is >= nseg) {
+                is -= nseg;
+                ++ig;
+            }
         }
     }
     if constexpr (FUSED) {
@@ -799,7 +879,7 @@ static hipError_t launch_chunks(const BatchParams &p, int waves, hipStream_t s)
     const int most = (p.units + p.segs - 1) / p.segs * p.chunk_segs; /* units of a chunk, at most */
     const size_t units = FUSED ? p.units : most < p.units ? most : p.units;
     const size_t bytes =
-        units * L::kBytes + (FUSED ? ((size_t)p.segs * p.wg_groups * L::P * 16 + L::P) * sizeof(float) : 0);
+        units * L::kBytes + 64 + (FUSED ? ((size_t)p.segs * p.wg_groups * L::P * 16 + L::P) * sizeof(float) : 0);
     if (bytes > 160 * 1024) return hipErrorInvalidValue;
     const int chunks = FUSED ? 1 : (p.segs + p.chunk_segs - 1) / p.chunk_segs;
     chunk_kernel<FMT, NR, R, WAVES, NORM, FUSED><<<chunks * p.chunk_wgs, waves * 64, bytes, s>>>(p);

@@ -263,3 +263,44 @@ def test_chunk_call_then_capture_of_another_kernel(qmv, oracle, gpu, hip, t, row
             dt.matvec(dx.ptr, warm, dy.ptr, s.handle)
             s.synchronize()
     dt.close()
+
+
+def _class(a):
+    """+inf, -inf, NaN or finite, as numbers"""
+    return np.where(np.isnan(a), 3, np.where(np.isinf(a), np.sign(np.where(np.isinf(a), a, 0)), 0))
+
+
+@pytest.mark.parametrize("t", B.ALL_TYPES)
+@pytest.mark.parametrize("rows,cols,batch", [(96, 1024, 2), (33, 1024, 4), (96, 512, 7), (70, 1024, 8), (48, 1024, 11),
+                                             (96, 5120, 16), (40, 8960, 21), (600, 1024, 32)])
+def test_chunk_infinities(qmv, oracle, gpu, hip, t, rows, cols, batch):
+    """An infinity gives the rows of its position the infinity of its
+    weight's sign (NaN where the weight is 0), as the reference's sum does;
+    two may cancel to NaN; a NaN stays NaN; the other positions keep their
+    bits, and nothing past the outputs is written."""
+    raw, dt = _tensor(qmv, t, rows, cols, 31)
+    x = qmv.synth_normal(batch * cols, seed=32).reshape(batch, cols)
+    bad = x.copy()
+    bad[0, cols // 3] = np.inf
+    bad[1, cols - 1] = -np.inf
+    if batch > 3:
+        bad[2, [0, cols // 2]] = np.inf
+        bad[batch - 1, 7] = np.nan
+    with hip.Stream() as s:
+        print(f"chunks: infinities {B.NAMES[t]} {rows}x{cols} M={batch}", flush=True)
+        ys = []
+        for v in (x, bad):
+            dx, dy = hip.DeviceBuffer.from_array(v), hip.DeviceBuffer(4 * (batch * rows + 64))
+            dy.fill(0x7F)
+            dt.matvec(dx.ptr, batch, dy.ptr, s.handle)
+            s.synchronize()
+            y = dy.to_array(np.float32, (batch * rows + 64,))
+            assert np.all(_bits(y[batch * rows:]) == 0x7F7F7F7F)
+            ys.append(y[:batch * rows].reshape(batch, rows))
+    for b in range(batch):
+        if np.isfinite(bad[b]).all():
+            assert np.array_equal(_bits(ys[1][b]), _bits(ys[0][b])), b
+        else:
+            ref = oracle.matvec(raw, t, rows, cols, bad[b])
+            assert np.array_equal(_class(ys[1][b]), _class(ref)), b
+    dt.close()
