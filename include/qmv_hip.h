@@ -170,7 +170,9 @@ int qmv_device_tensor_info(qmv_device_tensor tensor, int *rows, int *columns,
  * d_outputs[B,N] = d_inputs[B,K] * W^T with device pointers, enqueued on
  * stream without host synchronisation (1 <= batch_count <= QMV_MAX_BATCH).
  * Batches of 9 to 32 positions (prefill chunks larger than the reference's
- * 8, src/qwen2_internal.h:7) read the weights once, on the matrix cores.
+ * 8, src/qwen2_internal.h:7) read the weights once, on the matrix cores. There
+ * an activation is held to 2^-23 of itself, or, more than 2^28 below the largest
+ * of its 256 (Q8_0, Q5_0: 128) neighbours in K, to 2^-51 of that one.
  * Under graph capture a launch that would have to grow the stream's workspace
  * is made within the workspace there is, where it can be (rows of a few
  * K-units need none), and fails otherwise: run the call once before it is

@@ -19,9 +19,16 @@
  * Activations. x of one position and unit is scaled by the power of two that
  * brings the largest magnitude to [2^14, 2^15) and split into two f16 limbs,
  * xs = h + l * 2^-12 with h = f16(xs) and l = f16((xs - h) * 2^12). The two
- * limbs are summed apart, so l's range reaches 2^-36: every activation within
- * 2^28 of its unit's largest is held to its own 2^-24, as a float is. Below,
- * the error is at most 2^-51 of the largest.
+ * limbs are summed apart, so l's range reaches 2^-36. That is one bit less
+ * than a float: what h leaves takes up to 12 bits and l has 11, so a quarter of
+ * all floats lose their last place. An activation within 2^28 of its unit's
+ * largest is held to 2^-23 of itself; below, the error is at most 2^-51 of the
+ * largest. The matvec kernels multiply the float, or three bf16 limbs that are
+ * exact; the sums are still nearer to 64 bits here, because fewer roundings
+ * follow (7B layers, relative 2-norm, matvec and prefill kernels / this: 4
+ * positions 4.4e-7 / 3.3e-7, 13 4.6e-7 / 3.1e-7, 32 4.6e-7 / 3.1e-7; Q6_K
+ * vocabulary at 4 2.1e-7 / 1.2e-7). Q4_K's sums of x are two limbs as well.
+ * Infinities and NaN are not staged: wild_sum adds them.
  *
  * Weights. An integer in the low bits of an f16 is a subnormal, so a mask and
  * one packed multiply-add with a sub-block's integer scale make exact f16
@@ -217,8 +224,8 @@ template <int NJ> __device__ __forceinline__ uint32_t largest_bits(const f4_t (&
 
 /* Stage one position's share of a unit: lane i = 0..15 of the position holds
  * v[j] = x[64 j + 4 i ..]. Infinities and NaN, which two limbs cannot hold
- * (inf - inf), are staged as zeros; true if there are any (add_wild adds
- * them). */
+ * (inf - inf), are staged as zeros; true if there are any (wild_sum has what
+ * they add). */
 template <int FMT, int NR>
 __device__ __forceinline__ bool stage_position(uint8_t *lds, f4_t (&v)[BatchFmt<FMT>::kUnit / 64], int pos, int i)
 {

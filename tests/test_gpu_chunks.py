@@ -6,9 +6,9 @@ in chunks, partial 128-weight units.
 
 Bar: every row of every position within 1e-5 * sum |w x| of the oracle, the
 bar of every product here. The kernel's activations are two f16 limbs under a
-power of two per position and unit, exact to 2^-24 of each value within 2^28
-of the unit's largest, so a value 2^26 below its unit's largest must count
-as fully as on the VALU kernels."""
+power of two per position and unit, within 2^-23 of each value that is within
+2^28 of the unit's largest, so a value 2^26 below its unit's largest must
+count as on the VALU kernels."""
 import numpy as np
 import pytest
 
@@ -63,6 +63,40 @@ def test_chunk_edges(qmv, oracle, gpu, hip, t, rows, batch):
             assert np.all(_bits(y[batch * rows:]) == 0x7F7F7F7F)
             _check(oracle, raw, t, rows, cols, x, y[:batch * rows].reshape(batch, rows), f"K={cols}")
             dt.close()
+
+
+@pytest.mark.parametrize("t,one", [(B.Q8_0, 1), (B.Q5_0, 17)])
+@pytest.mark.parametrize("batch", [2, 8, 24])
+def test_chunk_holds_activations(qmv, gpu, hip, t, one, batch):
+    """Row r has the weight 1 at column r and zeros, whose products are exact,
+    so the outputs are the activations as the limbs hold them: within 2^-23 of
+    the value down to 2^-28 of its unit's largest, else within 2^-51 of that."""
+    n = 128
+    w = np.zeros((n, n // 32, B.BLOCK_BYTES[t]), np.uint8)
+    w[:, :, 1] = 0x3C  # f16 1.0
+    for r in range(n):
+        if t == B.Q8_0:
+            w[r, r // 32, 2 + r % 32] = one
+        else:  # codes of 16, and one of 17
+            w[r, :, 2:6] = 0xFF
+            w[r, r // 32, 6 + r % 16] = (one & 15) << (4 * (r % 32 // 16))
+    dt = qmv.DeviceTensor(qmv.make_view(np.ascontiguousarray(w.reshape(-1)), t, n, n))
+    rng = np.random.default_rng(batch)
+    x = (rng.uniform(1, 2, (batch, n)) * rng.choice([-1, 1], (batch, n))).astype(np.float32)
+    x[0] *= np.float32(2.0) ** rng.integers(-60, 60, n).astype(np.float32)
+    x[1] *= np.float32(2.0) ** rng.integers(-25, 1, n).astype(np.float32)
+    x[1, 5] = 2.0 ** -120  # far below the rest
+    with hip.Stream() as s:
+        dx, dy = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(4 * batch * n)
+        print(f"chunks: activations held {B.NAMES[t]} M={batch}", flush=True)
+        dt.matvec(dx.ptr, batch, dy.ptr, s.handle)
+        s.synchronize()
+        y = dy.to_array(np.float32, (batch, n)).astype(np.float64)
+    v = x.astype(np.float64)
+    largest = np.abs(v).max(1, keepdims=True)
+    err = np.abs(y - v)
+    assert (err <= np.where(np.abs(v) >= largest * 2.0 ** -28, np.abs(v) * 2.0 ** -23, largest * 2.0 ** -51)).all()
+    dt.close()
 
 
 @pytest.mark.parametrize("t", B.ALL_TYPES)
