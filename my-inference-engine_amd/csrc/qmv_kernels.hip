@@ -1893,8 +1893,9 @@ dequant_kernel(const uint8_t *__restrict__ w, float *__restrict__ out, int rows,
  * sit at lane id % 64 of its slab. An id outside [0, rows) fills its output
  * row with NaN (ids live in device memory, so the host cannot check them);
  * status[0], when given, is written by the first workgroup, which looks at
- * every id (1 if all are in range, else 0: the caller can fail as the
- * reference does for such a token), so no launch sets it beforehand. 32 rows of
+ * every id, eight loads in flight a thread (1 if all are in range, else 0: the
+ * caller can fail as the reference does for such a token), so no launch sets
+ * it beforehand. 32 rows of
  * 151936 x 3584 Q6_K: 6.4 us a call in a row of calls, 9.5 with a wave per
  * unit and a launch that set the status first. */
 /* Part Q of QMV_GATHER_PARTS of a unit's regions. */
@@ -1927,11 +1928,25 @@ gather_rows_kernel(const uint8_t *__restrict__ w, const int *__restrict__ ids, i
     constexpr int SLAB = UnitOf<FMT>::kBytes * 64;
     constexpr int UW = UnitOf<FMT>::kWeights;
     const int lane = threadIdx.x & 63, part = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    if (status != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && part == 0) {
-        int bad = 0;
-        for (int k = lane; k < count; k += 64) bad |= ids[k] < 0 || ids[k] >= rows;
+    if (status != nullptr && blockIdx.x == 0 && blockIdx.y == 0) {
+        __shared__ int waves_bad[QMV_GATHER_PARTS];
+        constexpr int kThreads = 64 * QMV_GATHER_PARTS, kAhead = 8;
+        bool bad = false;
+        for (int k = threadIdx.x; k < count; k += kThreads * kAhead) {
+            int v[kAhead];
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) v[j] = ids[min(k + j * kThreads, count - 1)];
+#pragma unroll
+            for (int j = 0; j < kAhead; ++j) bad |= v[j] < 0 || v[j] >= rows;
+        }
         const bool any = __any(bad);
-        if (lane == 0) status[0] = any ? 0 : 1;
+        if (lane == 0) waves_bad[part] = any;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int all = 0;
+            for (int j = 0; j < QMV_GATHER_PARTS; ++j) all |= waves_bad[j];
+            status[0] = all ? 0 : 1;
+        }
     }
     const int i = blockIdx.y;
     const int unit = blockIdx.x * 64 + lane;

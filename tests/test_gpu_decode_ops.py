@@ -533,3 +533,25 @@ def test_concurrent_streams_share_weights(qmv, gpu, hip):
     assert not errors, errors
     for d in (dg, du, dd):
         d.close()
+
+
+@pytest.mark.parametrize("count", [1, 255, 256, 2049, 65535])
+def test_embed_status_of_many_ids(qmv, gpu, hip, count):
+    """The status looks at every id: one bad id anywhere clears it (the first,
+    the last, at the edges of a thread's loads), none leaves it at 1."""
+    t, rows, cols = B.Q8_0, 70, 64
+    raw, dt = _tensor(qmv, t, rows, cols, seed=3)
+    ids = (np.arange(count) * 7 % rows).astype(np.int32)
+    with hip.Stream() as s:
+        dy, ds = hip.DeviceBuffer(4 * count * cols), hip.DeviceBuffer(4)
+        print(f"embed status {count}", flush=True)
+        for at in (None, *sorted({0, count // 2, min(255, count - 1), max(0, count - 256), count - 1})):
+            bad = ids.copy()
+            if at is not None:
+                bad[at] = rows if at % 2 else -1
+            di = hip.DeviceBuffer.from_array(bad)
+            ds.fill(0x55)
+            qmv.device_embed_rows(dt, di.ptr, count, dy.ptr, s.handle, ds.ptr)
+            s.synchronize()
+            assert ds.to_array(np.int32, (1,))[0] == (at is None), at
+    dt.close()
