@@ -1887,9 +1887,11 @@ dequant_kernel(const uint8_t *__restrict__ w, float *__restrict__ out, int rows,
 /* ---- embedding-row gather -----------------------------------------------------
  * out[i * cols + k] = row ids[i] of the tensor, decoded exactly like
  * dequant_kernel (bit-identical to the block decoders). One lane per
- * (position i, K-unit), a quarter of the unit per wave: a row has few units
- * (14 at K = 3584), so a launch is bound by one lane's chain of loads, decodes
- * and stores, and by what the launch itself costs. The row's bytes of a unit
+ * (position i, K-unit), in launches of few rows a quarter of the unit per
+ * wave (PARTS): a row has few units (14 at K = 3584), so such a launch is bound
+ * by one lane's chain of loads, decodes and stores, and by what the launch
+ * itself costs; one of many rows by its stores, which a whole unit per lane
+ * serves better (gather_split). The row's bytes of a unit
  * sit at lane id % 64 of its slab. An id outside [0, rows) fills its output
  * row with NaN (ids live in device memory, so the host cannot check them);
  * status[0], when given, is written by the first workgroup, which looks at
@@ -1898,13 +1900,13 @@ dequant_kernel(const uint8_t *__restrict__ w, float *__restrict__ out, int rows,
  * it beforehand. 32 rows of
  * 151936 x 3584 Q6_K: 6.4 us a call in a row of calls, 9.5 with a wave per
  * unit and a launch that set the status first. */
-/* Part Q of QMV_GATHER_PARTS of a unit's regions. */
+/* Part Q of PARTS of a unit's regions. */
 #define QMV_GATHER_PARTS 4
-template <int FMT, int Q>
+template <int FMT, int PARTS, int Q>
 __device__ __forceinline__ void gather_part(const uint8_t *slab, int lane_row, float *dst, int kleft)
 {
-    constexpr int UW = UnitOf<FMT>::kWeights, N = RegionCount<FMT>::value / QMV_GATHER_PARTS;
-    static_assert(RegionCount<FMT>::value % QMV_GATHER_PARTS == 0, "whole regions");
+    constexpr int UW = UnitOf<FMT>::kWeights, N = RegionCount<FMT>::value / PARTS;
+    static_assert(RegionCount<FMT>::value % PARTS == 0, "whole regions");
     typename UnitOf<FMT>::T u;
     load_unit(u, slab, lane_row);
     const UnitScales<FMT> s = unit_scales<FMT>(u);
@@ -1920,8 +1922,8 @@ __device__ __forceinline__ void gather_part(const uint8_t *slab, int lane_row, f
     }
 }
 
-template <int FMT>
-__global__ void __launch_bounds__(64 * QMV_GATHER_PARTS)
+template <int FMT, int PARTS>
+__global__ void __launch_bounds__(64 * PARTS)
 gather_rows_kernel(const uint8_t *__restrict__ w, const int *__restrict__ ids, int count, float *__restrict__ out,
                    int rows, int cols, int units, int *__restrict__ status)
 {
@@ -1929,8 +1931,8 @@ gather_rows_kernel(const uint8_t *__restrict__ w, const int *__restrict__ ids, i
     constexpr int UW = UnitOf<FMT>::kWeights;
     const int lane = threadIdx.x & 63, part = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     if (status != nullptr && blockIdx.x == 0 && blockIdx.y == 0) {
-        __shared__ int waves_bad[QMV_GATHER_PARTS];
-        constexpr int kThreads = 64 * QMV_GATHER_PARTS, kAhead = 8;
+        __shared__ int waves_bad[PARTS];
+        constexpr int kThreads = 64 * PARTS, kAhead = 8;
         bool bad = false;
         for (int k = threadIdx.x; k < count; k += kThreads * kAhead) {
             int v[kAhead];
@@ -1944,7 +1946,7 @@ gather_rows_kernel(const uint8_t *__restrict__ w, const int *__restrict__ ids, i
         __syncthreads();
         if (threadIdx.x == 0) {
             int all = 0;
-            for (int j = 0; j < QMV_GATHER_PARTS; ++j) all |= waves_bad[j];
+            for (int j = 0; j < PARTS; ++j) all |= waves_bad[j];
             status[0] = all ? 0 : 1;
         }
     }
@@ -1955,16 +1957,20 @@ gather_rows_kernel(const uint8_t *__restrict__ w, const int *__restrict__ ids, i
     float *dst = out + (size_t)i * cols + (size_t)unit * UW;
     const int kleft = cols - unit * UW;
     if (id < 0 || id >= rows) {
-        for (int k = part * (UW / QMV_GATHER_PARTS); k < (part + 1) * (UW / QMV_GATHER_PARTS) && k < kleft; ++k)
+        for (int k = part * (UW / PARTS); k < (part + 1) * (UW / PARTS) && k < kleft; ++k)
             dst[k] = __builtin_nanf("");
         return;
     }
     const uint8_t *slab = w + ((size_t)(id >> 6) * units + unit) * SLAB;
-    switch (part) { /* the same in every lane of a wave */
-    case 0: gather_part<FMT, 0>(slab, id & 63, dst, kleft); break;
-    case 1: gather_part<FMT, 1>(slab, id & 63, dst, kleft); break;
-    case 2: gather_part<FMT, 2>(slab, id & 63, dst, kleft); break;
-    default: gather_part<FMT, 3>(slab, id & 63, dst, kleft); break;
+    if constexpr (PARTS == 1) {
+        gather_part<FMT, 1, 0>(slab, id & 63, dst, kleft);
+    } else {
+        switch (part) { /* the same in every lane of a wave */
+        case 0: gather_part<FMT, PARTS, 0>(slab, id & 63, dst, kleft); break;
+        case 1: gather_part<FMT, PARTS, 1>(slab, id & 63, dst, kleft); break;
+        case 2: gather_part<FMT, PARTS, 2>(slab, id & 63, dst, kleft); break;
+        default: gather_part<FMT, PARTS, 3>(slab, id & 63, dst, kleft); break;
+        }
     }
 }
 
@@ -2990,19 +2996,39 @@ hipError_t launch_dequant(int fmt, const uint8_t *w, float *out, int rows, int c
     return hipGetLastError();
 }
 
+/* Whether a unit's rows are split over four waves: in launches that do not fill
+ * the chip with a wave a unit. Us, a wave / four: Q6_K at K = 3584 512 rows
+ * 8.3 / 7.2, 1024 10.1 / 12.5, 16384 168 / 195; Q4_K at K = 1536 2048 rows 10.8
+ * / 10.1, 4096 17.3 / 17.4, 16384 48.4 / 55.6; Q8_0 and Q5_0 (units of 128) four
+ * are up to 1.8 times as fast and within 1% at 65535 rows. */
+static bool gather_split(int fmt, double elements)
+{
+    return fmt == QMV_FMT_Q6_K ? elements <= 2.5e6 : fmt != QMV_FMT_Q4_K || elements <= 6e6;
+}
+
+#define QMV_GATHER(FMT, PARTS)                                                                                       \
+    gather_rows_kernel<FMT, PARTS><<<dim3((units + 63) / 64, count), 64 * PARTS, 0, s>>>(w, ids, count, out, rows, cols, \
+                                                                                       units, status)
 hipError_t launch_gather(int fmt, const uint8_t *w, const int *ids, int count, float *out, int rows, int cols,
                          int units, int *status, hipStream_t s)
 {
-    const dim3 grid((units + 63) / 64, count);
+    const bool split = gather_split(fmt, (double)count * cols);
     switch (fmt) {
-    case QMV_FMT_Q4_K: hipLaunchKernelGGL(gather_rows_kernel<QMV_FMT_Q4_K>, grid, dim3(64 * QMV_GATHER_PARTS), 0, s, w, ids, count, out, rows, cols, units, status); break;
-    case QMV_FMT_Q6_K: hipLaunchKernelGGL(gather_rows_kernel<QMV_FMT_Q6_K>, grid, dim3(64 * QMV_GATHER_PARTS), 0, s, w, ids, count, out, rows, cols, units, status); break;
-    case QMV_FMT_Q8_0: hipLaunchKernelGGL(gather_rows_kernel<QMV_FMT_Q8_0>, grid, dim3(64 * QMV_GATHER_PARTS), 0, s, w, ids, count, out, rows, cols, units, status); break;
-    case QMV_FMT_Q5_0: hipLaunchKernelGGL(gather_rows_kernel<QMV_FMT_Q5_0>, grid, dim3(64 * QMV_GATHER_PARTS), 0, s, w, ids, count, out, rows, cols, units, status); break;
+    case QMV_FMT_Q4_K:
+        if (split) QMV_GATHER(QMV_FMT_Q4_K, QMV_GATHER_PARTS);
+        else QMV_GATHER(QMV_FMT_Q4_K, 1);
+        break;
+    case QMV_FMT_Q6_K:
+        if (split) QMV_GATHER(QMV_FMT_Q6_K, QMV_GATHER_PARTS);
+        else QMV_GATHER(QMV_FMT_Q6_K, 1);
+        break;
+    case QMV_FMT_Q8_0: QMV_GATHER(QMV_FMT_Q8_0, QMV_GATHER_PARTS); break;
+    case QMV_FMT_Q5_0: QMV_GATHER(QMV_FMT_Q5_0, QMV_GATHER_PARTS); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
+#undef QMV_GATHER
 
 hipError_t launch_repack(int fmt, const uint8_t *raw, uint8_t *out, int rows, int blocks_per_row,
                          int units, int blocks_per_unit, int block_bytes, int unit_bytes, int tiles,

@@ -555,3 +555,25 @@ def test_embed_status_of_many_ids(qmv, gpu, hip, count):
             s.synchronize()
             assert ds.to_array(np.int32, (1,))[0] == (at is None), at
     dt.close()
+
+
+@pytest.mark.parametrize("t,cols,counts", [(B.Q6_K, 512, (4882, 4883)), (B.Q4_K, 768, (7812, 7813))])
+def test_embed_rows_at_the_split(qmv, oracle, gpu, hip, t, cols, counts):
+    """Launches on both sides of the size from which a unit is one lane's, bit
+    for bit the decoded rows, with an id out of range."""
+    rows = 300
+    raw, dt = _tensor(qmv, t, rows, cols, seed=5)
+    want = oracle.dequantize_rows(raw, t, rows, cols, 0, rows)
+    with hip.Stream() as s:
+        for count in counts:
+            ids = (np.arange(count) * 7 % rows).astype(np.int32)
+            ids[count - 2] = rows
+            di, dy, ds = hip.DeviceBuffer.from_array(ids), hip.DeviceBuffer(4 * count * cols), hip.DeviceBuffer(4)
+            print(f"embed {B.NAMES[t]} {count}", flush=True)
+            qmv.device_embed_rows(dt, di.ptr, count, dy.ptr, s.handle, ds.ptr)
+            s.synchronize()
+            y = dy.to_array(np.float32, (count, cols))
+            good = ids < rows
+            assert np.array_equal(_bits(y[good]), _bits(want.reshape(rows, cols)[ids[good]]))
+            assert np.isnan(y[~good]).all() and ds.to_array(np.int32, (1,))[0] == 0
+    dt.close()
