@@ -290,8 +290,8 @@ Workspace &workspace_for(int device, hipStream_t stream)
 
 struct CtxPool;
 
-/* Launches of a host call whose results may wait to be copied out. */
-constexpr int kPasses = 4;
+/* Parts in which a host call of several launches copies its output out. */
+constexpr int kPasses = 16;
 
 struct HostCtx {
     int device = -1;
@@ -302,7 +302,7 @@ struct HostCtx {
     size_t h_in_cap = 0, h_out_cap = 0;
     float *d_in = nullptr, *d_out = nullptr; /* d_out: dequantised rows, sampler results */
     size_t d_in_cap = 0, d_out_cap = 0;
-    hipEvent_t passed[kPasses] = {}; /* the end of a call's launches, in turn */
+    hipEvent_t passed[kPasses] = {}; /* the ends of a call's parts */
     bool busy = false; /* checked out; guarded by the pool's mutex */
 };
 
@@ -1620,7 +1620,8 @@ int host_matmul(const QmvTensorView *m, const float *in, int in_count, int batch
     };
     /* Calls of several launches and 1 MB or more: a launch's input is copied
      * to the pinned buffer and its kernels enqueued while the one before it
-     * runs, and its output is copied out while the next ones run. 77
+     * runs; once all are enqueued (a launch that fails leaves the output
+     * untouched), outputs are copied out while later launches run. 77
      * positions of 8960 x 1536 Q4_K: 154 us against 212 with both host copies
      * outside, around all launches; below 1 MB the events cost what the
      * overlap gains (90 positions of 500 x 1024 Q5_0, 0.5 MB: 74-80 us against
@@ -1634,27 +1635,25 @@ int host_matmul(const QmvTensorView *m, const float *in, int in_count, int batch
         HIP_TRY(hipStreamSynchronize(c->stream));
         download(0, batch);
     } else {
-        struct Pass {
-            int b0, count;
-        } waiting[kPasses];
-        int made = 0, taken = 0;
-        const auto take = [&]() {
-            const int slot = taken++ % kPasses;
-            HIP_TRY(hipEventSynchronize(c->passed[slot]));
-            download(waiting[slot].b0, waiting[slot].count);
-            return 1;
-        };
-        for (int b0 = 0; b0 < batch;) {
-            if (made - taken == kPasses && !take()) return 0;
+        int launches = 0;
+        for (int b0 = 0; b0 < batch; ++launches) b0 += next_chunk(tp->geo.format, batch, b0);
+        const int passes = launches < kPasses ? launches : kPasses;
+        int ends[kPasses]; /* the positions done when passed[i] is */
+        for (int i = 0, b0 = 0, made = 0; i < launches; ++i) {
             const int nb = next_chunk(tp->geo.format, batch, b0);
             if (!upload((size_t)b0 * (size_t)in_count, (size_t)nb * (size_t)in_count)) return 0;
             if (!launch_chunk(&tp, 1, c->d_in, b0, nb, &hout, c->stream, *c->ws, Epilogue())) return 0;
-            HIP_TRY(hipEventRecord(c->passed[made % kPasses], c->stream));
-            waiting[made++ % kPasses] = Pass{b0, nb};
             b0 += nb;
+            if ((i + 1) * passes >= (made + 1) * launches) {
+                HIP_TRY(hipEventRecord(c->passed[made], c->stream));
+                ends[made++] = b0;
+            }
         }
-        while (taken < made)
-            if (!take()) return 0;
+        for (int i = 0; i < passes; ++i) {
+            HIP_TRY(hipEventSynchronize(c->passed[i]));
+            const int begin = i ? ends[i - 1] : 0;
+            download(begin, ends[i] - begin);
+        }
     }
     lease.done = true; /* the stream's last launch has ended */
     if (armed > 0) {

@@ -222,10 +222,12 @@ def test_chunk_output_over_norm_weights(qmv, oracle, gpu, hip):
     dt.close()
 
 
-@pytest.mark.parametrize("t,rows,cols,batch", [(B.Q4_K, 4000, 1024, 170), (B.Q8_0, 3000, 512, 77)])
+@pytest.mark.parametrize("t,rows,cols,batch", [(B.Q4_K, 4000, 1024, 170), (B.Q8_0, 3000, 512, 77),
+                                               (B.Q8_0, 900, 256, 550)])
 def test_host_calls_of_several_launches(qmv, oracle, gpu, hip, t, rows, cols, batch):
-    """A host call of more launches than may wait at once (170 positions: 6)
-    and one of three, whose inputs and outputs are copied while launches run:
+    """A host call of more launches than parts in which it is copied out (550
+    positions: 18), one of 6 and one of three, whose inputs and outputs are
+    copied while launches run:
     the bits of the same positions in calls of one launch each; an input
     inside the output's memory is read before it is overwritten."""
     raw = qmv.synth_tensor(t, rows, cols, seed=21)

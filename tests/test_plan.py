@@ -1,6 +1,6 @@
-"""The launch planner over many shapes without a GPU (tests/cxx/plan_test.cpp,
-the host shim's source compiled into a program that plans and launches
-nothing)."""
+"""The host shim without a GPU: its source is compiled into programs that plan
+and launch nothing (tests/cxx/plan_test.cpp: the launch planner over many
+shapes; host_call_test.cpp: host-pointer calls whose launches fail)."""
 import os
 import subprocess
 
@@ -9,9 +9,17 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
+def _run(*command):
+    exe = os.path.join(ROOT, "tests", "cxx", command[0])
+    assert os.path.exists(exe), f"tests/cxx/{command[0]} missing: run __graft_entry__.build()"
+    r = subprocess.run([exe, *command[1:]], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-1000:]
+
+
 @pytest.mark.parametrize("what", ["scratch", "capture"])
 def test_plans(what):
-    exe = os.path.join(ROOT, "tests", "cxx", "plan_test")
-    assert os.path.exists(exe), "tests/cxx/plan_test missing: run __graft_entry__.build()"
-    r = subprocess.run([exe, what], capture_output=True, text=True, timeout=120)
-    assert r.returncode == 0, r.stdout[-4000:] + r.stderr[-1000:]
+    _run("plan_test", what)
+
+
+def test_host_call_that_fails_writes_nothing():
+    _run("host_call_test")
