@@ -340,3 +340,45 @@ def test_chunk_infinities(qmv, oracle, gpu, hip, t, rows, cols, batch):
             ref = oracle.matvec(raw, t, rows, cols, bad[b])
             assert np.array_equal(_class(ys[1][b]), _class(ref)), b
     dt.close()
+
+
+@pytest.mark.parametrize("t", [B.Q4_K, B.Q6_K])
+@pytest.mark.parametrize("batch", [2, 7, 16, 32])
+def test_chunk_subnormal_operands(qmv, oracle, gpu, hip, t, batch):
+    """Sub-block scales of 1 (Q6_K: and -1) and codes next to the centre, whose
+    matrix operands are f16 subnormals: they count in full. Against 64 bits
+    (measured 6e-8 to 8e-8; the bar is the rounding of an fp32 sum, and operands
+    taken as zero would be off by more than 0.1)."""
+    rows, cols = 64, 1024
+    rng = np.random.default_rng(batch)
+    raw = qmv.synth_tensor(t, rows, cols, seed=9).reshape(rows, cols // 256, -1).copy()
+    if t == B.Q4_K:  # scales 1, minimums 0; codes 7, 8, 9
+        raw[:, :, 2:4] = 0
+        raw[:, :, 4:16] = 0
+        raw[:, :, 4:8] = 1
+        raw[:, :, 12:16] = 1
+        q = rng.integers(7, 10, (2, rows, cols // 256, 128))
+        raw[:, :, 16:] = q[0] | q[1] << 4
+    else:  # scales 1 and -1; low nibbles 5 .. 11
+        raw[:, :, 192:208] = rng.choice([1, 255], (rows, cols // 256, 16))
+        q = rng.integers(5, 12, (2, rows, cols // 256, 128))
+        raw[:, :, :128] = q[0] | q[1] << 4
+    raw = np.ascontiguousarray(raw.reshape(-1))
+    dt = qmv.DeviceTensor(qmv.make_view(raw, t, rows, cols))
+    w = oracle.dequantize_rows(raw, t, rows, cols, 0, rows).reshape(rows, cols).astype(np.float64)
+    if t == B.Q4_K:  # pairs that cancel: the 8 of every code adds nothing
+        x = rng.standard_normal((batch, cols)).astype(np.float32)
+        x[:, 1::2] = -x[:, ::2]
+    else:
+        x = rng.standard_normal((batch, cols)).astype(np.float32)
+    ref = x.astype(np.float64) @ w.T
+    with hip.Stream() as s:
+        dx, dy = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(4 * batch * rows)
+        print(f"chunks: subnormal operands {B.NAMES[t]} M={batch}", flush=True)
+        dt.matvec(dx.ptr, batch, dy.ptr, s.handle)
+        s.synchronize()
+        y = dy.to_array(np.float32, (batch, rows)).astype(np.float64)
+    err = np.linalg.norm(y - ref) / np.linalg.norm(ref)
+    print(f"relative error {err:.2g}", flush=True)
+    assert err <= 3e-7
+    dt.close()
