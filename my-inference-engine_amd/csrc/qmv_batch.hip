@@ -28,7 +28,8 @@
  * follow (7B layers, relative 2-norm, matvec and prefill kernels / this: 4
  * positions 4.4e-7 / 3.3e-7, 13 4.6e-7 / 3.1e-7, 32 4.6e-7 / 3.1e-7; Q6_K
  * vocabulary at 4 2.1e-7 / 1.2e-7). Q4_K's sums of x are two limbs as well.
- * Infinities and NaN are not staged: wild_sum adds them.
+ * Sums of infinities and NaN are taken
+ * again (finish_rows).
  *
  * Weights. An integer in the low bits of an f16 is a subnormal, so a mask and
  * one packed multiply-add with a sub-block's integer scale make exact f16
@@ -51,6 +52,8 @@
  */
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "qmv_kernels.h"
 
@@ -207,10 +210,15 @@ template <int FMT, int NR> struct BatchStage {
     __device__ static int l_row(int pos) { return F == 1 ? P + pos : pos & 15; }
 };
 
-/* The largest magnitude of a position's share of a unit as bits, shifted left
- * by one: 0xff000000 and up for an infinity or a NaN. */
-template <int NJ> __device__ __forceinline__ uint32_t largest_bits(const f4_t (&v)[NJ])
+/* Stage one position's share of a unit: lane i = 0..15 of the position holds
+ * v[j] = x[64 j + 4 i ..]. */
+template <int FMT, int NR>
+__device__ __forceinline__ void stage_position(uint8_t *lds, const f4_t (&v)[BatchFmt<FMT>::kUnit / 64], int pos, int i)
 {
+    using B = BatchFmt<FMT>;
+    using L = BatchStage<FMT, NR>;
+    constexpr int NJ = B::kUnit / 64;
+    /* the largest magnitude as bits (a NaN counts as the largest) */
     uint32_t mx = 0;
 #pragma unroll
     for (int j = 0; j < NJ; ++j)
@@ -219,28 +227,7 @@ template <int NJ> __device__ __forceinline__ uint32_t largest_bits(const f4_t (&
     mx = max(mx, dpp_bits<DPP_XOR1>(mx));
     mx = max(mx, dpp_bits<DPP_XOR2>(mx));
     mx = max(mx, dpp_bits<DPP_HALF_MIRROR>(mx));
-    return max(mx, dpp_bits<DPP_ROR8>(mx));
-}
-
-/* Stage one position's share of a unit: lane i = 0..15 of the position holds
- * v[j] = x[64 j + 4 i ..]. Infinities and NaN, which two limbs cannot hold
- * (inf - inf), are staged as zeros; true if there are any (wild_sum has what
- * they add). */
-template <int FMT, int NR>
-__device__ __forceinline__ bool stage_position(uint8_t *lds, f4_t (&v)[BatchFmt<FMT>::kUnit / 64], int pos, int i)
-{
-    using B = BatchFmt<FMT>;
-    using L = BatchStage<FMT, NR>;
-    constexpr int NJ = B::kUnit / 64;
-    uint32_t mx = largest_bits(v);
-    const bool wild = __any(mx >= 0xff000000u);
-    if (wild) { /* the whole wave, which the exchange of maxima needs */
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[j][e] = __builtin_isfinite(v[j][e]) ? v[j][e] : 0.0f;
-        mx = largest_bits(v);
-    }
+    mx = max(mx, dpp_bits<DPP_ROR8>(mx));
     /* 2^(14 - its exponent), at most 2^114 (all-zero and tiny units) */
     const int e = 268 - (int)(mx >> 24);
     const int b = e < 241 ? e : 241;
@@ -276,7 +263,6 @@ __device__ __forceinline__ bool stage_position(uint8_t *lds, f4_t (&v)[BatchFmt<
             }
         }
     }
-    return wild;
 }
 
 /* ---- a unit's products --------------------------------------------------------------- */
@@ -566,13 +552,18 @@ template <typename T, typename S>
 __device__ __forceinline__ T strided_sum(const S *s, size_t stride, int n)
 {
     T v[4] = {T(0), T(0), T(0), T(0)};
-    for (int i = 0; i < n; i += 8) {
-        T q[8];
+    const auto add = [&](int i, auto count) { /* s[i ..], as many as count */
+        constexpr int N = decltype(count)::value;
+        T q[N];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) q[j] = *(const T *)(s + (i + j < n ? i + j : n - 1) * stride);
+        for (int j = 0; j < N; ++j) q[j] = *(const T *)(s + (i + j < n ? i + j : n - 1) * stride);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j & 3] += i + j < n ? q[j] : T(0);
-    }
+        for (int j = 0; j < N; ++j) v[j & 3] += i + j < n ? q[j] : T(0);
+    };
+    if (n <= 4)
+        add(0, std::integral_constant<int, 4>());
+    else
+        for (int i = 0; i < n; i += 8) add(i, std::integral_constant<int, 8>());
     return (v[0] + v[1]) + (v[2] + v[3]);
 }
 
@@ -598,25 +589,90 @@ template <int FMT> __device__ float tiled_weight(const uint8_t *slab, int row, i
     return __fsub_rn(__fmul_rn(half(row * 16), (float)sc) * (float)q, __fmul_rn(half(row * 16 + 2), (float)m));
 }
 
-/* What infinities and NaN among the activations add to one row: each times
- * its weight, over the units [u0, u1) of x. */
+/* One row's product with one position of x, as the reference's loops take it. */
 template <int FMT>
-__device__ float wild_sum(const float *x, const float *norm_w, int cols, const uint8_t *tile, int row, int u0, int u1)
+__device__ float plain_row(const BatchParams &p, const uint8_t *w, int row, int pos, float denom)
 {
     constexpr int kUnit = BatchFmt<FMT>::kUnit;
+    constexpr size_t kSlab = 64 * BatchFmt<FMT>::kUnitBytes;
+    const uint8_t *tile = w + (size_t)(row >> 6) * p.units * kSlab;
+    const float *x = p.x + (size_t)pos * p.cols;
     float sum = 0.0f;
-    for (int k = u0 * kUnit; k < u1 * kUnit && k < cols; ++k) {
-        const float v = norm_w ? x[k] * norm_w[k] : x[k];
-        if (!__builtin_isfinite(v))
-            sum += v * tiled_weight<FMT>(tile + (size_t)(k / kUnit) * (64 * BatchFmt<FMT>::kUnitBytes), row, k % kUnit);
+#pragma unroll 1
+    for (int k = 0; k < p.cols; ++k) {
+        const float v = p.norm_w ? x[k] / denom * p.norm_w[k] : x[k];
+        sum += v * tiled_weight<FMT>(tile + (k / kUnit) * kSlab, row & 63, k % kUnit);
     }
     return sum;
 }
 
-__device__ __forceinline__ void store_row(const BatchJob &job, int pos, int row, float v)
+__device__ __forceinline__ float lane_of(float v, int) { return v; }
+__device__ __forceinline__ float lane_of(const f4_t &v, int e) { return v[e]; }
+
+/* Where N rows (1 or 4) from `r` of a row group and one position go, and what is
+ * added to them: read before their segments are summed, so that these reads
+ * and the sums' run together. */
+template <int N> struct RowsOut {
+    float *y;
+    const uint8_t *w;
+    int row, left; /* rows of the tensor from `row` on */
+    bool whole;    /* N of them, and y aligned */
+    float add[N];
+};
+
+template <int N> __device__ __forceinline__ RowsOut<N> rows_out(const BatchParams &p, int pos, int group, int r)
 {
-    if (job.add) v += job.add[(size_t)pos * job.ldadd + row];
-    job.y[(size_t)pos * job.rows + row] = v;
+    RowsOut<N> o;
+    int job, rg;
+    locate_group(p, group, job, rg);
+    const BatchJob &j = p.job[job];
+    o.row = rg * 16 + r;
+    o.left = j.rows - o.row;
+    o.w = j.w;
+    o.y = j.y + (size_t)pos * j.rows + o.row;
+    o.whole = o.left >= N && (N == 1 || ((size_t)j.y | (size_t)j.rows * 4) % 16 == 0);
+#pragma unroll
+    for (int e = 0; e < N; ++e) o.add[e] = j.add && e < o.left ? j.add[(size_t)pos * j.ldadd + o.row + e] : 0.0f;
+    return o;
+}
+
+/* What is left of the rows once their segments are summed (v2: the up
+ * projection's, with SwiGLU): the norm's division, SwiGLU, the addend, the
+ * store. Sums that are not finite, which two limbs of an infinity (inf - inf)
+ * never are, are taken again in the plain way: an infinity gives the infinity
+ * of its weight's sign. */
+template <int FMT, int N, bool NORM, typename T>
+__device__ __forceinline__ void finish_rows(const BatchParams &p, int pos, const RowsOut<N> &o, T v, T v2, float denom)
+{
+    float out[N];
+    bool finite = true;
+#pragma unroll
+    for (int e = 0; e < N; ++e) {
+        float a = lane_of(v, e), b = lane_of(v2, e);
+        finite = finite && __builtin_isfinite(a) && (!p.swiglu || __builtin_isfinite(b));
+        if (NORM) a /= denom;
+        if (p.swiglu) a = silu_product(a, NORM ? b / denom : b);
+        out[e] = a + o.add[e];
+    }
+    if (__builtin_expect(!finite, 0)) {
+#pragma unroll 1
+        for (int e = 0; e < N && e < o.left; ++e) {
+            float a = plain_row<FMT>(p, o.w, o.row + e, pos, denom);
+            if (p.swiglu) a = silu_product(a, plain_row<FMT>(p, p.job[1].w, o.row + e, pos, denom));
+            float add = o.add[0];
+#pragma unroll
+            for (int i = 1; i < N; ++i) add = e == i ? o.add[i] : add;
+            o.y[e] = a + add;
+        }
+        return;
+    }
+    if (N == 4 && o.whole) {
+        *(f4_t *)o.y = f4_t{out[0], out[1 % N], out[2 % N], out[3 % N]};
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < N; ++e)
+        if (e < o.left) o.y[e] = out[e];
 }
 
 /* A workgroup stages the activations of a chunk of K (segments [seg0, seg1))
@@ -675,7 +731,6 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
     /* Stage the chunk: a wave per unit and round of 4 positions, up to four
      * loads ahead of the first split. */
     const int stages = nu * NR;
-    bool wild = false;
     for (int s0 = wave; s0 < stages; s0 += 4 * nw) {
         f4_t v[4][NJ];
 #pragma unroll
@@ -719,21 +774,13 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
                     if (!FUSED && g0 == 0) p.ssq[(u0 + su) * P + pos] = ssq;
                 }
             }
-            wild |= stage_position<FMT, NR>(out, v[q], pos, n);
+            stage_position<FMT, NR>(out, v[q], pos, n);
         }
     }
-    uint32_t *flags = (uint32_t *)(lds + nu * L::kBytes); /* of each wave: whether it staged infinities or NaN */
-    if (lane == 0) flags[wave] = wild;
     __syncthreads();
 
     const int arow = F == 1 ? (n >> 3) * P + (n & (P - 1)) : n; /* this lane's row of a fragment */
-    float *part = (float *)(flags + 16); /* FUSED: [segment][row group][position][16] */
-    /* Where the sums of segment seg and row group g go: of position pos, at pos * ld. */
-    const auto sums = [&](int seg, int g) {
-        return FUSED ? part + ((size_t)seg * p.wg_groups + g) * (P * 16) + n
-                     : p.partials + (size_t)(seg0 + seg) * p.positions * p.groups * 16 + (size_t)(g0 + g) * 16 + n;
-    };
-    const size_t ld = FUSED ? 16 : (size_t)p.groups * 16;
+    float *part = (float *)(lds + nu * L::kBytes); /* FUSED: [segment][row group][position][16] */
     f4_t y[R][L::kBlocks];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -765,7 +812,10 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int g = set * R + r; /* of the workgroup */
-            float *o = sums(seg, g);
+            float *o = FUSED ? part + ((size_t)seg * p.wg_groups + g) * (P * 16) + n
+                             : p.partials + (size_t)(seg0 + seg) * p.positions * p.groups * 16 +
+                                   (size_t)(g0 + g) * 16 + n;
+            const size_t ld = FUSED ? 16 : (size_t)p.groups * 16;
             const bool real = R == 1 || g < ng;
 #pragma unroll
             for (int f = 0; f < L::kBlocks; ++f)
@@ -783,26 +833,6 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
             for (int f = 0; f < L::kBlocks; ++f) y[r][f] = f4_t{0, 0, 0, 0};
         }
     }
-    if (__any(lane < nw && flags[lane & 15])) { /* rare: the wave's items again, for what was not staged */
-        for (ig = wave / nseg, is = wave % nseg; ig * R < ng;) {
-            open_item();
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int g = ig * R + r;
-                if (g >= ng) break;
-                float *o = sums(is, g);
-                for (int pos = 4 * kc; pos < p.positions; pos += (pos & 3) < 3 ? 1 : 13) /* this lane's */
-                    o[pos * ld] += wild_sum<FMT>(p.x + (size_t)pos * p.cols, NORM ? p.norm_w : nullptr, p.cols, wp[r],
-                                                 wrow[r], u, uend);
-            }
-            is += step_s;
-            ig += step_g;
-            if (is >= nseg) {
-                is -= nseg;
-                ++ig;
-            }
-        }
-    }
     if constexpr (FUSED) {
         __syncthreads();
         float *denom = part + (size_t)p.segs * p.wg_groups * (P * 16);
@@ -813,69 +843,49 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
             }
             __syncthreads();
         }
+        /* A row a thread, or four where that takes several rounds */
         const int rows = (p.swiglu ? ng / 2 : ng) * 16;
-        for (int o = threadIdx.x; o < rows * p.positions; o += blockDim.x) {
-            const int pos = o / rows, lr = o % rows, g = lr >> 4;
-            const float *s = part + (size_t)(p.swiglu ? 2 * g : g) * (P * 16) + pos * 16 + (lr & 15);
-            const size_t stride = (size_t)p.wg_groups * (P * 16);
-            int job, rg;
-            locate_group(p, g0 + (p.swiglu ? 2 * g : g), job, rg);
-            const int row = rg * 16 + (lr & 15);
-            float v = strided_sum<float>(s, stride, p.segs);
-            if (NORM) v /= denom[pos];
-            if (p.swiglu) {
-                float v2 = strided_sum<float>(s + P * 16, stride, p.segs);
-                if (NORM) v2 /= denom[pos];
-                v = silu_product(v, v2);
-            }
-            if (row < p.job[job].rows) store_row(p.job[job], pos, row, v);
-        }
+        const size_t stride = (size_t)p.wg_groups * (P * 16);
+        const auto finish = [&](auto width, int o) {
+            constexpr int N = decltype(width)::value;
+            typedef std::conditional_t<N == 4, f4_t, float> T;
+            const int pos = o / (rows / N), lr = o % (rows / N) * N, group = p.swiglu ? lr >> 4 << 1 : lr >> 4;
+            const float *s = part + (size_t)group * (P * 16) + pos * 16 + (lr & 15);
+            const RowsOut<N> out = rows_out<N>(p, pos, g0 + group, lr & 15);
+            const T v = strided_sum<T>(s, stride, p.segs);
+            finish_rows<FMT, N, NORM>(p, pos, out, v, p.swiglu ? strided_sum<T>(s + P * 16, stride, p.segs) : v,
+                                      NORM ? denom[pos] : 0.0f);
+        };
+        if (rows * p.positions <= 2 * (int)blockDim.x)
+            for (int o = threadIdx.x; o < rows * p.positions; o += blockDim.x) finish(std::integral_constant<int, 1>(), o);
+        else
+            for (int o = threadIdx.x; o < rows / 4 * p.positions; o += blockDim.x) finish(std::integral_constant<int, 4>(), o);
     }
 }
 
 /* The segments' sums of one position, four rows a thread (of gate and up:
  * four of each), and the epilogue. */
-template <bool NORM>
+template <int FMT, bool NORM>
 __global__ void __launch_bounds__(256) reduce_kernel(BatchParams p, int ssq_ld)
 {
     const int pos = blockIdx.y, lr = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4, g = lr >> 4;
     __shared__ float denom;
-    if (NORM && threadIdx.x == 0)
-        denom = sqrtf((float)(strided_sum<double>(p.ssq + pos, (size_t)ssq_ld, p.units) / p.cols + p.norm_eps));
+    if (NORM && threadIdx.x < 64) { /* a lane per unit: 74 units by one thread were 1.7 us that the others waited */
+        double t = 0.0;
+        for (int u = threadIdx.x; u < p.units; u += 64) t += p.ssq[(size_t)u * ssq_ld + pos];
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) t += __shfl_xor(t, m, 64);
+        if (threadIdx.x == 0) denom = sqrtf((float)(t / p.cols + p.norm_eps));
+    }
     const int group = p.swiglu ? 2 * g : g;
     const bool in = group < p.groups;
     const size_t stride = (size_t)p.positions * p.groups * 16;
     const float *s = p.partials + (size_t)pos * p.groups * 16 + (size_t)(in ? group : 0) * 16 + (lr & 15);
     f4_t v = strided_sum<f4_t>(s, stride, p.segs), v2 = {0, 0, 0, 0};
     if (p.swiglu) v2 = strided_sum<f4_t>(s + 16, stride, p.segs);
-    if (NORM) {
-        __syncthreads();
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] /= denom;
-            v2[e] /= denom;
-        }
-    }
-    if (!in) return;
-    int job, rg;
-    locate_group(p, group, job, rg);
-    const BatchJob &j = p.job[job];
-    const int row = rg * 16 + (lr & 15);
-    if (p.swiglu) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = silu_product(v[e], v2[e]);
-    }
-    if (row + 3 < j.rows && ((size_t)j.y | (size_t)j.rows * 4) % 16 == 0) { /* whole aligned quads: one store */
-        if (j.add) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] += j.add[(size_t)pos * j.ldadd + row + e];
-        }
-        *(f4_t *)(j.y + (size_t)pos * j.rows + row) = v;
-        return;
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-        if (row + e < j.rows) store_row(j, pos, row + e, v[e]);
+    const RowsOut<4> out = rows_out<4>(p, pos, in ? group : 0, lr & 15);
+    if (NORM) __syncthreads();
+    if (in) finish_rows<FMT, 4, NORM>(p, pos, out, v, v2, NORM ? denom : 0.0f);
 }
 
 template <int FMT, int NR, int R, int WAVES, bool NORM, bool FUSED>
@@ -886,13 +896,13 @@ static hipError_t launch_chunks(const BatchParams &p, int waves, hipStream_t s)
     const int most = (p.units + p.segs - 1) / p.segs * p.chunk_segs; /* units of a chunk, at most */
     const size_t units = FUSED ? p.units : most < p.units ? most : p.units;
     const size_t bytes =
-        units * L::kBytes + 64 + (FUSED ? ((size_t)p.segs * p.wg_groups * L::P * 16 + L::P) * sizeof(float) : 0);
+        units * L::kBytes + (FUSED ? ((size_t)p.segs * p.wg_groups * L::P * 16 + L::P) * sizeof(float) : 0);
     if (bytes > 160 * 1024) return hipErrorInvalidValue;
     const int chunks = FUSED ? 1 : (p.segs + p.chunk_segs - 1) / p.chunk_segs;
     chunk_kernel<FMT, NR, R, WAVES, NORM, FUSED><<<chunks * p.chunk_wgs, waves * 64, bytes, s>>>(p);
     if (!FUSED) {
         const int rows = (p.swiglu ? p.groups / 2 : p.groups) * 16;
-        reduce_kernel<NORM><<<dim3((rows + 1023) / 1024, p.positions), 256, 0, s>>>(p, L::P);
+        reduce_kernel<FMT, NORM><<<dim3((rows + 1023) / 1024, p.positions), 256, 0, s>>>(p, L::P);
     }
     return hipGetLastError();
 }

@@ -1031,7 +1031,7 @@ struct BatchShape {
     size_t partials; /* floats of workspace */
 };
 
-constexpr int kLdsBytes = 160 * 1024 - 64 /* the waves' flags */, kCus = 256;
+constexpr int kLdsBytes = 160 * 1024, kCus = 256;
 
 /* The cut with the least estimated time, over segment lengths and segments
  * per workgroup: one workgroup per CU; staging rounds and items per wave times

@@ -50,7 +50,7 @@ bool lds_fits(const ChunkPlan &cp)
     const int most = (p.units + p.segs - 1) / p.segs * p.chunk_segs;
     const size_t units = cp.bt_fused || most > p.units ? p.units : most;
     const size_t slots = 4 * cp.bt_nr;
-    return units * qmv::batch_stage_bytes(cp.fmt, cp.bt_nr) + 64 +
+    return units * qmv::batch_stage_bytes(cp.fmt, cp.bt_nr) +
                (cp.bt_fused ? ((size_t)p.segs * p.wg_groups * slots * 16 + slots) * sizeof(float) : 0) <=
            160 * 1024;
 }
