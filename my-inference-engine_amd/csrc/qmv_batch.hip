@@ -679,12 +679,17 @@ __device__ __forceinline__ void finish_rows(const BatchParams &p, int pos, const
  * for all positions, once; its waves then take the items (R row groups, one
  * segment) of its rows in turn, reading weights one unit ahead. FUSED: the
  * chunk is all of K, the segments' sums meet in LDS and the workgroup writes
- * the rows. Otherwise the sums go to memory, [segment][position][row], and
- * reduce_kernel adds them. Either way a row's segments are added in order, so
- * its bits do not depend on the launch's other rows. */
-template <int FMT, int NR, int R, int WAVES, bool NORM, bool FUSED>
+ * the rows. DIRECT: there is one segment, and a wave writes the rows of an
+ * item (no norm, no SwiGLU) when it has done it, while others read weights.
+ * CHUNKS: the sums go to memory, [segment][position][row], and
+ * reduce_kernel adds them. A row's segments are always added in their
+ * order; how many there are depends on the format, K, the launch's rows in all
+ * and, up to 8 positions or with a norm or SwiGLU, on those (batch_shape), so a
+ * grouped launch may sum in another order than its tensors alone. */
+template <int FMT, int NR, int R, int WAVES, bool NORM, int MODE>
 __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
 {
+    constexpr bool FUSED = MODE != QMV_BATCH_CHUNKS;
     using B = BatchFmt<FMT>;
     using L = BatchStage<FMT, NR>;
     constexpr int F = L::F, P = L::P, NJ = B::kUnit / 64;
@@ -780,7 +785,9 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
     __syncthreads();
 
     const int arow = F == 1 ? (n >> 3) * P + (n & (P - 1)) : n; /* this lane's row of a fragment */
-    float *part = (float *)(lds + nu * L::kBytes); /* FUSED: [segment][row group][position][16] */
+    /* FUSED: [segment][row group][position][16]; DIRECT: of each wave [R][position][16] */
+    float *part = (float *)(lds + nu * L::kBytes);
+    if (MODE == QMV_BATCH_DIRECT) part += wave * (R * P * 16);
     f4_t y[R][L::kBlocks];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -812,7 +819,8 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int g = set * R + r; /* of the workgroup */
-            float *o = FUSED ? part + ((size_t)seg * p.wg_groups + g) * (P * 16) + n
+            float *o = MODE == QMV_BATCH_DIRECT ? part + r * (P * 16) + n
+                       : FUSED ? part + ((size_t)seg * p.wg_groups + g) * (P * 16) + n
                              : p.partials + (size_t)(seg0 + seg) * p.positions * p.groups * 16 +
                                    (size_t)(g0 + g) * 16 + n;
             const size_t ld = FUSED ? 16 : (size_t)p.groups * 16;
@@ -832,8 +840,19 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
 #pragma unroll
             for (int f = 0; f < L::kBlocks; ++f) y[r][f] = f4_t{0, 0, 0, 0};
         }
+        if constexpr (MODE == QMV_BATCH_DIRECT) { /* the item's rows, four a lane */
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            for (int o = lane; o < R * 4 * p.positions; o += 64) {
+                const int r = R == 1 ? 0 : o / (4 * p.positions), pos = (o >> 2) - r * p.positions, q = (o & 3) * 4;
+                if (R > 1 && set * R + r >= ng) break;
+                const f4_t v = strided_sum<f4_t>(part + r * (P * 16) + pos * 16 + q, 0, 1);
+                finish_rows<FMT, 4, false>(p, pos, rows_out<4>(p, pos, g0 + set * R + r, q), v, v, 0.0f);
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
     }
-    if constexpr (FUSED) {
+    if constexpr (MODE == QMV_BATCH_FUSED) {
         __syncthreads();
         float *denom = part + (size_t)p.segs * p.wg_groups * (P * 16);
         if (NORM) {
@@ -888,18 +907,22 @@ __global__ void __launch_bounds__(256) reduce_kernel(BatchParams p, int ssq_ld)
     if (in) finish_rows<FMT, 4, NORM>(p, pos, out, v, v2, NORM ? denom : 0.0f);
 }
 
-template <int FMT, int NR, int R, int WAVES, bool NORM, bool FUSED>
+template <int FMT, int NR, int R, int WAVES, bool NORM, int MODE>
 static hipError_t launch_chunks(const BatchParams &p, int waves, hipStream_t s)
 {
     using L = BatchStage<FMT, NR>;
+    constexpr bool FUSED = MODE != QMV_BATCH_CHUNKS;
+    if (MODE == QMV_BATCH_DIRECT && (p.segs != 1 || p.swiglu)) return hipErrorInvalidValue;
     if (waves > WAVES || p.wg_groups % R || p.wg_groups < 1 || p.segs < 1 || p.segs > p.units) return hipErrorInvalidValue;
     const int most = (p.units + p.segs - 1) / p.segs * p.chunk_segs; /* units of a chunk, at most */
     const size_t units = FUSED ? p.units : most < p.units ? most : p.units;
-    const size_t bytes =
-        units * L::kBytes + (FUSED ? ((size_t)p.segs * p.wg_groups * L::P * 16 + L::P) * sizeof(float) : 0);
+    const size_t sums = MODE == QMV_BATCH_DIRECT  ? (size_t)waves * R * L::P * 16
+                        : MODE == QMV_BATCH_FUSED ? (size_t)p.segs * p.wg_groups * L::P * 16 + L::P
+                                                  : 0;
+    const size_t bytes = units * L::kBytes + sums * sizeof(float);
     if (bytes > 160 * 1024) return hipErrorInvalidValue;
     const int chunks = FUSED ? 1 : (p.segs + p.chunk_segs - 1) / p.chunk_segs;
-    chunk_kernel<FMT, NR, R, WAVES, NORM, FUSED><<<chunks * p.chunk_wgs, waves * 64, bytes, s>>>(p);
+    chunk_kernel<FMT, NR, R, WAVES, NORM, MODE><<<chunks * p.chunk_wgs, waves * 64, bytes, s>>>(p);
     if (!FUSED) {
         const int rows = (p.swiglu ? p.groups / 2 : p.groups) * 16;
         reduce_kernel<FMT, NORM><<<dim3((rows + 1023) / 1024, p.positions), 256, 0, s>>>(p, L::P);
@@ -908,20 +931,27 @@ static hipError_t launch_chunks(const BatchParams &p, int waves, hipStream_t s)
 }
 
 template <int FMT, int NR, int R, int WAVES>
-static hipError_t launch_shape(const BatchParams &p, bool fused, int waves, hipStream_t s)
+static hipError_t launch_shape(const BatchParams &p, int mode, int waves, hipStream_t s)
 {
-    if (fused)
-        return p.norm_w ? launch_chunks<FMT, NR, R, WAVES, true, true>(p, waves, s)
-                        : launch_chunks<FMT, NR, R, WAVES, false, true>(p, waves, s);
-    return p.norm_w ? launch_chunks<FMT, NR, R, WAVES, true, false>(p, waves, s)
-                    : launch_chunks<FMT, NR, R, WAVES, false, false>(p, waves, s);
+    if (mode == QMV_BATCH_DIRECT) {
+        if constexpr (NR >= 4 && R == 1)
+            if (!p.norm_w) return launch_chunks<FMT, NR, R, WAVES, false, QMV_BATCH_DIRECT>(p, waves, s);
+        return hipErrorInvalidValue;
+    }
+    if (mode == QMV_BATCH_FUSED)
+        return p.norm_w ? launch_chunks<FMT, NR, R, WAVES, true, QMV_BATCH_FUSED>(p, waves, s)
+                        : launch_chunks<FMT, NR, R, WAVES, false, QMV_BATCH_FUSED>(p, waves, s);
+    if constexpr (WAVES <= 12) /* what batch_shape cuts chunks for */
+        return p.norm_w ? launch_chunks<FMT, NR, R, WAVES, true, QMV_BATCH_CHUNKS>(p, waves, s)
+                        : launch_chunks<FMT, NR, R, WAVES, false, QMV_BATCH_CHUNKS>(p, waves, s);
+    return hipErrorInvalidValue;
 }
 
 template <int FMT>
-static hipError_t launch_fmt(const BatchParams &p, int nr, int r, bool fused, int waves, hipStream_t s)
+static hipError_t launch_fmt(const BatchParams &p, int nr, int r, int mode, int waves, hipStream_t s)
 {
 #define QMV_BATCH(NR, R, W) \
-    if (nr == NR && r == R && waves <= W) return launch_shape<FMT, NR, R, W>(p, fused, waves, s);
+    if (nr == NR && r == R && waves <= W) return launch_shape<FMT, NR, R, W>(p, mode, waves, s);
     QMV_BATCH(1, 1, 12)
     QMV_BATCH(2, 1, 12)
     if constexpr (FMT == QMV_FMT_Q6_K) {
@@ -953,13 +983,13 @@ size_t batch_stage_bytes(int fmt, int nr)
 #undef QMV_BYTES
 }
 
-hipError_t launch_batch(int fmt, const BatchParams &p, int nr, int r, bool fused, int waves, hipStream_t s)
+hipError_t launch_batch(int fmt, const BatchParams &p, int nr, int r, int mode, int waves, hipStream_t s)
 {
     switch (fmt) {
-    case QMV_FMT_Q8_0: return launch_fmt<QMV_FMT_Q8_0>(p, nr, r, fused, waves, s);
-    case QMV_FMT_Q5_0: return launch_fmt<QMV_FMT_Q5_0>(p, nr, r, fused, waves, s);
-    case QMV_FMT_Q4_K: return launch_fmt<QMV_FMT_Q4_K>(p, nr, r, fused, waves, s);
-    case QMV_FMT_Q6_K: return launch_fmt<QMV_FMT_Q6_K>(p, nr, r, fused, waves, s);
+    case QMV_FMT_Q8_0: return launch_fmt<QMV_FMT_Q8_0>(p, nr, r, mode, waves, s);
+    case QMV_FMT_Q5_0: return launch_fmt<QMV_FMT_Q5_0>(p, nr, r, mode, waves, s);
+    case QMV_FMT_Q4_K: return launch_fmt<QMV_FMT_Q4_K>(p, nr, r, mode, waves, s);
+    case QMV_FMT_Q6_K: return launch_fmt<QMV_FMT_Q6_K>(p, nr, r, mode, waves, s);
     default: return hipErrorInvalidValue;
     }
 }

@@ -158,8 +158,12 @@ inline size_t argmax_words(size_t tiles) { return tiles + (tiles + 63) / 64; }
 inline size_t argmax_counts(size_t tiles) { return (tiles + 63) / 64 + 1; }
 
 /* Matrix-core launch: nr rounds of 4 positions (1, 2, 4 or 8), r row groups
- * per wave (1 or 2). */
-hipError_t launch_batch(int fmt, const BatchParams &p, int nr, int r, bool fused, int waves, hipStream_t s);
+ * per wave (1 or 2), and what a workgroup holds: a chunk of K, all of K, or all
+ * of K in one segment (no norm, no SwiGLU). */
+#define QMV_BATCH_CHUNKS 0
+#define QMV_BATCH_FUSED 1
+#define QMV_BATCH_DIRECT 2
+hipError_t launch_batch(int fmt, const BatchParams &p, int nr, int r, int mode, int waves, hipStream_t s);
 /* LDS bytes of one unit's activations. */
 size_t batch_stage_bytes(int fmt, int nr);
 hipError_t launch_matvec(int fmt, const MatvecParams &p, int m, int grid, int waves, hipStream_t s);

@@ -839,7 +839,7 @@ struct ChunkPlan {
     qmv::BatchParams bp;                   /* matrix-core launch (batch): its parameters */
     bool batch = false;                    /* batch_kernel */
     int bt_nr = 0, bt_r = 0; /* its position rounds and row groups per wave */
-    bool bt_fused = false;
+    int bt_mode = 0;                       /* QMV_BATCH_* */
     qmv::RowdotParams rp;                  /* row-major launch (rowdot): its parameters */
     bool rowdot = false;                   /* rowgroup_q4k_kernel */
     int rd_rows = 0, rd_seg = 0, rd_epi = 0; /* rows per segment, lanes per row segment, epilogue */
@@ -1006,10 +1006,15 @@ bool plan_rowdot(QmvDeviceTensor *const *ts, int count, const float *d_in, int b
  * 1.02-1.09 from 17, at 4 0.86 in launches of 50 MB; at 2 0.57-0.93 up to 8
  * units, 1.18 at 17-24. Q8_0 and Q5_0 (units of 128 weights): 0.55-0.89 up to
  * 12 units (Q5_0 at 3 and 4 1.03-1.07 from 9), 0.95-1.12 at 13-16, with the
- * norm 0.68-0.89 up to 20, 1.05-1.6 beyond 24. One position: Q8_0 and Q5_0
+ * norm 0.68-0.89 up to 20, 1.05-1.6 beyond 24. Rows of few units in launches of
+ * few positions do better there the more rows there are, whose sums the matvec
+ * kernels store from registers: one unit of 128 0.97-1.5 (Q5_0 at 4 to 8 over
+ * 300-3584 rows 0.91-0.93), two at 2 positions 1.03-1.33 and at 3 and 4 over
+ * 19000-260000 rows 1.0-1.23, Q5_0 of 3 to 6 at 2 over 65000 1.05-1.15, one and
+ * two of 256 at 2 over 65000 1.0-1.08. One position: Q8_0 and Q5_0
  * with the norm, 0.87-0.94 up to 8 units (Q8_0: 12), 1.0-1.1 at 13-20, 1.2-2.5
  * beyond; without it never. */
-bool use_chunks(int fmt, int units, double bytes, int batch, bool norm)
+bool use_chunks(int fmt, int units, long long groups, double bytes, int batch, bool norm, bool swiglu)
 {
     if (batch > QMV_VALU_MAX_POSITIONS) return use_prefill(fmt, batch);
     /* A plan or threshold set by the caller applies to the matvec kernels. */
@@ -1017,6 +1022,11 @@ bool use_chunks(int fmt, int units, double bytes, int batch, bool norm)
         return false;
     const bool q8 = fmt == QMV_FMT_Q8_0, q5 = fmt == QMV_FMT_Q5_0;
     if (batch == 1) return norm && ((q8 && units <= 12) || (q5 && units <= 8));
+    if (units <= 7 && !norm && !swiglu) { /* few units, few positions, many rows */
+        if (units == 1 && (q8 || (q5 && (batch <= 3 || groups > 256)))) return false;
+        if (units == 2 && (q8 || q5) && (batch == 2 || (batch <= 4 && groups > 1024))) return false;
+        if (batch == 2 && groups > (q5 ? 1536 : 2048) && (q5 || (units <= 2 && !q8))) return false;
+    }
     if (q8 || q5) return units <= (norm ? 20 : batch == 2 || (q5 && batch <= 4) ? 8 : 12);
     if (batch == 2) return units <= (fmt == QMV_FMT_Q4_K ? 24 : 8);
     if (fmt == QMV_FMT_Q4_K) return units <= (batch >= 7 ? 16 : 24) || bytes >= 6e6;
@@ -1026,12 +1036,30 @@ bool use_chunks(int fmt, int units, double bytes, int batch, bool norm)
 /* How a chunk_kernel launch is cut up. */
 struct BatchShape {
     int nr, r;  /* rounds of 4 positions; row groups per wave */
-    bool fused; /* all of K in one workgroup */
+    int mode;   /* QMV_BATCH_* */
     int waves, segs, chunk_segs, wg_groups;
     size_t partials; /* floats of workspace */
 };
 
 constexpr int kLdsBytes = 160 * 1024, kCus = 256;
+
+/* Launches of 9 to 32 positions, without norm or SwiGLU, that take K in one
+ * segment with the rows stored by the wave that has them, where LDS holds all
+ * of K: many rows of few units. Time against the removed prefill kernel's, with
+ * segments / so, at 9-32 positions: 1 unit 0.8-1.6 / 0.6-1.2 from 9000 rows
+ * (0.57-0.94 / 0.51-0.85 below), 2 0.5-1.4 / 0.45-1.1, 4 0.6-1.1 / 0.5-1.0 from
+ * 9000 rows (0.6-0.78 / 0.7-0.8 below), 6 to 8 0.55-0.97 / 0.48-0.9 (below
+ * 0.61-0.9 / 0.75-1.1; Q6_K of 8 0.58-0.81 / 0.58-0.84), 12 to 16 (units of
+ * 128) from 32000 rows Q5_0 0.7-1.0 / 0.7-0.97, from 150000 Q8_0 0.82-0.99 /
+ * 0.82-0.97, below 0.7-1.1 / 0.95-1.35. */
+bool use_direct(int fmt, int units, long long groups)
+{
+    if (units <= 2) return true;
+    if (units <= (fmt == QMV_FMT_Q6_K ? 6 : 8)) return groups >= 512;
+    return groups >= (fmt == QMV_FMT_Q5_0 ? 2000 : 8000);
+}
+
+constexpr int kDirectWaves = 12;
 
 /* The cut with the least estimated time, over segment lengths and segments
  * per workgroup: one workgroup per CU; staging rounds and items per wave times
@@ -1047,8 +1075,7 @@ constexpr int kLdsBytes = 160 * 1024, kCus = 256;
  * spills); past 8 positions 12, and 8 where a wave takes two row groups to
  * read the staged activations half as often (gate|up at 32 positions: 41.5
  * us against 48.9 with one) or for Q6_K (down at 32: 36 against 58 at 12).
- * The segments are the same with `swiglu` as without, and past 8 positions
- * they do not depend on the positions. room: at most this many floats of
+ * room: at most this many floats of
  * workspace, which may take other cuts than those (waves = 0 if there is
  * none). */
 BatchShape batch_shape(int fmt, int units, long long groups, int batch, bool swiglu, bool norm, size_t room)
@@ -1057,9 +1084,18 @@ BatchShape batch_shape(int fmt, int units, long long groups, int batch, bool swi
     const bool wide = batch > QMV_VALU_MAX_POSITIONS;
     BatchShape best = {};
     best.nr = batch <= 4 ? 1 : batch <= 8 ? 2 : batch <= 16 ? 4 : 8;
-    best.r = wide && groups > 512 && !q6 ? 2 : 1;
-    const int nr = best.nr, r = best.r, limbs = nr <= 2 ? 1 : nr / 2;
+    const int nr = best.nr, limbs = nr <= 2 ? 1 : nr / 2;
     const int stage = (int)qmv::batch_stage_bytes(fmt, nr);
+    if (wide && !norm && !swiglu && use_direct(fmt, units, groups) &&
+        (long long)units * stage + kDirectWaves * 256 * nr <= kLdsBytes) {
+        best.r = 1;
+        best.mode = QMV_BATCH_DIRECT;
+        best.segs = best.chunk_segs = 1;
+        best.wg_groups = (int)((groups + kCus - 1) / kCus);
+        best.waves = std::min(q6 ? 8 : kDirectWaves, std::max(best.wg_groups, units * nr));
+        return best;
+    }
+    const int r = best.r = wide && groups > 512 && !q6 ? 2 : 1;
     const auto round_to = [](long long g, int m) { return (g + m - 1) / m * m; };
     const double stage_us = (q32 ? 100 : 185) * 4 / 2400.0;
     const int instr = (fmt == QMV_FMT_Q4_K ? 130 : q6 ? 190 : fmt == QMV_FMT_Q8_0 ? 75 : 105) +
@@ -1078,33 +1114,34 @@ BatchShape batch_shape(int fmt, int units, long long groups, int batch, bool swi
         if (length == 0) continue;
         const int segs = (units + length - 1) / length;
         const int longest = (units + segs - 1) / segs;
-        for (int cs = 0; cs <= (wide ? 1 : 4) && cs <= segs; ++cs) { /* 0: fused */
+        for (int cs = 0; cs <= (wide ? 1 : 4) && cs <= segs; ++cs) { /* 0: all of K in a workgroup */
             BatchShape c = best;
-            c.fused = cs == 0;
+            const bool fused = cs == 0;
+            c.mode = fused ? QMV_BATCH_FUSED : QMV_BATCH_CHUNKS;
             c.segs = segs;
-            c.chunk_segs = c.fused ? segs : cs;
+            c.chunk_segs = fused ? segs : cs;
             const int chunks = (segs + c.chunk_segs - 1) / c.chunk_segs;
             const long long per = std::max(1, kCus / chunks);
             long long g1 = round_to((groups + per - 1) / per, r), g2 = round_to(g1, 2);
-            const int staged = c.fused ? units : c.chunk_segs * longest;
-            if (c.fused && room != SIZE_MAX) { /* more workgroups than CUs rather than no cut */
+            const int staged = fused ? units : c.chunk_segs * longest;
+            if (fused && room != SIZE_MAX) { /* more workgroups than CUs rather than no cut */
                 const long long fit = ((long long)kLdsBytes - (long long)staged * stage - 16 * nr) / (segs * 256 * nr) & ~1ll;
                 if (fit >= 2 && g2 > fit) g1 = g2 = fit;
             }
             const double rounds = (double)std::max(1LL, (groups + g1 * kCus - 1) / (g1 * kCus));
-            const long long lds = (long long)staged * stage + (c.fused ? (segs * g2 * 64 + 4) * 4 * nr : 0);
+            const long long lds = (long long)staged * stage + (fused ? (segs * g2 * 64 + 4) * 4 * nr : 0);
             if (lds > kLdsBytes) continue;
-            c.partials = c.fused ? 0 : (size_t)segs * batch * groups * 16 + (norm ? (size_t)units * 8 * nr : 0);
+            c.partials = fused ? 0 : (size_t)segs * batch * groups * 16 + (norm ? (size_t)units * 8 * nr : 0);
             if (c.partials > room) continue;
             c.wg_groups = (int)(swiglu ? g2 : g1);
             const long long items = g1 / r * c.chunk_segs, made = c.wg_groups / r * c.chunk_segs;
-            c.waves = r == 2 || (q6 && wide) ? 8 : wide || q6 || !c.fused ? 12 : 16;
+            c.waves = r == 2 || (q6 && wide) ? 8 : wide || q6 || !fused ? 12 : 16;
             c.waves = (int)std::min<long long>(c.waves, std::max<long long>(made, staged * nr));
             const long long busy = std::min<long long>(c.waves, items);
             const double per_unit = std::max(unit_us * ((busy + 3) / 4), 0.45);
             double us = stage_us * ((c.waves + 3) / 4) * ((staged * nr + c.waves - 1) / c.waves);
-            us = (us + (items + busy - 1) / busy * longest * per_unit) * (c.fused ? rounds : 1) + 0.5 * weights_us;
-            us += 0.15 * longest + (c.fused ? 0.6 + 0.09 * segs : 4.6 + 2.0 * segs * batch * groups * 64 / 4.0e6);
+            us = (us + (items + busy - 1) / busy * longest * per_unit) * (fused ? rounds : 1) + 0.5 * weights_us;
+            us += 0.15 * longest + (fused ? 0.6 + 0.09 * segs : 4.6 + 2.0 * segs * batch * groups * 64 / 4.0e6);
             if (us < best_us) {
                 best_us = us;
                 best = c;
@@ -1126,7 +1163,8 @@ bool plan_batch(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0
     long long groups = 0;
     for (int i = 0; i < count; ++i) groups += (ts[i]->rows + 15) / 16;
     if (groups > INT_MAX / 16) return false;
-    if (!use_chunks(fmt, units, (double)groups * 16 * units * t0->geo.unit_bytes, batch, epi.norm_w != nullptr))
+    if (!use_chunks(fmt, units, groups, (double)groups * 16 * units * t0->geo.unit_bytes, batch,
+                    epi.norm_w != nullptr, epi.swiglu))
         return false;
     const BatchShape b = batch_shape(fmt, units, groups, batch, epi.swiglu, epi.norm_w != nullptr, room);
     if (b.waves == 0) return false;
@@ -1166,7 +1204,7 @@ bool plan_batch(QmvDeviceTensor *const *ts, int count, const float *d_in, int b0
     cp->rowdot = cp->paired = false;
     cp->bt_nr = b.nr;
     cp->bt_r = b.r;
-    cp->bt_fused = b.fused;
+    cp->bt_mode = b.mode;
     cp->waves = b.waves;
     cp->fmt = fmt;
     cp->partials = b.partials;
@@ -1380,15 +1418,16 @@ struct Cut {
 int piece_positions(int batch, int pieces, int i) { return batch / pieces + (i < batch % pieces ? 1 : 0); }
 
 /* Whether every piece of a launch needs at most `partials` floats and
- * `counters` words when planned within c->room. */
+ * `counters` words when planned within c->room, and (segs != 0) takes K in as
+ * many segments. */
 bool cut_fits(QmvDeviceTensor *const *ts, int count, const float *d_in, int batch, float *const *d_out,
-              const Epilogue &epi, const Cut &c, size_t partials, size_t counters)
+              const Epilogue &epi, const Cut &c, size_t partials, size_t counters, int segs = 0)
 {
     ChunkPlan cp;
     const int longer = piece_positions(batch, c.pieces, 0), shorter = piece_positions(batch, c.pieces, c.pieces - 1);
     for (int nb = longer; nb >= shorter; --nb)
         if (!plan_chunk(ts, count, d_in, 0, nb, d_out, epi, &cp, c.room) || cp.partials > partials ||
-            cp.counters > counters)
+            cp.counters > counters || (segs && (!cp.batch || cp.bp.segs != segs)))
             return false;
     return true;
 }
@@ -1462,8 +1501,12 @@ WorkspaceNeed workspace_rule(QmvDeviceTensor *const *ts, int count, const float 
 bool scratch_cut(QmvDeviceTensor *const *ts, int count, const float *d_in, int batch, float *const *d_out, Cut *c)
 {
     *c = Cut();
-    for (c->pieces = 1; c->pieces == 1 || batch / c->pieces > QMV_VALU_MAX_POSITIONS; ++c->pieces)
-        if (cut_fits(ts, count, d_in, batch, d_out, Epilogue(), *c, kScratchPartials, kScratchCounters)) return true;
+    if (cut_fits(ts, count, d_in, batch, d_out, Epilogue(), *c, kScratchPartials, kScratchCounters)) return true;
+    ChunkPlan whole;
+    if (plan_batch(ts, count, d_in, 0, batch, d_out, Epilogue(), &whole))
+        for (c->pieces = 2; batch / c->pieces > QMV_VALU_MAX_POSITIONS; ++c->pieces)
+            if (cut_fits(ts, count, d_in, batch, d_out, Epilogue(), *c, kScratchPartials, kScratchCounters, whole.bp.segs))
+                return true;
     return cut_within(ts, count, d_in, batch, d_out, Epilogue(), kScratchPartials, kScratchCounters, c);
 }
 
@@ -1473,7 +1516,7 @@ void bind_workspace(ChunkPlan &cp, float *partials, unsigned *counters)
 {
     cp.p.partials = partials;
     cp.p.counters = counters;
-    if (cp.batch && !cp.bt_fused) {
+    if (cp.batch && cp.bt_mode == QMV_BATCH_CHUNKS) {
         cp.bp.partials = partials;
         cp.bp.ssq = (double *)(partials + (size_t)cp.bp.segs * cp.bp.positions * cp.bp.groups * 16);
     }
@@ -1486,7 +1529,7 @@ void bind_workspace(ChunkPlan &cp, float *partials, unsigned *counters)
 int enqueue_chunk(const ChunkPlan &cp, hipStream_t stream)
 {
     if (cp.batch)
-        HIP_TRY(qmv::launch_batch(cp.fmt, cp.bp, cp.bt_nr, cp.bt_r, cp.bt_fused, cp.waves, stream));
+        HIP_TRY(qmv::launch_batch(cp.fmt, cp.bp, cp.bt_nr, cp.bt_r, cp.bt_mode, cp.waves, stream));
     else if (cp.rowdot && cp.fmt == QMV_FMT_Q6_K)
         HIP_TRY(qmv::launch_rowloop_q6k(cp.rp, cp.rd_epi, cp.grid, cp.waves, stream));
     else if (cp.rowdot)

@@ -382,3 +382,41 @@ def test_chunk_subnormal_operands(qmv, oracle, gpu, hip, t, batch):
     print(f"relative error {err:.2g}", flush=True)
     assert err <= 3e-7
     dt.close()
+
+
+@pytest.mark.parametrize("t", B.ALL_TYPES)
+@pytest.mark.parametrize("rows,units,batch", [(1, 1, 9), (8193, 2, 16), (8200, 3, 17), (12300, 6, 12), (8192, 4, 32), (20011, 1, 31),
+                                              (8195, 8, 10)])
+def test_chunk_direct(qmv, oracle, gpu, hip, t, rows, units, batch):
+    """Launches whose waves store their own rows: one segment of K, at the
+    sizes where they begin, with rows that fill no group and a partial last
+    unit; three tensors at once with an addend each, one in place and one
+    bias; an infinity keeps its sign."""
+    cols = units * (256 if t in (B.Q4_K, B.Q6_K) else 128) - (0 if t in (B.Q4_K, B.Q6_K) else 32)
+    shape = [rows, 33, 16]
+    raws, dts = zip(*[_tensor(qmv, t, r, cols, 60 + i) for i, r in enumerate(shape)])
+    rng = np.random.default_rng(rows)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    x[1, cols // 2] = np.inf
+    adds = [rng.standard_normal((batch, rows)).astype(np.float32), rng.standard_normal(33).astype(np.float32), None]
+    with hip.Stream() as s:
+        dx = hip.DeviceBuffer.from_array(x)
+        ys = [hip.DeviceBuffer(4 * (batch * r + 64)) for r in shape]
+        for y in ys:
+            y.fill(0x7F)
+        ys[0] = hip.DeviceBuffer.from_array(np.concatenate([adds[0].reshape(-1), np.full(64, 7, np.float32)]))
+        bias = hip.DeviceBuffer.from_array(adds[1])
+        print(f"chunks: direct {B.NAMES[t]} {rows}x{cols} M={batch}", flush=True)
+        qmv.device_matvec_add_group(list(dts), dx.ptr, batch, [ys[0].ptr, bias.ptr, 0], [rows, 0, 0], [y.ptr for y in ys],
+                                    s.handle)
+        s.synchronize()
+        out = [y.to_array(np.float32, (batch * r + 64,)) for y, r in zip(ys, shape)]
+    assert (out[0][batch * rows:] == 7).all()
+    assert all((_bits(o[batch * r:]) == 0x7F7F7F7F).all() for o, r in zip(out[1:], shape[1:]))
+    for raw, r, o, add in zip(raws, shape, out, (adds[0], adds[1][None, :], np.zeros((1, 1), np.float32))):
+        y = o[:batch * r].reshape(batch, r)
+        some = [0, 2, batch // 2, batch - 1]
+        _check(oracle, raw, t, r, cols, x[some], (y - add)[some], f"rows {r}", scale=1.5)
+        assert np.array_equal(_class(y[1]), _class(oracle.matvec(raw, t, r, cols, x[1])))
+    for d in dts:
+        d.close()
