@@ -962,8 +962,9 @@ static hipError_t launch_fmt(const BatchParams &p, int nr, int r, int mode, int 
         QMV_BATCH(2, 1, 16)
         QMV_BATCH(4, 1, 12)
         QMV_BATCH(8, 1, 12)
+    }
+    if constexpr (FMT == QMV_FMT_Q4_K || FMT == QMV_FMT_Q8_0) {
         QMV_BATCH(4, 2, 8)
-        QMV_BATCH(8, 2, 8)
     }
 #undef QMV_BATCH
     return hipErrorInvalidValue;

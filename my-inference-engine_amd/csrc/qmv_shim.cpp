@@ -1012,8 +1012,8 @@ bool plan_rowdot(QmvDeviceTensor *const *ts, int count, const float *d_in, int b
  * 300-3584 rows 0.91-0.93), two at 2 positions 1.03-1.33 and at 3 and 4 over
  * 19000-260000 rows 1.0-1.23, Q5_0 of 3 to 6 at 2 over 65000 1.05-1.15, one and
  * two of 256 at 2 over 65000 1.0-1.08. One position: Q8_0 and Q5_0
- * with the norm, 0.87-0.94 up to 8 units (Q8_0: 12), 1.0-1.1 at 13-20, 1.2-2.5
- * beyond; without it never. */
+ * with the norm, 0.87-0.94 up to 8 units (Q8_0: 12; Q5_0 over 9000-32000 rows
+ * 1.04-1.11), 1.0-1.1 at 13-20, 1.2-2.5 beyond; without it never. */
 bool use_chunks(int fmt, int units, long long groups, double bytes, int batch, bool norm, bool swiglu)
 {
     if (batch > QMV_VALU_MAX_POSITIONS) return use_prefill(fmt, batch);
@@ -1021,7 +1021,7 @@ bool use_chunks(int fmt, int units, long long groups, double bytes, int batch, b
     if (g_target_waves.load() > 0 || g_force_u.load() > 0 || g_force_w.load() > 0 || g_mfma_min_batch.load() > 0)
         return false;
     const bool q8 = fmt == QMV_FMT_Q8_0, q5 = fmt == QMV_FMT_Q5_0;
-    if (batch == 1) return norm && ((q8 && units <= 12) || (q5 && units <= 8));
+    if (batch == 1) return norm && ((q8 && units <= 12) || (q5 && units <= 8 && groups <= 512));
     if (units <= 7 && !norm && !swiglu) { /* few units, few positions, many rows */
         if (units == 1 && (q8 || (q5 && (batch <= 3 || groups > 256)))) return false;
         if (units == 2 && (q8 || q5) && (batch == 2 || (batch <= 4 && groups > 1024))) return false;
@@ -1029,7 +1029,7 @@ bool use_chunks(int fmt, int units, long long groups, double bytes, int batch, b
     }
     if (q8 || q5) return units <= (norm ? 20 : batch == 2 || (q5 && batch <= 4) ? 8 : 12);
     if (batch == 2) return units <= (fmt == QMV_FMT_Q4_K ? 24 : 8);
-    if (fmt == QMV_FMT_Q4_K) return units <= (batch >= 7 ? 16 : 24) || bytes >= 6e6;
+    if (fmt == QMV_FMT_Q4_K) return units <= (batch >= 7 ? 16 : 24) || bytes >= (batch == 7 ? 8e6 : 6e6);
     return batch >= 5 || units <= 16 || (batch == 4 && bytes >= 30e6);
 }
 
@@ -1072,9 +1072,17 @@ constexpr int kDirectWaves = 12;
  * segments of five a workgroup 23.2 us, of four 23.8, three of five 24.3).
  * Waves: 16 (the registers of one row group of Q4_K, Q8_0, Q5_0 allow them),
  * 12 for Q6_K and for chunks (down at 4: 23.8 us at 12 against 31.3 at 16 with
- * spills); past 8 positions 12, and 8 where a wave takes two row groups to
- * read the staged activations half as often (gate|up at 32 positions: 41.5
- * us against 48.9 with one) or for Q6_K (down at 32: 36 against 58 at 12).
+ * spills); past 8 positions 12, and 8 where a wave takes two row groups or for
+ * Q6_K (down at 32: 36 against 58 at 12).
+ * Two row groups a wave (r) read the staged activations half as often but
+ * leave a workgroup half the items: time with one to that with two, 384 launches
+ * of 8960 to 32000 rows and K of 1536 to 8960, plain, with norm and with SwiGLU:
+ * Q5_0 0.90-0.94 (at most 1.03), Q4_K and Q8_0 at 17 to 32 positions 0.94-0.97
+ * (1.03), at 9 to 16 over 8960 rows 0.86-1.0, beyond 0.92-1.05, Q8_0 up to 1.13.
+ * Past 8 positions the segments' length is fixed (twice that in units of 128 from
+ * 17 on): 320 launches of 896 to 8000 rows under lengths of 1, 2, 3, 4, 6 and 8,
+ * mean by format and K: the one taken is the fastest or within 4% of it, the
+ * others 0.97-1.4 times its time.
  * room: at most this many floats of
  * workspace, which may take other cuts than those (waves = 0 if there is
  * none). */
@@ -1095,7 +1103,7 @@ BatchShape batch_shape(int fmt, int units, long long groups, int batch, bool swi
         best.waves = std::min(q6 ? 8 : kDirectWaves, std::max(best.wg_groups, units * nr));
         return best;
     }
-    const int r = best.r = wide && groups > 512 && !q6 ? 2 : 1;
+    const int r = best.r = nr == 4 && groups > 640 && (fmt == QMV_FMT_Q4_K || fmt == QMV_FMT_Q8_0) ? 2 : 1;
     const auto round_to = [](long long g, int m) { return (g + m - 1) / m * m; };
     const double stage_us = (q32 ? 100 : 185) * 4 / 2400.0;
     const int instr = (fmt == QMV_FMT_Q4_K ? 130 : q6 ? 190 : fmt == QMV_FMT_Q8_0 ? 75 : 105) +
