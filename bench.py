@@ -39,23 +39,30 @@ sys.path.insert(0, ROOT)
 
 METRIC = "weight-stream GB/s and % of HBM peak; µs per decode-step matvec set (1 GPU)"
 HBM_PEAK_GBS = 8000.0
-FP32_PEAK_TFLOPS = 157.3  # MI355X vector fp32 (the reference's arithmetic: fp32 FMA)
+F16_PEAK_TFLOPS = 2500.0  # MI355X matrix cores, f16, dense
+
+
+def matrix_flops(M, tensors):
+    """What the matrix-core kernel issues for a product of M positions with
+    [(type, rows, cols)]: two f16 limbs per activation, in 16 matrix rows up to
+    8 positions and 32 per block of 16 beyond; Q6_K has two operands a weight.
+    One position runs on the vector units."""
+    rows = 0 if M == 1 else 16 if M <= 8 else 32 if M <= 16 else 64
+    return sum(2 * rows * r * c * (2 if t == Q6_K else 1) for t, r, c in tensors)
 
 
 def batch_roofline(weight_bytes, flops, seconds):
     """Both bounds of a configuration: packed weight bytes over the HBM peak
-    and the product's fp32 arithmetic (2 x positions x rows x columns flops)
-    over the fp32 vector peak; `bound` names the larger fraction. The
-    matrix-core path computes the same products from two f16 limbs per
-    activation, so this fp32 figure is the algorithmic rate, not the
-    matrix-core issue rate."""
+    and matrix_flops over the matrix cores' f16 peak; `bound` names the larger
+    fraction. (What bounds the kernel at 32 positions is neither: the vector
+    instructions that decode the weights.)"""
     gbs = weight_bytes / seconds / 1e9
     tflops = flops / seconds / 1e12
-    hbm, fp32 = gbs / HBM_PEAK_GBS, tflops / FP32_PEAK_TFLOPS
-    return {"bound": "hbm" if hbm >= fp32 else "fp32", "frac": round(max(hbm, fp32), 4),
+    hbm, f16 = gbs / HBM_PEAK_GBS, tflops / F16_PEAK_TFLOPS
+    return {"bound": "hbm" if hbm >= f16 else "matrix", "frac": round(max(hbm, f16), 4),
             "hbm": {"achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(hbm, 4)},
-            "fp32": {"achieved": round(tflops, 2), "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(fp32, 4)}}
+            "matrix": {"achieved": round(tflops, 2), "peak": F16_PEAK_TFLOPS, "unit": "TFLOP/s",
+                       "frac": round(f16, 4)}}
 LAYERS, HIDDEN, INTER, KV = 28, 3584, 18944, 512
 Q4_K, Q6_K = 12, 14
 
@@ -192,11 +199,24 @@ ROWDOT_MAX_UNITS = 2048
 ROWDOT_SHARED_SB = 16
 
 
+def chunked(fmt, M, units, tiled_units):
+    """Whether a Q4_K / Q6_K launch of 2 to 8 positions over rows of `units`
+    runs on chunk_kernel (use_chunks in the library, default tuning)."""
+    nbytes = tiled_units * 64 * (144 if fmt == "Q4_K" else 210)
+    if M == 2 and units <= 2 and tiled_units // max(units, 1) > 512:
+        return False
+    if fmt == "Q4_K":
+        return units <= 24 if M == 2 else units <= (16 if M >= 7 else 24) or nbytes >= (8e6 if M == 7 else 6e6)
+    return units <= 8 if M == 2 else M >= 5 or units <= 16 or (M == 4 and nbytes >= 30e6)
+
+
 def kernel_name(fmt, M, tiled_units=None, cols=None):
     """The kernel a Q4_K / Q6_K launch of M positions over `tiled_units`
     (tile, unit) pairs of rows of `cols` columns runs (default tuning)."""
-    if M >= 5 or (M >= 2 and cols is not None and cols <= 16 * 256):
+    if cols is not None and M >= 2 and (M > 8 or chunked(fmt, M, cols // 256, tiled_units or 0)):
         return "chunk_kernel<%s,%d>" % (fmt, 1 if M <= 4 else 2 if M <= 8 else 4 if M <= 16 else 8)
+    if M >= (7 if fmt == "Q4_K" else 8):
+        return "matvec_mfma_kernel<%s,%d>" % (fmt, M)
     rowdot = os.environ.get("QMV_ROWDOT", "1") != "0"
     if fmt == "Q6_K" and M == 1 and cols is not None and rowdot and os.environ.get("QMV_ROWDOT_Q6K", "1") != "0":
         sb = cols // 256
@@ -523,7 +543,7 @@ def small_configs_bench(qmv, hip, stream, reps):
         raws = {t[0]: qmv.synth_tensor(t[1], t[2], t[3], seed=900 + i)
                 for i, t in enumerate(x for g in groups for x in g)}
         nbytes = sum(r.size for r in raws.values())
-        flops = 2 * m * sum(t[2] * t[3] for g in groups for t in g)
+        flops = matrix_flops(m, [t[1:] for g in groups for t in g])
         copies = max(2, -(-(1 << 30) // nbytes))
         sets = [{t[0]: qmv.DeviceTensor(qmv.make_view(raws[t[0]], t[1], t[2], t[3])) for g in groups for t in g}
                 for _ in range(copies)]
@@ -626,7 +646,6 @@ def main():
         outs.append(o)
     hip.synchronize()
 
-    set_weights = LAYERS * sum(rows * cols for _, _, rows, cols in layer_shapes())  # rows x columns
     launches = build_launches(lib, layers, acts, outs, M)
     main_run = run_set(qmv, hip, stream, launches, args.steps, args.warmup, not args.no_graph)
     passes = max(1, args.profile_passes)
@@ -655,7 +674,8 @@ def main():
                                    "weight_gbs": round(total_bytes / (rb["elapsed"] / max(5, args.steps // 5)) / 1e9,
                                                        1),
                                    "positions_per_s": round(mb / (rb["ms_per_step"] * 1e-3), 1),
-                                   "roofline": batch_roofline(total_bytes, 2 * mb * set_weights,
+                                   "roofline": batch_roofline(total_bytes,
+                                                              LAYERS * matrix_flops(mb, [x[1:] for x in layer_shapes()]),
                                                               rb["ms_per_step"] * 1e-3)}
         extra["vocab_projection"] = vocab_bench(qmv, hip, stream, max(10, args.steps // 2))
         if M == 1:

@@ -266,7 +266,8 @@ int qmv_device_matvec_swiglu_f32(qmv_device_tensor gate, qmv_device_tensor up,
  * written and one launch is saved. Otherwise a norm launch writes h to
  * d_normed (batch_count x K floats, clear of the input, the weights and the
  * outputs) and the projection reads it, or the chunked matrix-core kernel of
- * 2 to 32 positions applies it as it stages the input; after the call the contents of
+ * 2 to 32 positions (and of one, over short Q8_0 and Q5_0 rows) applies it as
+ * it stages the input; after the call the contents of
  * d_normed are unspecified. Results are within the row tolerance of the
  * reference's norm followed by its matvec either way. Argument rules: those
  * of qmv_device_rms_norm_f32 (epsilon <= 0 fails) and of the plain entry

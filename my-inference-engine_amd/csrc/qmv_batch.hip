@@ -1,6 +1,6 @@
 /*
  * gfx950 kernels of the packed products of 2 to 32 positions on the matrix
- * cores.
+ * cores, and of one position over short Q8_0 and Q5_0 rows with the RMSNorm.
  *
  * A workgroup takes a chunk of K (all of it where its activations fit LDS)
  * and a range of 16-row groups. It stages the chunk's activations in LDS

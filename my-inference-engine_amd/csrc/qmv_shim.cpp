@@ -824,7 +824,7 @@ struct Epilogue {
     const int *ldadd = nullptr;        /* per tensor: 0 = one vector for all positions */
     int *argmax = nullptr;             /* one tensor, batch 1: greedy argmax of y here */
     bool swiglu = false;               /* tensors (gate, up): out[0] = up * silu(gate) */
-    const float *norm_w = nullptr;     /* row-major launches only: RMSNorm of the input fused in */
+    const float *norm_w = nullptr;     /* row-major and chunk_kernel launches: RMSNorm of the input fused in */
     float norm_eps = 0.0f;
 };
 
@@ -837,11 +837,11 @@ struct Epilogue {
 struct ChunkPlan {
     qmv::MatvecParams p;
     qmv::BatchParams bp;                   /* matrix-core launch (batch): its parameters */
-    bool batch = false;                    /* batch_kernel */
+    bool batch = false;                    /* chunk_kernel */
     int bt_nr = 0, bt_r = 0; /* its position rounds and row groups per wave */
     int bt_mode = 0;                       /* QMV_BATCH_* */
     qmv::RowdotParams rp;                  /* row-major launch (rowdot): its parameters */
-    bool rowdot = false;                   /* rowgroup_q4k_kernel */
+    bool rowdot = false;                   /* rowgroup_q4k_kernel or rowloop_q6k_kernel */
     int rd_rows = 0, rd_seg = 0, rd_epi = 0; /* rows per segment, lanes per row segment, epilogue */
     bool rd_norm = false;                    /* the fused RMSNorm of the input */
     bool paired = false;
@@ -1841,7 +1841,6 @@ QMV_API int qmv_dequantize_rows_f32(const QmvTensorView *matrix, int first_row, 
     return 1;
 }
 
-/* Address ranges of device buffers, for the no-overlap rules. */
 QMV_API int qmv_device_rms_norm_f32(const float *d_input, const float *d_weight, int length, int batch_count,
                                     float epsilon, float *d_output, void *stream)
 {
@@ -2162,8 +2161,9 @@ QMV_API int qmv_device_matvec_swiglu_f32(qmv_device_tensor gate, qmv_device_tens
 }
 
 /* RMSNorm of the input followed by a grouped launch. The norm runs inside
- * the row-major launch where that launch takes the call (one position, Q4_K
- * rows of at most 16 super-blocks: each workgroup holds the whole input);
+ * the row-major launch (one position, Q4_K rows of at most 16 super-blocks:
+ * each workgroup holds the whole input) or inside chunk_kernel (2 to 32
+ * positions, and one of short Q8_0 and Q5_0 rows) where that takes the call;
  * otherwise a norm launch writes d_normed and the group reads it. */
 static int norm_then_group(QmvDeviceTensor *const *ts, int count, const float *d_in, const float *d_w, float eps,
                            int batch, float *const *d_out, float *d_normed, hipStream_t s, Workspace &ws,

@@ -325,8 +325,8 @@ def test_random_sweep_with_plans(qmv, oracle, gpu):
 def test_activation_dynamic_range(qmv, oracle, gpu, t, batch, scale):
     """Activations far from N(0,1) stay within the row bar on every kernel:
     M = 1 on the VALU (Q4_K/Q6_K codes on v_fma_mix_f32, whose sums run scaled
-    by 2^-24), M = 8 on the matrix cores (exact bf16 limbs), 20 positions in
-    the prefill kernel (Q8_0/Q5_0: passes of 8 on the VALU). The whole vector
+    by 2^-24), 8 and 20 positions on the matrix cores (two f16 limbs under a
+    power of two per position and unit). The whole vector
     at 1e-28 or 1e28, or magnitudes from 1e-20 to 1e20 element by element."""
     cols = 4 * 256
     rng = np.random.default_rng(batch * 7 + len(scale))
