@@ -679,8 +679,8 @@ __device__ __forceinline__ void finish_rows(const BatchParams &p, int pos, const
  * for all positions, once; its waves then take the items (R row groups, one
  * segment) of its rows in turn, reading weights one unit ahead. FUSED: the
  * chunk is all of K, the segments' sums meet in LDS and the workgroup writes
- * the rows. DIRECT: there is one segment, and a wave writes the rows of an
- * item (no norm, no SwiGLU) when it has done it, while others read weights.
+ * the rows. DIRECT: a wave takes all segments of a row group and writes its
+ * rows (no norm, no SwiGLU) when it has them, while others read weights.
  * CHUNKS: the sums go to memory, [segment][position][row], and
  * reduce_kernel adds them. A row's segments are always added in their
  * order; how many there are depends on the format, K, the launch's rows in all
@@ -706,8 +706,9 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
     const size_t tile_bytes = (size_t)p.units * 64 * B::kUnitBytes;
 
     /* The items of this wave: (ig, is) = row group set and segment. */
-    const int step_g = nw / nseg, step_s = nw % nseg;
-    int ig = wave / nseg, is = wave % nseg, u = 0, uend = 0;
+    constexpr bool DIRECT = MODE == QMV_BATCH_DIRECT; /* a wave takes all segments of its row groups */
+    const int step_g = DIRECT ? nw : nw / nseg, step_s = DIRECT ? 1 : nw % nseg;
+    int ig = DIRECT ? wave : wave / nseg, is = DIRECT ? 0 : wave % nseg, u = 0, uend = 0;
     const uint8_t *wp[R];
     int wrow[R];
     const auto open_item = [&]() {
@@ -785,9 +786,9 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
     __syncthreads();
 
     const int arow = F == 1 ? (n >> 3) * P + (n & (P - 1)) : n; /* this lane's row of a fragment */
-    /* FUSED: [segment][row group][position][16]; DIRECT: of each wave [R][position][16] */
+    /* FUSED: [segment][row group][position][16]; DIRECT: of each wave [segment][position][16] */
     float *part = (float *)(lds + nu * L::kBytes);
-    if (MODE == QMV_BATCH_DIRECT) part += wave * (R * P * 16);
+    if (DIRECT) part += wave * (nseg * P * 16);
     f4_t y[R][L::kBlocks];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -805,13 +806,16 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
         const bool last = ++u == uend;
         if (last) { /* the next item's first unit */
             is += step_s;
-            ig += step_g;
+            if (!DIRECT) ig += step_g;
             if (is >= nseg) {
                 is -= nseg;
-                ++ig;
+                ig += DIRECT ? step_g : 1;
             }
             more = ig * R < ng;
-            if (more) open_item();
+            if (DIRECT && is) /* the same rows */
+                uend = segment_begin(p, is + 1);
+            else if (more)
+                open_item();
         }
         load_w(more ? u : u - 1); /* past the last: that one again */
         unit_product<FMT, NR, R>(b, a, stage, arow, kc, y);
@@ -819,7 +823,7 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const int g = set * R + r; /* of the workgroup */
-            float *o = MODE == QMV_BATCH_DIRECT ? part + r * (P * 16) + n
+            float *o = DIRECT  ? part + seg * (P * 16) + n
                        : FUSED ? part + ((size_t)seg * p.wg_groups + g) * (P * 16) + n
                              : p.partials + (size_t)(seg0 + seg) * p.positions * p.groups * 16 +
                                    (size_t)(g0 + g) * 16 + n;
@@ -840,14 +844,15 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
 #pragma unroll
             for (int f = 0; f < L::kBlocks; ++f) y[r][f] = f4_t{0, 0, 0, 0};
         }
-        if constexpr (MODE == QMV_BATCH_DIRECT) { /* the item's rows, four a lane */
+        if constexpr (DIRECT) { /* the row group's rows, four a lane */
+            if (seg + 1 < nseg) continue;
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
-            for (int o = lane; o < R * 4 * p.positions; o += 64) {
-                const int r = R == 1 ? 0 : o / (4 * p.positions), pos = (o >> 2) - r * p.positions, q = (o & 3) * 4;
-                if (R > 1 && set * R + r >= ng) break;
-                const f4_t v = strided_sum<f4_t>(part + r * (P * 16) + pos * 16 + q, 0, 1);
-                finish_rows<FMT, 4, false>(p, pos, rows_out<4>(p, pos, g0 + set * R + r, q), v, v, 0.0f);
+            for (int o = lane; o < 4 * p.positions; o += 64) {
+                const int pos = o >> 2, q = (o & 3) * 4;
+                const float *s = part + pos * 16 + q;
+                const f4_t v = nseg == 1 ? f4_t{0, 0, 0, 0} + *(const f4_t *)s : strided_sum<f4_t>(s, P * 16, nseg);
+                finish_rows<FMT, 4, false>(p, pos, rows_out<4>(p, pos, g0 + set, q), v, v, 0.0f);
             }
             __builtin_amdgcn_wave_barrier();
         }
@@ -885,7 +890,7 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
 /* The segments' sums of one position, four rows a thread (of gate and up:
  * four of each), and the epilogue. */
 template <int FMT, bool NORM>
-__global__ void __launch_bounds__(256) reduce_kernel(BatchParams p, int ssq_ld)
+__global__ void __launch_bounds__(256, 8) reduce_kernel(BatchParams p, int ssq_ld)
 {
     const int pos = blockIdx.y, lr = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4, g = lr >> 4;
     __shared__ float denom;
@@ -912,11 +917,11 @@ static hipError_t launch_chunks(const BatchParams &p, int waves, hipStream_t s)
 {
     using L = BatchStage<FMT, NR>;
     constexpr bool FUSED = MODE != QMV_BATCH_CHUNKS;
-    if (MODE == QMV_BATCH_DIRECT && (p.segs != 1 || p.swiglu)) return hipErrorInvalidValue;
+    if (MODE == QMV_BATCH_DIRECT && (R != 1 || p.swiglu)) return hipErrorInvalidValue;
     if (waves > WAVES || p.wg_groups % R || p.wg_groups < 1 || p.segs < 1 || p.segs > p.units) return hipErrorInvalidValue;
     const int most = (p.units + p.segs - 1) / p.segs * p.chunk_segs; /* units of a chunk, at most */
     const size_t units = FUSED ? p.units : most < p.units ? most : p.units;
-    const size_t sums = MODE == QMV_BATCH_DIRECT  ? (size_t)waves * R * L::P * 16
+    const size_t sums = MODE == QMV_BATCH_DIRECT  ? (size_t)waves * p.segs * L::P * 16
                         : MODE == QMV_BATCH_FUSED ? (size_t)p.segs * p.wg_groups * L::P * 16 + L::P
                                                   : 0;
     const size_t bytes = units * L::kBytes + sums * sizeof(float);

@@ -159,7 +159,7 @@ inline size_t argmax_counts(size_t tiles) { return (tiles + 63) / 64 + 1; }
 
 /* Matrix-core launch: nr rounds of 4 positions (1, 2, 4 or 8), r row groups
  * per wave (1 or 2), and what a workgroup holds: a chunk of K, all of K, or all
- * of K in one segment (no norm, no SwiGLU). */
+ * of K with each row group in one wave (r = 1, no norm, no SwiGLU). */
 #define QMV_BATCH_CHUNKS 0
 #define QMV_BATCH_FUSED 1
 #define QMV_BATCH_DIRECT 2

@@ -1043,23 +1043,25 @@ struct BatchShape {
 
 constexpr int kLdsBytes = 160 * 1024, kCus = 256;
 
-/* Launches of 9 to 32 positions, without norm or SwiGLU, that take K in one
- * segment with the rows stored by the wave that has them, where LDS holds all
- * of K: many rows of few units. Time against the removed prefill kernel's, with
- * segments / so, at 9-32 positions: 1 unit 0.8-1.6 / 0.6-1.2 from 9000 rows
- * (0.57-0.94 / 0.51-0.85 below), 2 0.5-1.4 / 0.45-1.1, 4 0.6-1.1 / 0.5-1.0 from
- * 9000 rows (0.6-0.78 / 0.7-0.8 below), 6 to 8 0.55-0.97 / 0.48-0.9 (below
- * 0.61-0.9 / 0.75-1.1; Q6_K of 8 0.58-0.81 / 0.58-0.84), 12 to 16 (units of
- * 128) from 32000 rows Q5_0 0.7-1.0 / 0.7-0.97, from 150000 Q8_0 0.82-0.99 /
- * 0.82-0.97, below 0.7-1.1 / 0.95-1.35. */
-bool use_direct(int fmt, int units, long long groups)
+/* Launches of 9 to 32 positions, without norm or SwiGLU, whose waves take all of
+ * K for their row groups and store the rows themselves, where LDS holds all of
+ * K: many rows of few units, whose sums would wait in LDS or go to memory. 728
+ * launches of 1000 to 152000 rows, time against the split-K kernel that this one
+ * replaced, tenth to ninetieth of a hundred, segments over the waves / so: from
+ * 8200 rows on, one unit of 256 0.74-1.20 / 0.70-1.03, two 0.61-1.01 /
+ * 0.57-0.93, four 0.61-0.87 / 0.57-0.85, six 0.51-0.92 / 0.49-0.86 with the
+ * medians 0.62 / 0.66; units of 128, one 0.95-1.50 / 0.78-1.25, two 0.81-1.25 /
+ * 0.66-1.11, four 0.79-1.08 / 0.64-1.00, eight 0.77-0.97 / 0.73-0.93, twelve
+ * (Q5_0 from 32000 rows, Q8_0 from 128000) 0.74-1.04 / 0.71-0.99. Below, one and
+ * two units 0.55-0.94 / 0.53-0.85 (of 256 at 17 to 32 positions 4% slower so), more with a wave for all of a row up to twice
+ * as long as with several. */
+bool use_direct(int fmt, int units, long long groups, int batch)
 {
-    if (units <= 2) return true;
-    if (units <= (fmt == QMV_FMT_Q6_K ? 6 : 8)) return groups >= 512;
-    return groups >= (fmt == QMV_FMT_Q5_0 ? 2000 : 8000);
+    const bool k_quant = fmt == QMV_FMT_Q4_K || fmt == QMV_FMT_Q6_K;
+    if (units <= 2 && (batch <= 16 || !k_quant)) return true;
+    if (k_quant) return units <= 4 && groups >= 512;
+    return groups >= (units <= 8 ? 512 : fmt == QMV_FMT_Q5_0 ? 2000 : 8000);
 }
-
-constexpr int kDirectWaves = 12;
 
 /* The cut with the least estimated time, over segment lengths and segments
  * per workgroup: one workgroup per CU; staging rounds and items per wave times
@@ -1094,15 +1096,6 @@ BatchShape batch_shape(int fmt, int units, long long groups, int batch, bool swi
     best.nr = batch <= 4 ? 1 : batch <= 8 ? 2 : batch <= 16 ? 4 : 8;
     const int nr = best.nr, limbs = nr <= 2 ? 1 : nr / 2;
     const int stage = (int)qmv::batch_stage_bytes(fmt, nr);
-    if (wide && !norm && !swiglu && use_direct(fmt, units, groups) &&
-        (long long)units * stage + kDirectWaves * 256 * nr <= kLdsBytes) {
-        best.r = 1;
-        best.mode = QMV_BATCH_DIRECT;
-        best.segs = best.chunk_segs = 1;
-        best.wg_groups = (int)((groups + kCus - 1) / kCus);
-        best.waves = std::min(q6 ? 8 : kDirectWaves, std::max(best.wg_groups, units * nr));
-        return best;
-    }
     const int r = best.r = nr == 4 && groups > 640 && (fmt == QMV_FMT_Q4_K || fmt == QMV_FMT_Q8_0) ? 2 : 1;
     const auto round_to = [](long long g, int m) { return (g + m - 1) / m * m; };
     const double stage_us = (q32 ? 100 : 185) * 4 / 2400.0;
@@ -1115,6 +1108,20 @@ BatchShape batch_shape(int fmt, int units, long long groups, int batch, bool swi
     const int fixed = !wide ? 0
                             : (kunits <= 40 && (groups <= 512 || (q6 && kunits <= 16 && groups <= 2048)) ? 2 : 4) *
                                   (q32 && units > 16 ? 2 : 1);
+    if (wide && !norm && !swiglu && use_direct(fmt, units, groups, batch)) {
+        best.segs = best.chunk_segs = (units + fixed - 1) / fixed;
+        best.wg_groups = (int)((groups + kCus - 1) / kCus);
+        const long long room_waves = ((long long)kLdsBytes - (long long)units * stage) / (best.segs * 256 * nr);
+        if (room_waves >= 8) {
+            best.waves = std::min(q6 || room_waves < 12 ? 8 : 12, std::max(best.wg_groups, units * nr));
+            best.r = 1;
+            best.mode = QMV_BATCH_DIRECT;
+            return best;
+        }
+        best = BatchShape();
+        best.nr = nr;
+        best.r = r;
+    }
     double best_us = 1e30;
     const int lengths[] = {fixed, 1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 16};
     for (int i = 0; i < 12; ++i) {

@@ -49,10 +49,10 @@ bool lds_fits(const ChunkPlan &cp)
     const qmv::BatchParams &p = cp.bp;
     const int most = (p.units + p.segs - 1) / p.segs * p.chunk_segs;
     const size_t units = cp.bt_mode != QMV_BATCH_CHUNKS || most > p.units ? p.units : most, slots = 4 * cp.bt_nr;
-    const size_t sums = cp.bt_mode == QMV_BATCH_DIRECT  ? (size_t)cp.waves * cp.bt_r * slots * 16
+    const size_t sums = cp.bt_mode == QMV_BATCH_DIRECT  ? (size_t)cp.waves * p.segs * slots * 16
                         : cp.bt_mode == QMV_BATCH_FUSED ? (size_t)p.segs * p.wg_groups * slots * 16 + slots
                                                         : 0;
-    return (cp.bt_mode != QMV_BATCH_DIRECT || (p.segs == 1 && !p.swiglu && !p.norm_w)) &&
+    return (cp.bt_mode != QMV_BATCH_DIRECT || (cp.bt_r == 1 && !p.swiglu && !p.norm_w)) &&
            units * qmv::batch_stage_bytes(cp.fmt, cp.bt_nr) + sums * sizeof(float) <= 160 * 1024;
 }
 
