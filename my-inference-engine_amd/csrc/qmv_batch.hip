@@ -13,8 +13,9 @@
  * the weight stream (gate|up 18944 x 3584 Q4_K with norm and SwiGLU at 8
  * positions 23.7 us, 76.6 MB: 3.2 TB/s with the launch, staging and epilogue;
  * 40.8 us before on split-K launches with bf16 limbs and a norm launch); at 32
- * the vector instructions that decode weights and apply scales, 35k of 55k
- * cycles of a SIMD, with the matrix cores' 19k (64 us before, 41).
+ * the vector instructions that decode weights and apply scales, 33k of 48k
+ * cycles of a SIMD, with the matrix cores' 19k (64 us before, 41 with its
+ * reduction).
  *
  * Activations. x of one position and unit is scaled by the power of two that
  * brings the largest magnitude to [2^14, 2^15) and split into two f16 limbs,

@@ -1,15 +1,14 @@
 """GPU parity of prefill batches of more than 8 positions (the reference
 prefills in chunks of QWEN2_PREFILL_CHUNK_SIZE = 8, src/qwen2_internal.h:7,
 through quantized_tensor_matmul_f32, src/quantized_matvec.cpp:164-224).
-Q4_K and Q6_K batches of 9..32 positions run as one launch of the prefill
-kernel (four tiles per workgroup sharing activations staged in LDS, two
-position blocks of 16 per decoded code tile); larger batches and the other
-formats run as consecutive launches.
+Batches of 9..32 positions run as one launch of chunk_kernel (activations
+staged in LDS once per workgroup, up to two position blocks of 16 per decoded
+weight); larger batches run as consecutive launches.
 
 Bars: every row of every position within 1e-5 * sum |w x| of the oracle;
-and, because a position's arithmetic in the prefill kernel does not depend
-on the other positions of its launch, a launch is bit-identical to the same
-positions run in smaller prefill launches.
+and, because a position's arithmetic past 8 positions does not depend on the
+other positions of its launch, a launch is bit-identical to the same positions
+run in smaller launches of 9 or more.
 """
 import os
 
@@ -78,12 +77,10 @@ def test_prefill_32_at_layer_shapes(qmv, oracle, gpu, t, rows, cols):
                                          (B.Q5_0, 130, 32 * 133)])
 @pytest.mark.parametrize("batch", [16, 27, 32])
 def test_prefill_long_rows_q5_q8(qmv, oracle, gpu, t, rows, cols, batch):
-    """Q8_0 / Q5_0 prefill launches over rows of 32 or more four-block units
-    (K >= 4096), where the plan takes two units per split for launches of at
-    most 8 tile groups and five otherwise; two shapes end in a partial last
-    unit (131 and 133 blocks). The first two shapes split K 19 and 35 ways, so
-    their launches finish in the reduction kernel (pf_reduce_kernel) at every
-    batch here, 16 position rows included."""
+    """Q8_0 / Q5_0 launches over rows of 32 or more four-block units
+    (K >= 4096), whose segments' sums are added by the reduction kernel
+    (reduce_kernel); two shapes end in a partial last unit (131 and 133
+    blocks)."""
     raw = qmv.synth_tensor(t, rows, cols, seed=340 + batch)
     x = qmv.synth_normal(batch * cols, seed=341 + batch).reshape(batch, cols)
     v = qmv.make_view(raw, t, rows, cols)
@@ -125,13 +122,10 @@ def test_prefill_positions_independent(qmv, gpu, hip, t, batch, parts):
                          ids=["32rows-reduction-kernel", "32rows-in-kernel", "16rows-reduction-kernel",
                               "16rows-in-kernel"])
 def test_prefill_epilogues(qmv, oracle, gpu, hip, cols, batch):
-    """Bias addend and fused SwiGLU on prefill launches (the positions past
-    the batch inside the kernel's position blocks are never stored), for both
-    split-K finishes: in the reduction kernel (pf_reduce_kernel) where the
-    in-kernel finish would take 5 or more rounds of partial loads (K = 3584:
-    14 splits at 32 position rows, 7 rounds; K = 7936: 31 splits at 16, 8
-    rounds), and inside the prefill kernel with its SwiGLU pair protocol
-    otherwise (K = 1024: 4 splits; K = 3584 at 16 position rows: 4 rounds)."""
+    """Bias addend and fused SwiGLU on launches past 8 positions (the positions
+    past the batch inside the kernel's position blocks are never stored), where
+    the sums of few segments meet in the workgroup (K = 1024) and where the
+    reduction kernel adds them (K = 3584, 7936)."""
     t, rows = B.Q4_K, 1000
     raw_g = qmv.synth_tensor(t, rows, cols, seed=330)
     raw_u = qmv.synth_tensor(t, rows, cols, seed=331)
@@ -169,10 +163,10 @@ def test_prefill_epilogues(qmv, oracle, gpu, hip, cols, batch):
 @pytest.mark.parametrize("batch", [27, 32])
 def test_prefill_group_of_unequal_tensors(qmv, oracle, gpu, hip, t, batch):
     """A grouped launch of three tensors of unequal rows (17, 2 and 1 tiles,
-    the last two partial) over K = 3584 (14 splits): its partials finish in
-    the reduction kernel, which finds each thread's tensor from the tile
-    counts. Every tensor within the row bar of the oracle and bit-identical
-    to the same tensor launched alone."""
+    the last two partial) over K = 3584: its segments' sums are added in the
+    reduction kernel, which finds each thread's tensor from the row groups.
+    Every tensor within the row bar of the oracle and, with as many segments
+    here, bit-identical to the same tensor launched alone."""
     rows, cols = [1030, 100, 7], 3584
     raws = [qmv.synth_tensor(t, r, cols, seed=380 + i) for i, r in enumerate(rows)]
     dts = [qmv.DeviceTensor(qmv.make_view(raw, t, r, cols)) for raw, r in zip(raws, rows)]
