@@ -889,9 +889,14 @@ __global__ void __launch_bounds__(WAVES * 64) chunk_kernel(BatchParams p)
 }
 
 /* The segments' sums of one position, four rows a thread (of gate and up:
- * four of each), and the epilogue. */
+ * four of each), and the epilogue. Seven waves a SIMD (72 registers, 5 of them
+ * spilled) stream the partial sums best: time over 28 launches of 4 to 32
+ * positions to that of the kernel without the check for infinities, seven waves
+ * 0.987, eight (11 spilled) 0.995, six 0.991, five (what the compiler takes by
+ * itself, 84 registers) 0.988; 151936 x 2048 Q6_K at 32 positions 101.7, 105.0,
+ * 103.9, 103.8 us. */
 template <int FMT, bool NORM>
-__global__ void __launch_bounds__(256, 8) reduce_kernel(BatchParams p, int ssq_ld)
+__global__ void __launch_bounds__(256, 7) reduce_kernel(BatchParams p, int ssq_ld)
 {
     const int pos = blockIdx.y, lr = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4, g = lr >> 4;
     __shared__ float denom;
