@@ -419,3 +419,24 @@ def test_chunk_direct(qmv, oracle, gpu, hip, t, rows, units, batch):
         assert np.array_equal(_class(y[1]), _class(oracle.matvec(raw, t, r, cols, x[1])))
     for d in dts:
         d.close()
+
+
+@pytest.mark.parametrize("t", B.ALL_TYPES)
+@pytest.mark.parametrize("batch,cols", [(3, 512), (20, 1024)])
+def test_chunk_norm_weights_that_overflow(qmv, oracle, gpu, hip, t, batch, cols):
+    """Inputs times norm weights past fp32's range where the normalised values
+    are within it: the reference divides first, and so must the rows."""
+    rows = 40
+    raw, dt = _tensor(qmv, t, rows, cols, 71)
+    x = (qmv.synth_normal(batch * cols, seed=72).reshape(batch, cols) * np.float32(1e15)).astype(np.float32)
+    nw = np.full(cols, 1e25, np.float32)
+    normed = np.stack([oracle.rms_norm(v, nw, 1e-6)[1] for v in x])
+    assert np.isfinite(normed).all()
+    with hip.Stream() as s:
+        dx, dw, dn = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer.from_array(nw), hip.DeviceBuffer(4 * batch * cols)
+        dy = hip.DeviceBuffer(4 * batch * rows)
+        print(f"chunks: norm overflow {B.NAMES[t]} K={cols} M={batch}", flush=True)
+        qmv.device_rms_norm_matvec_add_group([dt], dx.ptr, dw.ptr, 1e-6, batch, [0], [0], [dy.ptr], dn.ptr, s.handle)
+        s.synchronize()
+        _check(oracle, raw, t, rows, cols, normed, dy.to_array(np.float32, (batch, rows)), "overflow", scale=2.0)
+    dt.close()
